@@ -36,9 +36,13 @@ struct CalcgpPtrs {
 
 // NL > 0: exactly NL levels, every per-level array in registers; NL = 0:
 // a.nlev <= 64 levels at run time, the arrays in per-lane memory.
+// With sid (gridpointa) rcsq = 1 / cos^2 comes from the Gaussian abscissas, as
+// the model sets it up (src/plasim.f90:1897 csq = 1 - sid^2 in the real kind,
+// :205), and is written to rcsq_out; else it is read.
 template <typename R, int NL>
 __global__ __launch_bounds__(256) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, int nlev_rt,
-                                                int nhor, long mstride, int nqspec, int exp_gp) {
+                                                int nhor, long mstride, int nqspec, int exp_gp,
+                                                const double* sid, int nlon, R* rcsq_out) {
   constexpr int NA = NL > 0 ? NL : 64;
   const int n = NL > 0 ? NL : nlev_rt;
   const int h = blockIdx.x * 256 + threadIdx.x;
@@ -46,7 +50,15 @@ __global__ __launch_bounds__(256) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, i
   const long mo = (long)blockIdx.y * mstride;
   auto at = [&](const R* p, int j) -> R { return p[mo + (long)j * nhor + h]; };
   auto put = [&](R* p, int j, R x) { p[mo + (long)j * nhor + h] = x; };
-  const R gpm = f.gpm[mo + h], gpj = f.gpj[mo + h], rcsq = f.rcsq[mo + h];
+  const R gpm = f.gpm[mo + h], gpj = f.gpj[mo + h];
+  R rcsq;
+  if (sid) {
+    const double x = sid[h / nlon];
+    rcsq = R(1) / (R)(1.0 - x * x);
+    rcsq_out[mo + h] = rcsq;
+  } else {
+    rcsq = f.rcsq[mo + h];
+  }
   R gp = f.gp[mo + h];
   if (exp_gp) {
     gp = exp(gp);
@@ -185,16 +197,6 @@ __global__ __launch_bounds__(256) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, i
   }
 }
 
-// rcsq = 1 / cos^2 per grid point from the Gaussian abscissas, as the model
-// sets it up (src/plasim.f90:1897 csq = 1 - sid^2 in the real kind, :205)
-template <typename R>
-__global__ void k_rcsq(const double* sid, int nlat, int nlon, R* out, long mstride) {
-  const int h = blockIdx.x * 256 + threadIdx.x;
-  if (h >= nlat * nlon) return;
-  const R csq = (R)(1.0 - sid[h / nlon] * sid[h / nlon]);
-  out[blockIdx.y * mstride + h] = R(1) / csq;
-}
-
 // Fourier-space d/dlambda: one complex coefficient (m) per thread
 template <typename R>
 __global__ void k_gpmt(const R* in, R* out, int nlon, long total) {
@@ -297,7 +299,8 @@ extern "C" int exo_dyn_destroy(exo_dyn_t d) {
 
 template <typename R>
 static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int exp_gp,
-                    const exo_calcgp_fields* f, hipStream_t s) {
+                    const exo_calcgp_fields* f, hipStream_t s, const double* sid = nullptr,
+                    int nlon = 1, void* rcsq_out = nullptr) {
   CalcgpPtrs<R> p;
   p.gu = (const R*)f->gu;
   p.gv = (const R*)f->gv;
@@ -324,11 +327,14 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
   p.gvq = (R*)f->gvq;
   const DynVert<R> v = vert_of<R>(d);
   dim3 grid((unsigned)((nhor + 255) / 256), (unsigned)nmem);
+  auto launch = [&](auto kern) {
+    kern<<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp, sid, nlon, (R*)rcsq_out);
+  };
   switch (d->nlev) {
-    case 10: k_calcgp<R, 10><<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp); break;
-    case 20: k_calcgp<R, 20><<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp); break;
-    case 40: k_calcgp<R, 40><<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp); break;
-    default: k_calcgp<R, 0><<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp); break;
+    case 10: launch(k_calcgp<R, 10>); break;
+    case 20: launch(k_calcgp<R, 20>); break;
+    case 40: launch(k_calcgp<R, 40>); break;
+    default: launch(k_calcgp<R, 0>); break;
   }
   return hipGetLastError() == hipSuccess ? EXO_OK : EXO_ERR_LAUNCH;
 }
@@ -411,18 +417,6 @@ extern "C" int exo_gridpointa(exo_sht_plan_t p, exo_dyn_t d, int mode, int nmem,
   char* wk = (char*)work;
   auto slot = [&](int k) { return (void*)(wk + es * nhor * k); };
 
-  // 1 / cos^2 per grid point
-  {
-    const dim3 g((unsigned)((nhor + 255) / 256), (unsigned)nmem);
-    if (mode == MODE_F64)
-      k_rcsq<double><<<g, 256, 0, s>>>(tb.sid, tb.nlat, tb.nlon, (double*)slot(sl.rcsq),
-                                        work_stride);
-    else
-      k_rcsq<float><<<g, 256, 0, s>>>(tb.sid, tb.nlat, tb.nlon, (float*)slot(sl.rcsq),
-                                       work_stride);
-    if (hipGetLastError() != hipSuccess) return EXO_ERR_LAUNCH;
-  }
-
   // invlega (src/legmod.f90:635-656) fused with fc2gp, and gpmt
   InvArgs base{};
   base.sp = sp_state;
@@ -449,24 +443,20 @@ extern "C" int exo_gridpointa(exo_sht_plan_t p, exo_dyn_t d, int mode, int nmem,
     a.dst0 = dst0;
     a.nfield = nfield;
     a.dlam = dlam;
-    return launch_inverse(tb, mode, true, a, s);
+    return a;
   };
   // sz sd st (sq, sp) -> gz gd gt (gq, gp); with nqspec = 0 gq is the caller's
-  if (scalar(TQI, 0, sl.gz, nqspec ? nsp : 3 * n, 0)) return EXO_ERR_LAUNCH;
-  if (!nqspec && scalar(TQI, 4 * n, sl.gp, 1, 0)) return EXO_ERR_LAUNCH;
-  if (scalar(TQJ, 4 * n, sl.gpj, 1, 0)) return EXO_ERR_LAUNCH;
-  if (scalar(TQI, 4 * n, sl.gpm, 1, 1)) return EXO_ERR_LAUNCH;
-  {
-    InvArgs a = base;
-    a.kind = INV_UV;
-    a.var = p->uv_var[mode];
-    a.vor0 = 0;
-    a.div0 = n;
-    a.u0 = sl.gu;
-    a.v0 = sl.gv;
-    a.nlev = n;
-    if (launch_inverse(tb, mode, true, a, s)) return EXO_ERR_LAUNCH;
-  }
+  const InvArgs wide = scalar(TQI, 0, sl.gz, nqspec ? nsp : 3 * n, 0);
+  const InvArgs one[3] = {scalar(TQJ, 4 * n, sl.gpj, 1, 0), scalar(TQI, 4 * n, sl.gpm, 1, 1),
+                          scalar(TQI, 4 * n, sl.gp, 1, 0)};
+  InvArgs uv = base;
+  uv.kind = INV_UV;
+  uv.vor0 = 0;
+  uv.div0 = n;
+  uv.u0 = sl.gu;
+  uv.v0 = sl.gv;
+  uv.nlev = n;
+  if (launch_inverse_rt(tb, mode, wide, one, nqspec ? 2 : 3, uv, s)) return EXO_ERR_LAUNCH;
 
   // gp = exp(gp), calcgp and the products (src/plasim.f90:2434-2446)
   exo_calcgp_fields f{};
@@ -493,8 +483,10 @@ extern "C" int exo_gridpointa(exo_sht_plan_t p, exo_dyn_t d, int mode, int nmem,
   f.gke = slot(sl.gke);
   f.guq = nqspec ? slot(sl.guq) : nullptr;
   f.gvq = nqspec ? slot(sl.gvq) : nullptr;
-  int rc = mode == MODE_F64 ? calcgp_t<double>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s)
-                            : calcgp_t<float>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s);
+  int rc = mode == MODE_F64 ? calcgp_t<double>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s,
+                                               tb.sid, tb.nlon, slot(sl.rcsq))
+                            : calcgp_t<float>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s,
+                                              tb.sid, tb.nlon, slot(sl.rcsq));
   if (rc) return rc;
 
   // gp2fc of the nine tendency fields and gvpp, in place

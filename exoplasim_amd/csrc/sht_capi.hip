@@ -532,7 +532,7 @@ static int inverse_all_impl(exo_sht_plan_t p, int mode, int nmem, int nlev, cons
   au.u0 = nfl + 1;
   au.v0 = nfl + 1 + nlev;
   au.nlev = nlev;
-  rc = launch_inverse_rt(t, mode, aq, aj, au, s);
+  rc = launch_inverse_rt(t, mode, aq, &aj, 1, au, s);
   return rc == 0 ? EXO_OK : EXO_ERR_LAUNCH;
 }
 

@@ -69,6 +69,13 @@ struct InvArgs {
   int bpk_f0;
 };
 
+// what differs between the one-field jobs of launch_inverse_rt
+constexpr int INV_ONE_MAX = 3;
+struct InvOneJobs {
+  const void* tab[INV_ONE_MAX];  // packed table
+  int table[INV_ONE_MAX], dst0[INV_ONE_MAX], dlam[INV_ONE_MAX];
+};
+
 struct FwdArgs {
   const void* in;   // grid (fused) or Fourier (unfused) input
   void* sp;         // spectral output (or partial sums when npb > 1)
@@ -117,9 +124,11 @@ int launch_dirx(const Tables& T, int mode, const DirxArgs& a, void* scratch, siz
 size_t dirx_scratch_bytes(const Tables& T, int mode, int nlev);  // nlev: member-levels
 
 int launch_inverse(const Tables& T, int mode, bool fused, const InvArgs& a, hipStream_t s);
-// the sp2fc (aq), sp2fcdmu (aj) and dv2uv (au) transforms of a round trip,
-// fused with fc2gp, in one launch; tile variant aq.var
-int launch_inverse_rt(const Tables& T, int mode, const InvArgs& aq, const InvArgs& aj,
+// the sp2fc run (aq), nj <= INV_ONE_MAX one-field scalar jobs (aj: sp2fc,
+// sp2fcdmu or d/dlambda of one and the same field) and the dv2uv (au) of a
+// round trip or a dynamics step, fused with fc2gp, in one launch; tile
+// variant aq.var
+int launch_inverse_rt(const Tables& T, int mode, const InvArgs& aq, const InvArgs* aj, int nj,
                       const InvArgs& au, hipStream_t s);
 int launch_forward(const Tables& T, int mode, bool fused, const FwdArgs& a, void* scratch,
                    size_t scratch_bytes, hipStream_t s);

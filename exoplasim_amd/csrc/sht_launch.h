@@ -8,8 +8,8 @@ namespace exo {
 template <int MODE>
 int inv_mode(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s);
 template <int MODE>
-int inv_rt_mode(const Tables& tb, const InvArgs& aq, const InvArgs& aj, const InvArgs& au,
-                hipStream_t s);
+int inv_rt_mode(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
+                const InvArgs& au, hipStream_t s);
 template <int MODE>
 int fwd_mode(const Tables& tb, bool fused, const FwdArgs& a, void* scr, size_t sb, hipStream_t s);
 template <int MODE>

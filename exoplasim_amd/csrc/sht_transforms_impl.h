@@ -16,15 +16,22 @@ __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv(InvArgs a, con
                                     tabv, twp, lds);
 }
 
-// The three inverse transforms of a round trip in one launch: per member,
-// the sp2fc blocks (aq, table qi), the sp2fcdmu blocks (aj, table qj) and the
-// dv2uv blocks (au), each block the same work item as in its own kernel.
-// One launch instead of three removes two ramp-up/drain tails, and the
-// blocks of one member (which read the same spectral coefficients) run
-// close together.
+// The inverse transforms of a round trip or of a dynamics step in one launch:
+// per member, the sp2fc blocks (aq, table qi), the blocks of the one-field
+// jobs (aj with the table, destination and d/dlambda switch of job k: a round
+// trip's sp2fcdmu; a dynamics step's sp2fcdmu, d/dlambda and, without
+// spectral humidity, ln ps) and the dv2uv blocks (au), each block the same
+// work item as in its own kernel.  One launch instead of one per transform
+// removes their ramp-up/drain tails, and the blocks of one member (which read
+// the same spectral coefficients) run close together.  (gridpointa with one
+// launch per transform: T21 L10 FP64, one member, 42 us of inverse launches
+// against 15 us; T42 L20, 32 members, 107 us against 74 us.  All scalar jobs
+// as an array of arguments picked by index made the T42 round trip of 128
+// members 1.8% slower: every block then waits for one more scalar load
+// before its arguments.)
 template <int T, int MODE, int V>
 __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv_rt(InvArgs aq, InvArgs aj, InvArgs au, const void* tq,
-                                                const void* tj, const void* tv0, const void* tu,
+                                                InvOneJobs one, const void* tv0, const void* tu,
                                                 long plane, const void* tabv, const void* twp,
                                                 int gq, int gj, int gu) {
   __shared__ __align__(16) char lds[InvLds<T, MODE, true, V>::BYTES];
@@ -53,9 +60,14 @@ __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv_rt(InvArgs aq,
   }
   if (r < NPB * gq)
     inv_body<T, MODE, INV_SCALAR, true, V>(aq, mem * NPB * gq + r, tq, tu, plane, tabv, twp, lds);
-  else if (r < NPB * (gq + gj))
-    inv_body<T, MODE, INV_SCALAR, true, V>(aj, mem * NPB * gj + (r - NPB * gq), tj, tu, plane,
-                                           tabv, twp, lds);
+  else if (r < NPB * (gq + gj)) {
+    const int k = __builtin_amdgcn_readfirstlane((r - NPB * gq) / NPB);
+    aj.table = one.table[k];
+    aj.dst0 = one.dst0[k];
+    aj.dlam = one.dlam[k];
+    inv_body<T, MODE, INV_SCALAR, true, V>(aj, mem * NPB + (r - NPB * (gq + k)), one.tab[k], tu,
+                                           plane, tabv, twp, lds);
+  }
   else
     inv_body<T, MODE, INV_UV, true, V>(au, mem * NPB * gu + (r - NPB * (gq + gj)), tv0, tu, plane,
                                        tabv, twp, lds);
@@ -129,47 +141,54 @@ static int inv_t(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s) 
 }
 
 template <int T, int MODE, int V>
-static int inv_rt_tv(const Tables& tb, const InvArgs& aq, const InvArgs& aj, const InvArgs& au,
-                     hipStream_t s) {
+static int inv_rt_tv(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
+                     const InvArgs& au, hipStream_t s) {
   using C = InvCfg<T, MODE, V>;
   constexpr int NPB = TS<T>::NPAIR / C::LP;
-  if (aq.nmem != aj.nmem || aq.nmem != au.nmem) return -1;
+  if (nj < 1 || nj > INV_ONE_MAX || aq.nmem != au.nmem) return -1;
   const int gq = (aq.nfield + C::FB - 1) / C::FB;
-  const int gj = (aj.nfield + C::FB - 1) / C::FB;
   const int gu = (au.nlev + C::FB / 2 - 1) / (C::FB / 2);
-  const long nblk = (long)aq.nmem * NPB * (gq + gj + gu);
+  const long nblk = (long)aq.nmem * NPB * (gq + nj + gu);
   if (nblk <= 0) return 0;
-  const void *tq = nullptr, *tj = nullptr, *tv0 = nullptr, *tu = nullptr;
+  InvOneJobs one{};
+  for (int k = 0; k < nj; ++k) {
+    const InvArgs& a = aj[k];
+    if (a.nmem != aq.nmem || a.nfield != 1 || a.src0 != aj[0].src0) return -1;
+    one.tab[k] = MODE == MODE_BF16X3    ? (const void*)tb.inv_bf[a.table]
+                 : MODE == MODE_F32MFMA ? (const void*)tb.inv_f32[a.table]
+                                        : (const void*)tb.inv_f64[a.table];
+    one.table[k] = a.table;
+    one.dst0[k] = a.dst0;
+    one.dlam[k] = a.dlam;
+  }
+  const void *tq = nullptr, *tv0 = nullptr, *tu = nullptr;
   if (MODE == MODE_BF16X3) {
     tq = tb.inv_bf[TQI];
-    tj = tb.inv_bf[TQJ];
     tv0 = tb.inv_bf[TQV];
     tu = tb.inv_bf[TQU];
   } else if (MODE == MODE_F32MFMA) {
     tq = tb.inv_f32[TQI];
-    tj = tb.inv_f32[TQJ];
     tv0 = tb.inv_f32[TQV];
     tu = tb.inv_f32[TQU];
   } else if (MODE == MODE_F64) {
     tq = tb.inv_f64[TQI];
-    tj = tb.inv_f64[TQJ];
     tv0 = tb.inv_f64[TQV];
     tu = tb.inv_f64[TQU];
   }
   const void* tv = (MODE == MODE_F64) ? (const void*)tb.filt64 : (const void*)tb.filt32;
   const void* tw = (MODE == MODE_F64) ? (const void*)tb.tw64 : (const void*)tb.tw32;
-  k_inv_rt<T, MODE, V><<<(unsigned)nblk, C::NT, 0, s>>>(aq, aj, au, tq, tj, tv0, tu, tb.inv_elems,
-                                                       tv, tw, gq, gj, gu);
+  k_inv_rt<T, MODE, V><<<(unsigned)nblk, C::NT, 0, s>>>(aq, aj[0], au, tq, one, tv0, tu,
+                                                       tb.inv_elems, tv, tw, gq, nj, gu);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 template <int T, int MODE>
-static int inv_rt_t(const Tables& tb, const InvArgs& aq, const InvArgs& aj, const InvArgs& au,
-                    hipStream_t s) {
-  if (aq.var == 1) return inv_rt_tv<T, MODE, 1>(tb, aq, aj, au, s);
-  if (aq.var == 2) return inv_rt_tv<T, MODE, 2>(tb, aq, aj, au, s);
-  if (aq.var == 3) return inv_rt_tv<T, MODE, 3>(tb, aq, aj, au, s);
-  return inv_rt_tv<T, MODE, 0>(tb, aq, aj, au, s);
+static int inv_rt_t(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
+                    const InvArgs& au, hipStream_t s) {
+  if (aq.var == 1) return inv_rt_tv<T, MODE, 1>(tb, aq, aj, nj, au, s);
+  if (aq.var == 2) return inv_rt_tv<T, MODE, 2>(tb, aq, aj, nj, au, s);
+  if (aq.var == 3) return inv_rt_tv<T, MODE, 3>(tb, aq, aj, nj, au, s);
+  return inv_rt_tv<T, MODE, 0>(tb, aq, aj, nj, au, s);
 }
 
 template <int T, int MODE>
@@ -227,9 +246,9 @@ int inv_mode(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s) {
   EXO_DISPATCH_T(inv_t, tb, fused, a, s)
 }
 template <int MODE_X>
-int inv_rt_mode(const Tables& tb, const InvArgs& aq, const InvArgs& aj, const InvArgs& au,
-                hipStream_t s) {
-  EXO_DISPATCH_T(inv_rt_t, tb, aq, aj, au, s)
+int inv_rt_mode(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
+                const InvArgs& au, hipStream_t s) {
+  EXO_DISPATCH_T(inv_rt_t, tb, aq, aj, nj, au, s)
 }
 template <int MODE_X>
 int fwd_mode(const Tables& tb, bool fused, const FwdArgs& a, void* scr, size_t sb,
