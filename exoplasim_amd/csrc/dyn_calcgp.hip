@@ -494,44 +494,16 @@ extern "C" int exo_gridpointa(exo_sht_plan_t p, exo_dyn_t d, int mode, int nmem,
                  work_stride))
     return EXO_ERR_LAUNCH;
 
-  // scratch of the multi-block direct sums
-  const size_t need = std::max(forward_scratch_bytes(tb, mode, nmem, 1),
-                               dirx_scratch_bytes(tb, mode, nmem * n));
-  if (need > 0 && (rc = plan_grow(&p->scratch, &p->scratch_bytes, need)) != 0) return rc;
-
-  // fc2sp(gvpp) -> spt (field 4 nlev of the tendencies)
-  {
-    FwdArgs a{};
-    a.in = work;
-    a.sp = sp_tend;
-    a.in_stride = work_stride;
-    a.sp_stride = tend_stride;
-    a.nmem = nmem;
-    a.src0 = sl.gvp;
-    a.dst0 = 4 * n;
-    a.nfield = 1;
-    a.table = TQC;
-    if (launch_forward(tb, mode, false, a, p->scratch, p->scratch_bytes, s))
-      return EXO_ERR_LAUNCH;
-  }
-  // mktend -> sdt, stt, szt; qtend -> sqt (src/plasim.f90:2473-2486)
-  auto dirx = [&](const DirxTerm* terms, int nterm, std::initializer_list<int> ins, int out) {
-    DirxArgs a{};
-    int i = 0;
-    for (int k : ins) a.in[i++] = slot(k);
-    a.nin = i;
-    a.out = (char*)sp_tend + es * 2 * tb.ncsp * out;
-    a.nlev = n;
-    a.nmem = nmem;
-    a.in_stride = work_stride;
-    a.out_stride = tend_stride;
-    a.nterm = nterm;
-    for (int t = 0; t < nterm; ++t) a.terms[t] = terms[t];
-    return launch_dirx(tb, mode, a, p->scratch, p->scratch_bytes, s);
-  };
-  if (dirx(MKTEND_D, 6, {sl.gke, sl.guz, sl.gvz}, n)) return EXO_ERR_LAUNCH;
-  if (dirx(MKTEND_T, 6, {sl.gvt, sl.gtn, sl.gut}, 2 * n)) return EXO_ERR_LAUNCH;
-  if (dirx(MKTEND_Z, 4, {sl.gvz, sl.guz}, 0)) return EXO_ERR_LAUNCH;
-  if (nqspec && dirx(QTEND_Q, 6, {sl.gqn, sl.guq, sl.gvq}, 3 * n)) return EXO_ERR_LAUNCH;
+  // mktend -> szt, sdt, stt; qtend -> sqt; fc2sp(gvpp) -> spt (src/plasim.f90:2473-2486)
+  auto out = [&](int k) { return (void*)((char*)sp_tend + es * 2 * tb.ncsp * k); };
+  const DirxArgs jobs[4] = {
+      mktend_dz(slot(sl.gke), slot(sl.guz), slot(sl.gvz), out(n), out(0), n, nmem, work_stride,
+                tend_stride),
+      mktend_t(slot(sl.gvt), slot(sl.gtn), slot(sl.gut), out(2 * n), n, nmem, work_stride,
+               tend_stride),
+      fc2sp_job(slot(sl.gvp), out(4 * n), TQC, 1, nmem, work_stride, tend_stride),
+      mktend_t(slot(sl.gvq), slot(sl.gqn), slot(sl.guq), out(3 * n), n, nmem, work_stride,
+               tend_stride)};
+  if (launch_dirx(tb, mode, jobs, nqspec ? 4 : 3, s)) return EXO_ERR_LAUNCH;
   return EXO_OK;
 }

@@ -815,67 +815,41 @@ extern "C" int exo_fc2gp_f32(float* a, int n, int lot) { return fft_impl<float>(
 // ---------------------------------------------------------------------------
 // multi-input direct transforms (uv2dv, qtend, mktend)
 // ---------------------------------------------------------------------------
-// run one output field of a multi-input direct transform over nlev levels;
-// din[i] are device copies of the inputs
-template <typename R>
-static int dirx_one(exo_sht_plan_s* p, const R* const* din, int nin, R* dout,
-                    std::initializer_list<DirxTerm> terms) {
-  const int mode = sizeof(R) == 8 ? MODE_F64 : MODE_F32;
-  DirxArgs a{};
-  for (int i = 0; i < nin; ++i) a.in[i] = din[i];
-  a.out = dout;
-  a.nin = nin;
-  a.nlev = p->nlev;
-  a.nmem = 1;
-  a.nterm = 0;
-  for (const DirxTerm& t : terms) a.terms[a.nterm++] = t;
-  const size_t need = dirx_scratch_bytes(p->tb, mode, p->nlev);
-  if (need > 0) {
-    int rc = plan_grow(&p->scratch, &p->scratch_bytes, need);
-    if (rc) return rc;
-  }
-  return launch_dirx(p->tb, mode, a, p->scratch, p->scratch_bytes, 0);
-}
-
-// stage nin Fourier inputs and nout spectral outputs (all nlev levels)
+// stage the Fourier inputs (all nlev levels of each), run fn(plan, device
+// inputs, device outputs, values per input / output) and copy the outputs back
 template <typename R, typename Fn>
-static int dirx_staged(const R* const* in, int nin, R* const* out, int nout, Fn run) {
-  for (int i = 0; i < nin; ++i)
-    if (!in[i]) return EXO_ERR_ARG;
-  for (int o = 0; o < nout; ++o)
-    if (!out[o]) return EXO_ERR_ARG;
+static int dirx_staged(std::initializer_list<const R*> in, std::initializer_list<R*> out, Fn run) {
+  for (const R* x : in)
+    if (!x) return EXO_ERR_ARG;
+  for (R* x : out)
+    if (!x) return EXO_ERR_ARG;
   return with_plan([&](exo_sht_plan_s* pl) {
     const Tables& t = pl->tb;
     const long nhor = (long)t.nlat * t.nlon * pl->nlev;
     const long nsp = 2L * t.ncsp * pl->nlev;
-    std::vector<R> hin(nhor * nin), hout(nsp * nout);
-    for (int i = 0; i < nin; ++i) memcpy(hin.data() + i * nhor, in[i], sizeof(R) * nhor);
+    std::vector<R> hin(nhor * in.size()), hout(nsp * out.size());
+    long k = 0;
+    for (const R* x : in) memcpy(hin.data() + nhor * k++, x, sizeof(R) * nhor);
     int rc = staged<R>(pl, hin.size(), hin.data(), hout.size(), hout.data(),
-                       [&](exo_sht_plan_s* p, R* din, R* dout) {
-                         const R* ins[3] = {din, din + nhor, din + 2 * nhor};
-                         R* outs[3] = {dout, dout + nsp, dout + 2 * nsp};
-                         return run(p, ins, outs);
-                       });
+                       [&](exo_sht_plan_s* p, R* din, R* dout) { return run(p, din, dout, nhor, nsp); });
     if (rc) return rc;
-    for (int o = 0; o < nout; ++o) memcpy(out[o], hout.data() + o * nsp, sizeof(R) * nsp);
+    k = 0;
+    for (R* x : out) memcpy(x, hout.data() + nsp * k++, sizeof(R) * nsp);
     return EXO_OK;
   });
+}
+
+template <typename R>
+constexpr int mode_of_kind() {
+  return sizeof(R) == 8 ? MODE_F64 : MODE_F32;
 }
 
 // uv2dv(pu, pv, pd, pz), src/legmod.f90:356 (folded branch)
 template <typename R>
 static int uv2dv_impl(const R* pu, const R* pv, R* pd, R* pz) {
-  const R* in[2] = {pu, pv};
-  R* out[2] = {pd, pz};
-  return dirx_staged<R>(in, 2, out, 2, [&](exo_sht_plan_s* p, const R** din, R** dout) {
-    // pd = -qe.v + i qm.u ; pz = qe.u + i qm.v   (inputs 0 = u, 1 = v)
-    int rc = dirx_one<R>(p, din, 2, dout[0],
-                         {{1, 0, 0, -1, TQE}, {0, 1, 0, -1, TQM},
-                          {1, 1, 1, -1, TQE}, {0, 0, 1, +1, TQM}});
-    if (rc) return rc;
-    return dirx_one<R>(p, din, 2, dout[1],
-                       {{0, 0, 0, +1, TQE}, {1, 1, 0, -1, TQM},
-                        {0, 1, 1, +1, TQE}, {1, 0, 1, +1, TQM}});
+  return dirx_staged<R>({pu, pv}, {pd, pz}, [](exo_sht_plan_s* p, R* in, R* out, long f, long s) {
+    const DirxArgs a = uv2dv_dz(in, in + f, out, out + s, p->nlev, 1, 0, 0);
+    return launch_dirx(p->tb, mode_of_kind<R>(), &a, 1, 0);
   });
 }
 extern "C" int exo_uv2dv_f64(const double* pu, const double* pv, double* pd, double* pz) {
@@ -888,13 +862,9 @@ extern "C" int exo_uv2dv_f32(const float* pu, const float* pv, float* pd, float*
 // qtend(q, qn, uq, vq), src/legmod.f90:433 (folded branch)
 template <typename R>
 static int qtend_impl(R* q, const R* qn, const R* uq, const R* vq) {
-  const R* in[3] = {qn, uq, vq};
-  R* out[1] = {q};
-  return dirx_staged<R>(in, 3, out, 1, [&](exo_sht_plan_s* p, const R** din, R** dout) {
-    // q = qe.vq + qc.qn - i qm.uq   (inputs 0 = qn, 1 = uq, 2 = vq)
-    return dirx_one<R>(p, din, 3, dout[0],
-                       {{2, 0, 0, +1, TQE}, {0, 0, 0, +1, TQC}, {1, 1, 0, +1, TQM},
-                        {2, 1, 1, +1, TQE}, {0, 1, 1, +1, TQC}, {1, 0, 1, -1, TQM}});
+  return dirx_staged<R>({vq, qn, uq}, {q}, [](exo_sht_plan_s* p, R* in, R* out, long f, long) {
+    const DirxArgs a = mktend_t(in, in + f, in + 2 * f, out, p->nlev, 1, 0, 0);
+    return launch_dirx(p->tb, mode_of_kind<R>(), &a, 1, 0);
   });
 }
 extern "C" int exo_qtend_f64(double* q, const double* qn, const double* uq, const double* vq) {
@@ -908,37 +878,14 @@ extern "C" int exo_qtend_f32(float* q, const float* qn, const float* uq, const f
 template <typename R>
 static int mktend_impl(R* d, R* t, R* z, const R* tn, const R* fu, const R* fv, const R* ke,
                        const R* ut, const R* vt) {
-  const R* in_d[3] = {ke, fv, fu};
-  const R* in_t[3] = {vt, tn, ut};
-  const R* in_z[2] = {fu, fv};
-  int rc;
-  {
-    R* out[1] = {d};
-    // D = qq.ke - qe.fv + i qm.fu   (0 = ke, 1 = fv, 2 = fu)
-    rc = dirx_staged<R>(in_d, 3, out, 1, [&](exo_sht_plan_s* p, const R** din, R** dout) {
-      return dirx_one<R>(p, din, 3, dout[0],
-                         {{0, 0, 0, +1, TQQ}, {1, 0, 0, -1, TQE}, {2, 1, 0, -1, TQM},
-                          {0, 1, 1, +1, TQQ}, {1, 1, 1, -1, TQE}, {2, 0, 1, +1, TQM}});
-    });
-    if (rc) return rc;
-  }
-  {
-    R* out[1] = {t};
-    // T = qe.vt + qc.tn - i qm.ut   (0 = vt, 1 = tn, 2 = ut)
-    rc = dirx_staged<R>(in_t, 3, out, 1, [&](exo_sht_plan_s* p, const R** din, R** dout) {
-      return dirx_one<R>(p, din, 3, dout[0],
-                         {{0, 0, 0, +1, TQE}, {1, 0, 0, +1, TQC}, {2, 1, 0, +1, TQM},
-                          {0, 1, 1, +1, TQE}, {1, 1, 1, +1, TQC}, {2, 0, 1, -1, TQM}});
-    });
-    if (rc) return rc;
-  }
-  R* out[1] = {z};
-  // Z = qe.fu + i qm.fv   (0 = fu, 1 = fv)
-  return dirx_staged<R>(in_z, 2, out, 1, [&](exo_sht_plan_s* p, const R** din, R** dout) {
-    return dirx_one<R>(p, din, 2, dout[0],
-                       {{0, 0, 0, +1, TQE}, {1, 1, 0, -1, TQM},
-                        {0, 1, 1, +1, TQE}, {1, 0, 1, +1, TQM}});
-  });
+  return dirx_staged<R>({ke, fv, fu, vt, tn, ut}, {d, z, t},
+                        [](exo_sht_plan_s* p, R* in, R* out, long f, long s) {
+                          const DirxArgs a[2] = {
+                              mktend_dz(in, in + f, in + 2 * f, out, out + s, p->nlev, 1, 0, 0),
+                              mktend_t(in + 3 * f, in + 4 * f, in + 5 * f, out + 2 * s, p->nlev,
+                                       1, 0, 0)};
+                          return launch_dirx(p->tb, mode_of_kind<R>(), a, 2, 0);
+                        });
 }
 extern "C" int exo_mktend_f64(double* d, double* t, double* z, const double* tn,
                               const double* fu, const double* fv, const double* ke,
@@ -997,29 +944,8 @@ extern "C" int exo_sht_fft(exo_sht_plan_t p, int mode, int dir, void* a, long lo
   return rc == 0 ? EXO_OK : (rc == -2 ? EXO_ERR_UNSUPPORTED : EXO_ERR_LAUNCH);
 }
 
-// one output field of a multi-term direct transform over nmem members x
-// nlev levels of device Fourier arrays
-static int dirx_dev(exo_sht_plan_t p, int mode, int nmem, int nlev, const void* const* in,
-                    int nin, long in_stride, void* out, long out_stride,
-                    std::initializer_list<DirxTerm> terms, hipStream_t s) {
-  DirxArgs a{};
-  for (int i = 0; i < nin; ++i) a.in[i] = in[i];
-  a.out = out;
-  a.nin = nin;
-  a.nlev = nlev;
-  a.nmem = nmem;
-  a.in_stride = in_stride;
-  a.out_stride = out_stride;
-  a.nterm = 0;
-  for (const DirxTerm& t : terms) a.terms[a.nterm++] = t;
-  const size_t need = dirx_scratch_bytes(p->tb, mode, nmem * nlev);
-  if (need > 0) {
-    const int rc = plan_grow(&p->scratch, &p->scratch_bytes, need);
-    if (rc) return rc;
-  }
-  const int rc = launch_dirx(p->tb, mode, a, p->scratch, p->scratch_bytes, s);
-  return rc == 0 ? EXO_OK : (rc == -4 ? EXO_ERR_SCRATCH : EXO_ERR_LAUNCH);
-}
+// status of a launch_dirx on device arrays
+static int dirx_status(int rc) { return rc == 0 ? EXO_OK : EXO_ERR_LAUNCH; }
 
 static bool all_set(std::initializer_list<const void*> ps) {
   for (const void* q : ps)
@@ -1035,16 +961,8 @@ extern "C" int exo_sht_uv2dv(exo_sht_plan_t p, int mode, int nmem, int nlev, con
     return EXO_ERR_ARG;
   if (nmem == 0 || nlev == 0) return EXO_OK;
   std::lock_guard<std::mutex> lk(p->mu);
-  hipStream_t s = (hipStream_t)stream;
-  const void* in[2] = {pu, pv};
-  // pd = -qe.v + i qm.u ; pz = qe.u + i qm.v   (inputs 0 = u, 1 = v)
-  int rc = dirx_dev(p, mode, nmem, nlev, in, 2, f_stride, pd, s_stride,
-                    {{1, 0, 0, -1, TQE}, {0, 1, 0, -1, TQM}, {1, 1, 1, -1, TQE}, {0, 0, 1, +1, TQM}},
-                    s);
-  if (rc) return rc;
-  return dirx_dev(p, mode, nmem, nlev, in, 2, f_stride, pz, s_stride,
-                  {{0, 0, 0, +1, TQE}, {1, 1, 0, -1, TQM}, {0, 1, 1, +1, TQE}, {1, 0, 1, +1, TQM}},
-                  s);
+  const DirxArgs a = uv2dv_dz(pu, pv, pd, pz, nlev, nmem, f_stride, s_stride);
+  return dirx_status(launch_dirx(p->tb, mode, &a, 1, (hipStream_t)stream));
 }
 
 extern "C" int exo_sht_qtend(exo_sht_plan_t p, int mode, int nmem, int nlev, void* q,
@@ -1055,12 +973,8 @@ extern "C" int exo_sht_qtend(exo_sht_plan_t p, int mode, int nmem, int nlev, voi
     return EXO_ERR_ARG;
   if (nmem == 0 || nlev == 0) return EXO_OK;
   std::lock_guard<std::mutex> lk(p->mu);
-  const void* in[3] = {qn, uq, vq};
-  // q = qe.vq + qc.qn - i qm.uq   (inputs 0 = qn, 1 = uq, 2 = vq)
-  return dirx_dev(p, mode, nmem, nlev, in, 3, f_stride, q, s_stride,
-                  {{2, 0, 0, +1, TQE}, {0, 0, 0, +1, TQC}, {1, 1, 0, +1, TQM},
-                   {2, 1, 1, +1, TQE}, {0, 1, 1, +1, TQC}, {1, 0, 1, -1, TQM}},
-                  (hipStream_t)stream);
+  const DirxArgs a = mktend_t(vq, qn, uq, q, nlev, nmem, f_stride, s_stride);
+  return dirx_status(launch_dirx(p->tb, mode, &a, 1, (hipStream_t)stream));
 }
 
 extern "C" int exo_sht_mktend(exo_sht_plan_t p, int mode, int nmem, int nlev, void* d, void* t,
@@ -1072,24 +986,7 @@ extern "C" int exo_sht_mktend(exo_sht_plan_t p, int mode, int nmem, int nlev, vo
     return EXO_ERR_ARG;
   if (nmem == 0 || nlev == 0) return EXO_OK;
   std::lock_guard<std::mutex> lk(p->mu);
-  hipStream_t s = (hipStream_t)stream;
-  // D = qq.ke - qe.fv + i qm.fu   (0 = ke, 1 = fv, 2 = fu)
-  const void* in_d[3] = {ke, fv, fu};
-  int rc = dirx_dev(p, mode, nmem, nlev, in_d, 3, f_stride, d, s_stride,
-                    {{0, 0, 0, +1, TQQ}, {1, 0, 0, -1, TQE}, {2, 1, 0, -1, TQM},
-                     {0, 1, 1, +1, TQQ}, {1, 1, 1, -1, TQE}, {2, 0, 1, +1, TQM}},
-                    s);
-  if (rc) return rc;
-  // T = qe.vt + qc.tn - i qm.ut   (0 = vt, 1 = tn, 2 = ut)
-  const void* in_t[3] = {vt, tn, ut};
-  rc = dirx_dev(p, mode, nmem, nlev, in_t, 3, f_stride, t, s_stride,
-                {{0, 0, 0, +1, TQE}, {1, 0, 0, +1, TQC}, {2, 1, 0, +1, TQM},
-                 {0, 1, 1, +1, TQE}, {1, 1, 1, +1, TQC}, {2, 0, 1, -1, TQM}},
-                s);
-  if (rc) return rc;
-  // Z = qe.fu + i qm.fv   (0 = fu, 1 = fv)
-  const void* in_z[2] = {fu, fv};
-  return dirx_dev(p, mode, nmem, nlev, in_z, 2, f_stride, z, s_stride,
-                  {{0, 0, 0, +1, TQE}, {1, 1, 0, -1, TQM}, {0, 1, 1, +1, TQE}, {1, 0, 1, +1, TQM}},
-                  s);
+  const DirxArgs a[2] = {mktend_dz(ke, fv, fu, d, z, nlev, nmem, f_stride, s_stride),
+                         mktend_t(vt, tn, ut, t, nlev, nmem, f_stride, s_stride)};
+  return dirx_status(launch_dirx(p->tb, mode, a, 2, (hipStream_t)stream));
 }

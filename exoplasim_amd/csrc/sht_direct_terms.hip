@@ -6,162 +6,121 @@
 // Each output field is a sum of terms  sign * t[pair][w] * X_i[m][cls][pair][c]
 // where X_i is input i folded into E = N+S (class sym) / O = N-S (class anti)
 // and the class of table t at (m,n) is sym iff (n-m even) != (t is Q-type).
-// One launch computes one output field (re and im) for every level; the
-// caller launches once per output.  FP64 runs k_dirx (VALU sums, one block
-// per level and latitude-pair block); the FP32 modes run k_dirx_mf (MFMA,
-// 8 levels per block).
+//
+// Per zonal wavenumber m and parity p of n - m, each output is a GEMM over
+// the latitude pairs:  C[n][lev, oc] = sum_t sum_pair A_t[n][pair] B_t[pair][lev, oc]
+// with A_t the table t at the rows n = m + p + 2j and B_t[pair][lev, oc] =
+// sign * X_in[cls][pair][m][lev][ic] for the term of table t and output
+// component oc.  One 16x16x4 MFMA (v_mfma_f32_16x16x4_f32, in the FP64 mode
+// v_mfma_f64_16x16x4_f64) takes 16 rows n x 4 pairs of A and 4 pairs x 16
+// columns (8 levels x re/im) of B, so each table value serves 8 levels.
+//
+// A block owns one member, 8 levels and MR wavenumbers of one job: up to 3
+// inputs (one table each) and up to 2 outputs that share them.  It walks the
+// latitude pairs KC at a time: the folded Fourier values of those pairs
+// (all inputs, its levels and wavenumbers) are staged in LDS, every table
+// operand of the step is requested, then the next pairs' values, and the
+// MFMAs run while those are in flight; every (output, m, p, row tile)
+// accumulates in registers across all pairs, so the sum over latitudes is
+// complete in the block (no partial sums).  Wave w takes m = m0 + w.
+//
+// What bounds it is the latency of those steps (stage, barrier, tables), not
+// bytes or flops, so the jobs of one call run in one launch: the blocks of
+// mktend's and gridpointa's four outputs overlap, and divergence and
+// vorticity, which share two of their inputs and tables, are one job (one
+// launch per output before: mktend of T42 L20, 32 members, FP32, 69.6 -> 51
+// us; T63, 16 members, 81 -> 57; T127 L40, 4 members, 242 -> 184).  In FP64
+// the vector and matrix peaks are equal; the matrix form wins over one thread
+// per coefficient, which read each table value once per level, by that reuse
+// (mktend T42 251 -> 95 us, T63 388 -> 101, T127 2320 -> 273), and needs no
+// partial sums in scratch.
 #include <type_traits>
 
 #include "sht_internal.h"
 
 namespace exo {
 
-template <int MODE>
-using RealX = typename std::conditional<MODE == MODE_F64, double, float>::type;
+constexpr int DIRX_MR = 8;  // wavenumbers per block, one per wave
+constexpr int DIRX_NT = 512, DIRX_LG = 8;  // threads, levels per block
 
-// latitude pairs per block so that 3 folded FP64 inputs fit in about
-// 100 KB of LDS
-template <int T, int MODE>
+template <int T, typename R, int NIN>
 struct DirxCfg {
-  static constexpr int PB = (T == 21) ? 16 : (T == 42) ? 16 : (T == 63) ? 12 : 8;
-  static constexpr int NPB = TS<T>::NPAIR / PB;
+  static constexpr int NMR = (TS<T>::NM + DIRX_MR - 1) / DIRX_MR;
+  // Pairs per step: as many as the step's table operands allow in registers
+  // (fewer inputs, more pairs).  FP64 operands take twice the registers and
+  // the LDS.
+  static constexpr int KC = (sizeof(R) == 8) ? ((NIN == 1) ? 8 : 4)
+                            : (NIN == 1)     ? ((T == 127) ? 8 : 16)
+                            : (T == 127)     ? ((NIN == 2) ? 8 : 4)
+                            : (NIN == 3)     ? 8
+                            : (T == 63)      ? 16
+                                             : 8;
+  static constexpr int KS = DIRX_LG * 2 * DIRX_MR + 2;  // reals per (input, class, pair), padded
+  static constexpr size_t LDS = sizeof(R) * NIN * 2 * KC * KS;
 };
 
-template <int T, int MODE>
-__global__ __launch_bounds__(256) void k_dirx(DirxArgs a, const void* tabv, void* scratch) {
+// one job: the term list regrouped by table.  Slot s multiplies table tab[s]
+// by, for output o and component oc, sign[o][s][oc] * X_in[o][s][oc] component
+// ic[o][s][oc] (sign 0: no term); every list here has one table per input.
+template <typename R>
+struct DirxJob {
+  const R* in[3];
+  R* out[2];
+  const R* tab[3];  // FP32: the packed table (k_pack_dir); FP64: [pair][w]
+  int nin, nout, nlev, nlg;
+  long in_stride, out_stride;
+  int8_t sign[2][3][2], src[2][3][2], ic[2][3][2], isq[3];
+};
+constexpr int DIRX_JOBS = 4;
+template <typename R>
+struct DirxJobs {
+  int njob, nmem, per;        // per: blocks per member
+  int start[DIRX_JOBS + 1];   // first block of each job within a member
+  DirxJob<R> job[DIRX_JOBS];
+};
+
+template <int T, typename R, int NIN, int NOUT>
+__device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, int mr,
+                                          char* lds) {
   using S = TS<T>;
-  using R = RealX<MODE>;
-  constexpr int NM = S::NM, N = S::NLON, NLAT = S::NLAT;
-  constexpr int PB = DirxCfg<T, MODE>::PB, NPB = DirxCfg<T, MODE>::NPB;
-  // X[i][m][cls][pair][ri]
-  __shared__ R X[3 * NM * 2 * PB * 2];
-  __shared__ uint8_t mw[S::NCSP];
-  const int tid = threadIdx.x;
-  const int pb = blockIdx.x % NPB;
-  const int ml = blockIdx.x / NPB;  // member * nlev + level
-  if (ml >= a.nmem * a.nlev) return;
-  const int mem = ml / a.nlev, lev = ml - mem * a.nlev;
-  for (int m = tid; m <= T; m += 256)
-    for (int n = m; n <= T; ++n) mw[w0_of(T, m) + n - m] = (uint8_t)m;
-  auto xi = [](int i, int m, int cls, int pl, int ri) {
-    return (((i * NM + m) * 2 + cls) * PB + pl) * 2 + ri;
-  };
-  for (int idx = tid; idx < a.nin * PB * NM; idx += 256) {
-    const int pl = idx % PB, k = (idx / PB) % NM, i = idx / (PB * NM);
-    const int lat = pb * PB + pl;
-    const R* src = (const R*)a.in[i] + mem * a.in_stride + (long)lev * NLAT * N;
-    const R nx = src[(long)lat * N + 2 * k], ny = src[(long)lat * N + 2 * k + 1];
-    const R sx = src[(long)(NLAT - 1 - lat) * N + 2 * k];
-    const R sy = src[(long)(NLAT - 1 - lat) * N + 2 * k + 1];
-    X[xi(i, k, 0, pl, 0)] = nx + sx;
-    X[xi(i, k, 0, pl, 1)] = ny + sy;
-    X[xi(i, k, 1, pl, 0)] = nx - sx;
-    X[xi(i, k, 1, pl, 1)] = ny - sy;
-  }
-  __syncthreads();
-  const R* tv = (const R*)tabv;
-  const long tsz = (long)S::NPAIR * S::NCSP;
-  R* out;
-  if (NPB == 1)
-    out = (R*)a.out + mem * a.out_stride + (long)lev * S::NRSP;
-  else
-    out = (R*)scratch + ((long)pb * a.nmem * a.nlev + ml) * S::NRSP;
-  for (int w = tid; w < S::NCSP; w += 256) {
-    const int m = mw[w];
-    const int n = m + (w - w0_of(T, m));
-    const bool even = ((n - m) & 1) == 0;
-    R acc[2] = {R(0), R(0)};
-    for (int t = 0; t < a.nterm; ++t) {
-      const DirxTerm tm = a.terms[t];
-      const int cls = (even != table_is_q(tm.table)) ? 0 : 1;
-      const R* tp = tv + tm.table * tsz + (long)(pb * PB) * S::NCSP + w;
-      R s = R(0);
-      for (int pl = 0; pl < PB; ++pl) s += tp[(long)pl * S::NCSP] * X[xi(tm.in, m, cls, pl, tm.ic)];
-      acc[tm.oc] += tm.sign > 0 ? s : -s;
-    }
-    out[2 * w] = acc[0];
-    out[2 * w + 1] = acc[1];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// the same sums on MFMA (FP32 modes)
-// ---------------------------------------------------------------------------
-// Per zonal wavenumber m and parity p of n - m, each output is a GEMM over
-// the latitude pairs:  C[n][lev, oc] = sum_t sum_pair A_t[n][pair] B_t[pair][lev, oc]
-// with A_t the table t at the rows n = m + p + 2j (packed by k_pack_dir) and
-// B_t[pair][lev, oc] = sign * X_in[cls][pair][m][lev][ic] for the term of
-// table t and output component oc.  One v_mfma_f32_16x16x4_f32 takes 16 rows
-// n x 4 pairs of A and 4 pairs x 16 columns (8 levels x re/im) of B.
-//
-// A block owns one member, 8 levels and a range of MR wavenumbers; it walks
-// the latitude pairs KC at a time: the folded Fourier values of those pairs
-// (all inputs, its levels and wavenumbers) are staged in LDS, every table
-// operand of the step is requested, then the next pairs' values, and the
-// MFMAs run while those are in flight; every (m, p, row tile) accumulates in
-// registers across all pairs, so the sum over latitudes is complete in the
-// block (no partial sums).  Wave w takes m = m0 + w, m0 + w + 8, ...  KC is
-// as large as the step's table operands allow in registers: fewer inputs
-// (tables), more pairs per step.
-template <int T, int NIN>
-struct DirxMfCfg {
-  static constexpr int MR = 8;  // wavenumbers per block
-  static constexpr int NMR = (TS<T>::NM + MR - 1) / MR;
-  static constexpr int NT = 512, NW = NT / 64;
-  static constexpr int MPW = (MR + NW - 1) / NW;                     // wavenumbers per wave
-  static constexpr int LG = 8;                                       // levels per block
-  static constexpr int KC = (NIN == 1) ? ((T == 127) ? 8 : 16) : (T == 127) ? ((NIN == 2) ? 8 : 4) : (NIN == 3) ? 8 : (T == 63) ? 16 : 8;  // pairs per step
-  static constexpr int KS = LG * 2 * MR + 2;  // floats per (input, class, pair), padded
-};
-
-// the term list regrouped by table: slot s multiplies table tab[s] by, for
-// output component oc, sign[s][oc] * X_in[s][oc] component ic[s][oc]; every
-// term list here has one table per input (mktend, qtend, uv2dv, fc2sp)
-constexpr int NSLOT = 3;
-struct DirxSlots {
-  const float* tab[NSLOT];
-  float sign[NSLOT][2];
-  int in[NSLOT][2], ic[NSLOT][2];
-  int isq[NSLOT];
-  int nslot;
-};
-
-template <int T, int NIN>
-__global__ __launch_bounds__(512) void k_dirx_mf(DirxArgs a, DirxSlots sl) {
-  using S = TS<T>;
-  using C = DirxMfCfg<T, NIN>;
-  constexpr int N = S::NLON, NLAT = S::NLAT, NPAIR = S::NPAIR, RB = S::RB;
-  constexpr int MR = C::MR, LG = C::LG, KC = C::KC, KS = C::KS, MPW = C::MPW, NT = C::NT;
+  using C = DirxCfg<T, R, NIN>;
+  using R2 = R __attribute__((ext_vector_type(2)));
+  using Acc = typename std::conditional<sizeof(R) == 8, f64x4, f32x4>::type;
+  constexpr bool F64 = sizeof(R) == 8;
+  constexpr int N = S::NLON, NLAT = S::NLAT, NPAIR = S::NPAIR, RB = S::RB, NCSP = S::NCSP;
+  constexpr int MR = DIRX_MR, LG = DIRX_LG, KC = C::KC, KS = C::KS, NT = DIRX_NT;
   constexpr int NKS = KC / 4;  // MFMA K steps (4 pairs each) per staged step
   constexpr int NJ = 2 * MR;   // reals of one staged row segment
   static_assert(NPAIR % KC == 0, "pairs per step");
+  static_assert(MR == NT / 64, "one wavenumber per wave");
   // staged values per step: (input, level, pair, 4 reals) with the reals
-  // fastest, one 16-byte load per item
+  // fastest, 16-byte loads
   constexpr int NJ4 = NJ / 4;
   constexpr int NITEM = NIN * LG * KC * NJ4;
   constexpr int MAXIT = (NITEM + NT - 1) / NT;
-  __shared__ __align__(16) float X[NIN * 2 * KC * KS];  // [input][class][pair][level][m][re/im]
+  R* X = (R*)lds;  // [input][class][pair][level][m][re/im]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nlg = (a.nlev + LG - 1) / LG;
-  // neighbouring wavenumber ranges stage the two halves of the same 128-byte
-  // lines of a Fourier row: renumbered so that they run on one XCD's L2
-  const int b = xcd_block(blockIdx.x, gridDim.x);
-  const int mr = b % C::NMR;
-  const int lg = (b / C::NMR) % nlg;
-  const int mem = b / (C::NMR * nlg);
-  if (mem >= a.nmem) return;
   const int m0 = mr * MR, lev0 = lg * LG;
   const int nj = (S::NM - m0 < MR ? S::NM - m0 : MR) * 2;  // reals below the truncation
+  const int nl = a.nlev - lev0 < LG ? a.nlev - lev0 : LG;  // levels of this block
 
-  // each input's member as one buffer (2 m0 + NJ <= N: the 16-byte runs
-  // stay inside their rows; reals past the truncation are zeroed)
+  // each input's levels of this block as one buffer (2 m0 + NJ <= N: the
+  // 16-byte runs stay inside their rows; reals past the truncation are
+  // zeroed)
   __amdgpu_buffer_rsrc_t rsi[NIN];
 #pragma unroll
   for (int i = 0; i < NIN; ++i)
-    rsi[i] = buffer_rsrc((const float*)a.in[i] + mem * a.in_stride, a.nlev * NLAT * N * 4);
+    rsi[i] = buffer_rsrc(a.in[i] + mem * a.in_stride + (long)lev0 * NLAT * N,
+                         nl * NLAT * N * (int)sizeof(R));
   static_assert(2 * ((TS<T>::NM - 1) / MR * MR) + NJ <= N, "staged runs inside a row");
-  float rn[MAXIT][4], rs[MAXIT][4];
+  auto quad = [&](__amdgpu_buffer_rsrc_t rs, int off, R* v) {
+    uint4 u[sizeof(R) / 4];
+#pragma unroll
+    for (int h = 0; h < (int)sizeof(R) / 4; ++h) u[h] = buffer_load_x4(rs, off + 16 * h, 0);
+    __builtin_memcpy(v, u, 4 * sizeof(R));
+  };
+  R rn[MAXIT][4], rs[MAXIT][4];
   auto load = [&](int c) {
 #pragma unroll
     for (int it = 0; it < MAXIT; ++it) {
@@ -169,18 +128,18 @@ __global__ __launch_bounds__(512) void k_dirx_mf(DirxArgs a, DirxSlots sl) {
       const int j4 = e % NJ4, k = (e / NJ4) % KC, l = (e / (NJ4 * KC)) % LG,
                 i = e / (NJ4 * KC * LG);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) rn[it][q] = rs[it][q] = 0.f;
-      if (e < NITEM && lev0 + l < a.nlev && 4 * j4 < nj) {
+      for (int q = 0; q < 4; ++q) rn[it][q] = rs[it][q] = R(0);
+      if (e < NITEM && l < nl && 4 * j4 < nj) {
         const int pair = c * KC + k;
-        const int off = ((lev0 + l) * NLAT * N + 2 * m0 + 4 * j4) * 4;
-        const uint4 vn = buffer_load_x4(rsi[i], off + pair * N * 4, 0);
-        const uint4 vs = buffer_load_x4(rsi[i], off + (NLAT - 1 - pair) * N * 4, 0);
-        const unsigned un[4] = {vn.x, vn.y, vn.z, vn.w}, us[4] = {vs.x, vs.y, vs.z, vs.w};
+        const int off = (l * NLAT * N + 2 * m0 + 4 * j4) * (int)sizeof(R);
+        R vn[4], vs[4];
+        quad(rsi[i], off + pair * N * (int)sizeof(R), vn);
+        quad(rsi[i], off + (NLAT - 1 - pair) * N * (int)sizeof(R), vs);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           if (4 * j4 + q < nj) {
-            rn[it][q] = __uint_as_float(un[q]);
-            rs[it][q] = __uint_as_float(us[q]);
+            rn[it][q] = vn[q];
+            rs[it][q] = vs[q];
           }
       }
     }
@@ -193,13 +152,13 @@ __global__ __launch_bounds__(512) void k_dirx_mf(DirxArgs a, DirxSlots sl) {
       if (e < NITEM) {
         const int j4 = e % NJ4, k = (e / NJ4) % KC, l = (e / (NJ4 * KC)) % LG,
                   i = e / (NJ4 * KC * LG);
-        const int o = l * NJ + 4 * j4;  // even, and KS is even: 8-byte aligned
-        float2* xe = (float2*)&X[((i * 2 + 0) * KC + k) * KS + o];
-        float2* xo = (float2*)&X[((i * 2 + 1) * KC + k) * KS + o];
-        xe[0] = make_float2(rn[it][0] + rs[it][0], rn[it][1] + rs[it][1]);
-        xe[1] = make_float2(rn[it][2] + rs[it][2], rn[it][3] + rs[it][3]);
-        xo[0] = make_float2(rn[it][0] - rs[it][0], rn[it][1] - rs[it][1]);
-        xo[1] = make_float2(rn[it][2] - rs[it][2], rn[it][3] - rs[it][3]);
+        const int o = l * NJ + 4 * j4;  // even, and KS is even: pairs of reals are aligned
+        R2* xe = (R2*)&X[((i * 2 + 0) * KC + k) * KS + o];
+        R2* xo = (R2*)&X[((i * 2 + 1) * KC + k) * KS + o];
+        xe[0] = R2{rn[it][0] + rs[it][0], rn[it][1] + rs[it][1]};
+        xe[1] = R2{rn[it][2] + rs[it][2], rn[it][3] + rs[it][3]};
+        xo[0] = R2{rn[it][0] - rs[it][0], rn[it][1] - rs[it][1]};
+        xo[1] = R2{rn[it][2] - rs[it][2], rn[it][3] - rs[it][3]};
       }
     }
   };
@@ -207,27 +166,45 @@ __global__ __launch_bounds__(512) void k_dirx_mf(DirxArgs a, DirxSlots sl) {
   // A operand: row r = lane & 15, pair 4 ks + (lane >> 4) of the step; B
   // operand: column lane & 15 = (level l, component oc), the same pair
   const int r = lane & 15, kq = lane >> 4, l = (lane & 15) >> 1, oc = lane & 1;
-  f32x4 acc[MPW][2][RB];
+  const int m = m0 + wv;
+  const bool live = m <= T;  // the last range of wavenumbers may end early
+  const int w0 = w0_of(T, live ? m : T);
+  auto ntile = [](int mm, int p) {
+    const int d = T - mm - p;
+    return d < 0 ? 0 : (d / 2 + 16) / 16;
+  };
+  const int nt0 = live ? ntile(m, 0) : 0, nt1 = live ? ntile(m, 1) : 0;
+  Acc acc[NOUT][2][RB];
 #pragma unroll
-  for (int mi = 0; mi < MPW; ++mi)
+  for (int o = 0; o < NOUT; ++o)
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int rt = 0; rt < RB; ++rt) acc[mi][p][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // this lane's B source per slot: offset of (input, class 0, pair kq,
-  // level l, component ic) in X and the sign (0: no term for component oc)
-  int boff[NIN];
-  float bsg[NIN];
+      for (int rt = 0; rt < RB; ++rt) acc[o][p][rt] = Acc{0, 0, 0, 0};
+  // this lane's B source per output and slot: offset of (input, class 0,
+  // pair kq, level l, component ic) in X and the sign (0: no term for
+  // component oc); has: does the output have a term with the slot's table
+  int boff[NOUT][NIN];
+  R bsg[NOUT][NIN];
+  bool has[NOUT][NIN];
 #pragma unroll
-  for (int s = 0; s < NIN; ++s) {
-    boff[s] = ((oc ? sl.in[s][1] : sl.in[s][0]) * 2 * KC + kq) * KS + l * NJ +
-              (oc ? sl.ic[s][1] : sl.ic[s][0]);
-    bsg[s] = oc ? sl.sign[s][1] : sl.sign[s][0];
+  for (int o = 0; o < NOUT; ++o)
+#pragma unroll
+    for (int s = 0; s < NIN; ++s) {
+      boff[o][s] = ((oc ? a.src[o][s][1] : a.src[o][s][0]) * 2 * KC + kq) * KS + l * NJ +
+                   (oc ? a.ic[o][s][1] : a.ic[o][s][0]) + 2 * wv;
+      bsg[o][s] = (R)(oc ? a.sign[o][s][1] : a.sign[o][s][0]);
+      has[o][s] = a.sign[o][s][0] != 0 || a.sign[o][s][1] != 0;
+    }
+  // FP64 tables are read as they are, [pair][w]: the pair of reals at w0 +
+  // 2 (16 rt + r) holds the rows n of both parities, so one 16-byte load
+  // feeds both parities' MFMAs; rows past the truncation hold other
+  // coefficients, and their results are not stored
+  __amdgpu_buffer_rsrc_t rst[NIN];
+  if constexpr (F64) {
+#pragma unroll
+    for (int s = 0; s < NIN; ++s) rst[s] = buffer_rsrc(a.tab[s], NPAIR * NCSP * 8);
   }
-  auto ntile = [](int m, int p) {
-    const int d = T - m - p;
-    return d < 0 ? 0 : (d / 2 + 16) / 16;
-  };
 
   constexpr int NC = NPAIR / KC;
   load(0);
@@ -235,165 +212,216 @@ __global__ __launch_bounds__(512) void k_dirx_mf(DirxArgs a, DirxSlots sl) {
     __syncthreads();  // the previous step's MFMAs have read X
     store();
     __syncthreads();
-    // every A operand of this step first (all row tiles: the packed table is
-    // zero past the truncation), so that their latencies overlap; then the
-    // next step's inputs, whose loads stay in flight through the MFMAs
-    float av[MPW][NIN][2][RB][NKS];
-#pragma unroll
-    for (int mi = 0; mi < MPW; ++mi) {
-      const int ml = wv + C::NW * mi, m = m0 + ml;
-      if (ml >= MR || m > T) continue;
+    // every A operand of this step first, so that their latencies overlap;
+    // then the next step's inputs, whose loads stay in flight through the
+    // MFMAs
+    R av[NIN][2][RB][NKS];
+    if (live) {
 #pragma unroll
       for (int s = 0; s < NIN; ++s) {
-        const float* tp = sl.tab[s] + ((long)(m * 2) * RB * NPAIR + c * KC + kq) * 16 + r;
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
+        if constexpr (F64) {
 #pragma unroll
           for (int rt = 0; rt < RB; ++rt)
+            if (rt < nt0) {
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
-              av[mi][s][p][rt][ks] = tp[(((long)p * RB + rt) * NPAIR + 4 * ks) * 16];
+              for (int ks = 0; ks < NKS; ++ks) {
+                const uint4 v = buffer_load_x4(rst[s], (kq * NCSP + 2 * r) * 8,
+                                               ((c * KC + 4 * ks) * NCSP + w0 + 32 * rt) * 8);
+                R d[2];
+                __builtin_memcpy(d, &v, 16);
+                av[s][0][rt][ks] = d[0];
+                av[s][1][rt][ks] = d[1];
+              }
+            }
+        } else {
+          const R* tp = a.tab[s] + ((long)(m * 2) * RB * NPAIR + c * KC + kq) * 16 + r;
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int rt = 0; rt < RB; ++rt)
+#pragma unroll
+              for (int ks = 0; ks < NKS; ++ks)
+                av[s][p][rt][ks] = tp[(((long)p * RB + rt) * NPAIR + 4 * ks) * 16];
+        }
       }
     }
     if (c + 1 < NC) load(c + 1);
+    if (!live) continue;
 #pragma unroll
-    for (int mi = 0; mi < MPW; ++mi) {
-      const int ml = wv + C::NW * mi, m = m0 + ml;
-      if (ml >= MR || m > T) continue;
-      const int nt0 = ntile(m, 0), nt1 = ntile(m, 1);
+    for (int s = 0; s < NIN; ++s)
 #pragma unroll
-      for (int s = 0; s < NIN; ++s) {
+      for (int o = 0; o < NOUT; ++o) {
+        if (NOUT > 1 && !has[o][s]) continue;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-          float b[2];
+          R b[2];
 #pragma unroll
           for (int cls = 0; cls < 2; ++cls) {
-            const float x = X[boff[s] + (cls * KC + 4 * ks) * KS + 2 * ml];
-            b[cls] = bsg[s] == 0.f ? 0.f : bsg[s] * x;
+            const R x = X[boff[o][s] + (cls * KC + 4 * ks) * KS];
+            b[cls] = bsg[o][s] == R(0) ? R(0) : bsg[o][s] * x;
           }
 #pragma unroll
           for (int p = 0; p < 2; ++p) {
             // class of the folded input: symmetric (E) iff (n - m even) != Q-type table
-            const float bv = b[(p == 0) == (sl.isq[s] != 0) ? 1 : 0];
+            const R bv = b[(p == 0) == (a.isq[s] != 0) ? 1 : 0];
             const int nt = p ? nt1 : nt0;
 #pragma unroll
             for (int rt = 0; rt < RB; ++rt)
-              if (rt < nt)
-                acc[mi][p][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[mi][s][p][rt][ks], bv,
-                                                                      acc[mi][p][rt], 0, 0, 0);
+              if (rt < nt) {
+                if constexpr (F64)
+                  acc[o][p][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][p][rt][ks], bv,
+                                                                       acc[o][p][rt], 0, 0, 0);
+                else
+                  acc[o][p][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][p][rt][ks], bv,
+                                                                       acc[o][p][rt], 0, 0, 0);
+              }
           }
         }
       }
-    }
   }
-  // lane holds rows 4 kq + v of column (l, oc)
-  if (lev0 + l >= a.nlev) return;
-  float* out = (float*)a.out + mem * a.out_stride + (long)(lev0 + l) * S::NRSP;
+  // item v of a lane is row 4 kq + v of column (l, oc); in the FP64 form row
+  // 4 v + kq
+  if (l >= nl || !live) return;
 #pragma unroll
-  for (int mi = 0; mi < MPW; ++mi) {
-    const int ml = wv + C::NW * mi, m = m0 + ml;
-    if (ml >= MR || m > T) continue;
-    const int w0 = w0_of(T, m);
+  for (int o = 0; o < NOUT; ++o) {
+    R* out = a.out[o] + mem * a.out_stride + (long)(lev0 + l) * S::NRSP;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int rt = 0; rt < RB; ++rt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int dn = p + 2 * (16 * rt + 4 * kq + v);
-          if (m + dn <= T) out[2 * (w0 + dn) + oc] = acc[mi][p][rt][v];
+          const int dn = p + 2 * (16 * rt + (F64 ? 4 * v + kq : 4 * kq + v));
+          if (m + dn <= T) out[2 * (w0 + dn) + oc] = acc[o][p][rt][v];
         }
   }
 }
 
-// sum of the latitude-pair blocks' partial sums in a fixed order; n reals
-// per block, per_mem of them per member (member stride out_stride in out)
-template <typename R>
-__global__ void k_sum_blocks(const R* scratch, R* out, int npb, long n, long per_mem,
-                             long out_stride) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  R s = 0;
-  for (int b = 0; b < npb; ++b) s += scratch[(long)b * n + i];
-  const long mem = i / per_mem;
-  out[mem * out_stride + (i - mem * per_mem)] = s;
+// Minimum waves per SIMD asked of the compiler: two blocks per CU instead of
+// one where the FP64 registers come down to 128 with at most 18 of them
+// spilled (T42 L20, 32 members: mktend 95 against 100 us, uv2dv 38 against 46;
+// T63 mktend spills as much for 103 against 100 us, and T127 more: those keep
+// their registers)
+template <int T, typename R, int NOUT, int NIN>
+constexpr int dirx_waves() {
+  return sizeof(R) == 8 && (T == 42 || (T == 63 && NIN == 2)) ? 4 : 2;
 }
 
-template <int T>
-static int dirx_mf_t(const Tables& tb, const DirxArgs& a, hipStream_t s) {
-  if (a.nlev <= 0 || a.nmem <= 0) return 0;
-  DirxSlots sl{};
-  for (int t = 0; t < a.nterm; ++t) {
-    const DirxTerm& tm = a.terms[t];
-    int k = 0;
-    while (k < sl.nslot && sl.tab[k] != tb.dir_f32[tm.table]) ++k;
-    if (k == sl.nslot) {
-      if (k == NSLOT || !tb.dir_f32[tm.table]) return -2;
-      sl.tab[k] = tb.dir_f32[tm.table];
-      sl.isq[k] = table_is_q(tm.table) ? 1 : 0;
-      ++sl.nslot;
+// One job alone: fc2sp of Fourier fields, uv2dv, qtend.  (qtend in the kernel
+// below, which holds the two-output body's registers: T127 L40, 4 members,
+// 112 us against 89.)
+template <int T, typename R, int NIN, int NOUT>
+__global__ __launch_bounds__(DIRX_NT, (dirx_waves<T, R, NOUT, NIN>())) void k_dirx_one(
+    DirxJob<R> a, int per) {
+  __shared__ __align__(16) char lds[DirxCfg<T, R, NIN>::LDS];
+  constexpr int NMR = DirxCfg<T, R, NIN>::NMR;
+  // neighbouring wavenumber ranges stage the two halves of the same 128-byte
+  // lines of a Fourier row: renumbered so that they run on one XCD's L2
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int mem = b / per, i = b - mem * per;
+  dirx_body<T, R, NIN, NOUT>(a, mem, i / NMR, i % NMR, lds);
+}
+
+// mktend, gridpointa: jobs of three inputs and one or two outputs, and of one
+// input, in one launch (blocks as above, a member's jobs side by side)
+template <int T, typename R>
+__global__ __launch_bounds__(DIRX_NT, (dirx_waves<T, R, 2, 3>())) void k_dirx_mf(DirxJobs<R> j) {
+  __shared__ __align__(16) char lds[DirxCfg<T, R, 3>::LDS > DirxCfg<T, R, 1>::LDS
+                                        ? DirxCfg<T, R, 3>::LDS
+                                        : DirxCfg<T, R, 1>::LDS];
+  constexpr int NMR = DirxCfg<T, R, 1>::NMR;
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int mem = b / j.per;
+  const int q = b - mem * j.per;
+  int k = 0;
+#pragma unroll
+  for (int i = 1; i < DIRX_JOBS; ++i)
+    if (i < j.njob && q >= j.start[i]) k = i;
+  k = __builtin_amdgcn_readfirstlane(k);
+  const DirxJob<R>& a = j.job[k];
+  const int i = q - j.start[k];
+  const int mr = i % NMR, lg = i / NMR;
+  if (a.nin == 1)
+    dirx_body<T, R, 1, 1>(a, mem, lg, mr, lds);
+  else if (a.nout == 1)
+    dirx_body<T, R, 3, 1>(a, mem, lg, mr, lds);
+  else
+    dirx_body<T, R, 3, 2>(a, mem, lg, mr, lds);
+}
+
+template <int T, typename R>
+static int dirx_t(const Tables& tb, const DirxArgs* args, int njob, hipStream_t s) {
+  if (njob < 1 || njob > DIRX_JOBS) return -2;
+  DirxJobs<R> jobs{};
+  jobs.nmem = args[0].nmem;
+  bool wide = false;  // a job with three inputs
+  for (int k = 0; k < njob; ++k) {
+    const DirxArgs& a = args[k];
+    DirxJob<R>& g = jobs.job[jobs.njob];
+    if (a.nmem != jobs.nmem || a.nin < 1 || a.nin > 3 || a.nout < 1 || a.nout > 2) return -2;
+    if (a.nlev <= 0) continue;
+    const R* tabs[3] = {};
+    int nslot = 0;
+    for (int t = 0; t < a.nterm; ++t) {
+      const DirxTerm& tm = a.terms[t];
+      const R* tab;
+      if constexpr (sizeof(R) == 8)
+        tab = tb.filt64 + (long)tm.table * tb.npair * tb.ncsp;
+      else
+        tab = tb.dir_f32[tm.table];
+      int i = 0;
+      while (i < nslot && tabs[i] != tab) ++i;
+      if (i == nslot) {
+        if (i == 3 || !tab) return -2;
+        tabs[nslot++] = tab;
+        g.tab[i] = tab;
+        g.isq[i] = table_is_q(tm.table) ? 1 : 0;
+      }
+      if (g.sign[tm.o][i][tm.oc] != 0) return -2;  // one term per (output, table, component)
+      g.sign[tm.o][i][tm.oc] = tm.sign;
+      g.src[tm.o][i][tm.oc] = tm.in;
+      g.ic[tm.o][i][tm.oc] = tm.ic;
     }
-    if (sl.sign[k][tm.oc] != 0.f) return -2;  // one term per (table, component)
-    sl.sign[k][tm.oc] = tm.sign > 0 ? 1.f : -1.f;
-    sl.in[k][tm.oc] = tm.in;
-    sl.ic[k][tm.oc] = tm.ic;
+    if (nslot != a.nin) return -2;  // one table per input
+    if (a.nin < 3 && a.nin != a.nout) return -2;
+    wide = wide || a.nin == 3;
+    for (int i = 0; i < a.nin; ++i) g.in[i] = (const R*)a.in[i];
+    for (int o = 0; o < a.nout; ++o) g.out[o] = (R*)a.out[o];
+    g.nin = a.nin;
+    g.nout = a.nout;
+    g.nlev = a.nlev;
+    g.nlg = (a.nlev + DIRX_LG - 1) / DIRX_LG;
+    g.in_stride = a.in_stride;
+    g.out_stride = a.out_stride;
+    jobs.per += DirxCfg<T, R, 1>::NMR * g.nlg;
+    jobs.start[++jobs.njob] = jobs.per;
   }
-  if (sl.nslot != a.nin) return -2;  // one table per input
-  // a member's input levels are addressed as one buffer of 32-bit byte offsets
-  if ((long)a.nlev * TS<T>::NLAT * TS<T>::NLON * 4 > 0x7fffffffL) return -2;
-  const long nlg = (a.nlev + 7) / 8;
-  auto launch = [&](auto kern, int nmr) {
-    kern<<<(unsigned)((long)a.nmem * nlg * nmr), 512, 0, s>>>(a, sl);
-  };
-  switch (a.nin) {
-    case 1: launch(k_dirx_mf<T, 1>, DirxMfCfg<T, 1>::NMR); break;
-    case 2: launch(k_dirx_mf<T, 2>, DirxMfCfg<T, 2>::NMR); break;
-    case 3: launch(k_dirx_mf<T, 3>, DirxMfCfg<T, 3>::NMR); break;
-    default: return -2;
+  const long nblk = (long)jobs.nmem * jobs.per;
+  if (nblk <= 0) return 0;
+  const int nin = jobs.job[0].nin, nout = jobs.job[0].nout;
+  const dim3 grid((unsigned)nblk);
+  if (jobs.njob > 1 || (nin == 3 && nout == 2)) {
+    for (int k = 0; k < jobs.njob; ++k)
+      if (!wide || jobs.job[k].nin == 2) return -2;
+    k_dirx_mf<T, R><<<grid, DIRX_NT, 0, s>>>(jobs);
+  } else if (nin == 3) {
+    k_dirx_one<T, R, 3, 1><<<grid, DIRX_NT, 0, s>>>(jobs.job[0], jobs.per);
+  } else if (nin == 2) {
+    k_dirx_one<T, R, 2, 2><<<grid, DIRX_NT, 0, s>>>(jobs.job[0], jobs.per);
+  } else {
+    k_dirx_one<T, R, 1, 1><<<grid, DIRX_NT, 0, s>>>(jobs.job[0], jobs.per);
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <int T, int MODE>
-static int dirx_t(const Tables& tb, const DirxArgs& a, void* scratch, size_t sbytes,
-                  hipStream_t s) {
-  using C = DirxCfg<T, MODE>;
-  using R = RealX<MODE>;
-  if (a.nlev <= 0 || a.nmem <= 0) return 0;
-  const long per_mem = (long)a.nlev * TS<T>::NRSP;
-  const long n = (long)a.nmem * per_mem;
-  if (C::NPB > 1 && (!scratch || sbytes < sizeof(R) * n * C::NPB)) return -4;
-  const void* tv = (MODE == MODE_F64) ? (const void*)tb.filt64 : (const void*)tb.filt32;
-  k_dirx<T, MODE><<<(unsigned)((long)a.nmem * a.nlev * C::NPB), 256, 0, s>>>(a, tv, scratch);
-  if (C::NPB > 1)
-    k_sum_blocks<R><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
-        (const R*)scratch, (R*)a.out, C::NPB, n, per_mem, a.out_stride);
-  return hipGetLastError() == hipSuccess ? 0 : -3;
-}
-
-size_t dirx_scratch_bytes(const Tables& tb, int mode, int nlev) {
-  if (mode != MODE_F64) return 0;  // the MFMA form sums all pairs in one block
-  const long n = (long)nlev * 2 * tb.ncsp;
-  int npb = 1;
-  switch (tb.ntru) {
-    case 21: npb = DirxCfg<21, MODE_F64>::NPB; break;
-    case 42: npb = DirxCfg<42, MODE_F64>::NPB; break;
-    case 63: npb = DirxCfg<63, MODE_F64>::NPB; break;
-    case 127: npb = DirxCfg<127, MODE_F64>::NPB; break;
-  }
-  return npb > 1 ? sizeof(double) * n * npb : 0;
-}
-
-int launch_dirx(const Tables& tb, int mode, const DirxArgs& a, void* scratch, size_t sbytes,
-                hipStream_t s) {
-  // FP64: VALU sums per level; FP32 modes: MFMA over 8 levels per block
+int launch_dirx(const Tables& tb, int mode, const DirxArgs* args, int njob, hipStream_t s) {
   const bool d = (mode == MODE_F64);
   switch (tb.ntru) {
-    case 21: return d ? dirx_t<21, MODE_F64>(tb, a, scratch, sbytes, s) : dirx_mf_t<21>(tb, a, s);
-    case 42: return d ? dirx_t<42, MODE_F64>(tb, a, scratch, sbytes, s) : dirx_mf_t<42>(tb, a, s);
-    case 63: return d ? dirx_t<63, MODE_F64>(tb, a, scratch, sbytes, s) : dirx_mf_t<63>(tb, a, s);
+    case 21: return d ? dirx_t<21, double>(tb, args, njob, s) : dirx_t<21, float>(tb, args, njob, s);
+    case 42: return d ? dirx_t<42, double>(tb, args, njob, s) : dirx_t<42, float>(tb, args, njob, s);
+    case 63: return d ? dirx_t<63, double>(tb, args, njob, s) : dirx_t<63, float>(tb, args, njob, s);
     case 127:
-      return d ? dirx_t<127, MODE_F64>(tb, a, scratch, sbytes, s) : dirx_mf_t<127>(tb, a, s);
+      return d ? dirx_t<127, double>(tb, args, njob, s) : dirx_t<127, float>(tb, args, njob, s);
     default: return -2;
   }
 }

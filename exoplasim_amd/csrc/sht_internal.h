@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
+
 #include "sht_common.h"
 
 struct exo_sht_plan_s;
@@ -86,42 +88,76 @@ struct FwdArgs {
   int var;          // tile variant (0 default, 1 half the fields per block)
 };
 
-// One term of a multi-input direct transform: out[oc] += sign * t * X_in[ic]
+// One term of a multi-input direct transform: out_o[oc] += sign * t * X_in[ic]
 struct DirxTerm {
   int8_t in, ic, oc, sign;
   int8_t table;
+  int8_t o = 0;
 };
-// The term lists of the multi-input direct transforms (folded branches of
-// src/legmod.f90): {input, input component, output component, sign, table}
-// mktend (:538-549, fu <- gvz, fv <- guz as gridpointa calls it):
-//   D = qq.ke - qe.fv + i qm.fu     inputs (ke, fv, fu)
-//   T = qe.vt + qc.tn - i qm.ut     inputs (vt, tn, ut)
-//   Z = qe.fu + i qm.fv             inputs (fu, fv)
-// qtend (:468-496): q = qe.vq + qc.qn - i qm.uq   inputs (qn, uq, vq)
-inline constexpr DirxTerm MKTEND_D[6] = {{0, 0, 0, +1, TQQ}, {1, 0, 0, -1, TQE},
-                                         {2, 1, 0, -1, TQM}, {0, 1, 1, +1, TQQ},
-                                         {1, 1, 1, -1, TQE}, {2, 0, 1, +1, TQM}};
-inline constexpr DirxTerm MKTEND_T[6] = {{0, 0, 0, +1, TQE}, {1, 0, 0, +1, TQC},
-                                         {2, 1, 0, +1, TQM}, {0, 1, 1, +1, TQE},
-                                         {1, 1, 1, +1, TQC}, {2, 0, 1, -1, TQM}};
-inline constexpr DirxTerm MKTEND_Z[4] = {{0, 0, 0, +1, TQE}, {1, 1, 0, -1, TQM},
-                                         {0, 1, 1, +1, TQE}, {1, 0, 1, +1, TQM}};
-inline constexpr DirxTerm QTEND_Q[6] = {{2, 0, 0, +1, TQE}, {0, 0, 0, +1, TQC},
-                                        {1, 1, 0, +1, TQM}, {2, 1, 1, +1, TQE},
-                                        {0, 1, 1, +1, TQC}, {1, 0, 1, -1, TQM}};
-
+// One job of the multi-input direct transforms: nout spectral outputs (2*NCSP,
+// nlev) of nin Fourier inputs fc(2, NLON/2, NLAT, nlev), per member
 struct DirxArgs {
-  const void* in[3];  // Fourier inputs fc(2, NLON/2, NLAT, nlev) per member
-  void* out;          // spectral output (2*NCSP, nlev) per member
-  int nin, nlev, nterm;
-  DirxTerm terms[8];
+  const void* in[3];
+  void* out[2];
+  int nin, nout, nlev, nterm;
+  DirxTerm terms[10];
   int nmem;                   // members (>= 1)
   long in_stride, out_stride; // member strides of the inputs / the output, in reals
 };
+inline DirxArgs dirx_job(std::initializer_list<const void*> in, std::initializer_list<void*> out,
+                         std::initializer_list<DirxTerm> terms, int nlev, int nmem,
+                         long in_stride, long out_stride) {
+  DirxArgs a{};
+  for (const void* x : in) a.in[a.nin++] = x;
+  for (void* x : out) a.out[a.nout++] = x;
+  for (const DirxTerm& t : terms) a.terms[a.nterm++] = t;
+  a.nlev = nlev;
+  a.nmem = nmem;
+  a.in_stride = in_stride;
+  a.out_stride = out_stride;
+  return a;
+}
+// The jobs of the folded branches of src/legmod.f90; a term is {input, input
+// component, output component, sign, table[, output]}.
+// mktend (:538-549): D = qq.ke - qe.fv + i qm.fu and Z = qe.fu + i qm.fv,
+// which share their inputs
+inline DirxArgs mktend_dz(const void* ke, const void* fv, const void* fu, void* d, void* z,
+                          int nlev, int nmem, long fs, long ss) {
+  return dirx_job({ke, fv, fu}, {d, z},
+                  {{0, 0, 0, +1, TQQ}, {1, 0, 0, -1, TQE}, {2, 1, 0, -1, TQM},
+                   {0, 1, 1, +1, TQQ}, {1, 1, 1, -1, TQE}, {2, 0, 1, +1, TQM},
+                   {2, 0, 0, +1, TQE, 1}, {1, 1, 0, -1, TQM, 1},
+                   {2, 1, 1, +1, TQE, 1}, {1, 0, 1, +1, TQM, 1}},
+                  nlev, nmem, fs, ss);
+}
+// and T = qe.vt + qc.tn - i qm.ut; qtend (:468-496) is the same sum with (q;
+// vq, qn, uq) for (T; vt, tn, ut)
+inline DirxArgs mktend_t(const void* vt, const void* tn, const void* ut, void* t, int nlev,
+                         int nmem, long fs, long ss) {
+  return dirx_job({vt, tn, ut}, {t},
+                  {{0, 0, 0, +1, TQE}, {1, 0, 0, +1, TQC}, {2, 1, 0, +1, TQM},
+                   {0, 1, 1, +1, TQE}, {1, 1, 1, +1, TQC}, {2, 0, 1, -1, TQM}},
+                  nlev, nmem, fs, ss);
+}
+// uv2dv (:391-422): D = -qe.v + i qm.u, Z = qe.u + i qm.v
+inline DirxArgs uv2dv_dz(const void* u, const void* v, void* d, void* z, int nlev, int nmem,
+                         long fs, long ss) {
+  return dirx_job({u, v}, {d, z},
+                  {{1, 0, 0, -1, TQE}, {0, 1, 0, -1, TQM}, {1, 1, 1, -1, TQE}, {0, 0, 1, +1, TQM},
+                   {0, 0, 0, +1, TQE, 1}, {1, 1, 0, -1, TQM, 1},
+                   {0, 1, 1, +1, TQE, 1}, {1, 0, 1, +1, TQM, 1}},
+                  nlev, nmem, fs, ss);
+}
+// fc2sp (:178-223) of nlev fields with table t
+inline DirxArgs fc2sp_job(const void* fc, void* sp, int t, int nlev, int nmem, long fs, long ss) {
+  return dirx_job({fc}, {sp}, {{0, 0, 0, +1, (int8_t)t}, {0, 1, 1, +1, (int8_t)t}}, nlev, nmem,
+                  fs, ss);
+}
 
-int launch_dirx(const Tables& T, int mode, const DirxArgs& a, void* scratch, size_t sbytes,
-                hipStream_t s);
-size_t dirx_scratch_bytes(const Tables& T, int mode, int nlev);  // nlev: member-levels
+// all jobs (over the same members) in one launch: uv2dv_dz or an fc2sp_job
+// alone, or up to four of mktend_dz, mktend_t and fc2sp_job with at least
+// one of the former
+int launch_dirx(const Tables& T, int mode, const DirxArgs* jobs, int njob, hipStream_t s);
 
 int launch_inverse(const Tables& T, int mode, bool fused, const InvArgs& a, hipStream_t s);
 // the sp2fc run (aq), nj <= INV_ONE_MAX one-field scalar jobs (aj: sp2fc,

@@ -147,18 +147,9 @@ int launch_forward(const Tables& tb, int mode, bool fused, const FwdArgs& a, voi
       fin = scratch;
       fstride = ms;
     }
-    DirxArgs d{};
-    d.in[0] = fin;
-    d.out = (float*)a.sp + (long)a.dst0 * 2 * tb.ncsp;
-    d.nin = 1;
-    d.nlev = a.nfield;
-    d.nmem = a.nmem;
-    d.in_stride = fstride;
-    d.out_stride = a.sp_stride;
-    d.nterm = 2;
-    d.terms[0] = DirxTerm{0, 0, 0, +1, (int8_t)a.table};
-    d.terms[1] = DirxTerm{0, 1, 1, +1, (int8_t)a.table};
-    return launch_dirx(tb, MODE_F32, d, nullptr, 0, s);
+    const DirxArgs d = fc2sp_job(fin, (float*)a.sp + (long)a.dst0 * 2 * tb.ncsp, a.table, a.nfield,
+                                 a.nmem, fstride, a.sp_stride);
+    return launch_dirx(tb, mode, &d, 1, s);
   }
   switch (mode) {
     case MODE_F64: return fwd_mode<MODE_F64>(tb, fused, a, scratch, sbytes, s);
