@@ -6,14 +6,26 @@
 //             gqn, guz, gvz, the geopotential term gphi and dw; with it the
 //             products of gridpointa (src/plasim.f90:2436-2446) and, on
 //             request, gp = exp(gp) (:2434)
+//             request, gp = exp(gp) (:2434); in gridpointa also gp2fc of the
+//             fields that go to the direct transforms
 //   k_gpmt    the Fourier-space d/dlambda of ln(ps) (src/plasim.f90:2425-2430)
 //
-// One thread per grid point and member runs down the column.  calcgp is a
-// pointwise column computation: every level of every field is read once and
-// written once, coalesced along the grid points, so the kernel is bound by
-// HBM; the two triangular sums over levels (ztpta/ztptb against c, gphi
-// against g) run from registers, with c and g read through scalar loads
-// (every lane of a wave reads the same element).
+// calcgp is a column computation of pointwise terms, prefix sums over the
+// levels and two matrix products over the levels (c and g).  A block takes 64
+// grid points, or one latitude row in gridpointa, and all levels; its 8 waves
+// share the levels, a lane owning the same points at each.  What a level needs
+// of the others -- v . grad ln ps, the divergence and the humidity term --
+// meets in LDS, and c and g are read through scalar loads (a wave's lanes all
+// work on one level).  The kernel is bound by HBM and L2: 6 fields are read
+// and 11 written per level.
+//
+// (One thread per column with its level arrays in registers held 202 VGPRs at
+// L20 in FP32 and spilled at L40 in FP64; level counts without an
+// instantiation of their own kept the arrays in scratch.  gridpointa of T42
+// L20, 32 members, FP32: 336 us with it and the row FFT as a launch, 318 with
+// this kernel on the grid, 273 with the rows transformed in it; T21 L10, one
+// member, FP64: 49, 39.5, 37.5 us; T63 L20, 3 members, FP64: 294 and 253 us on
+// the grid.)
 #include "../../include/exo_dyn.h"
 #include "sht_plan.h"
 
@@ -34,166 +46,290 @@ struct CalcgpPtrs {
   R *gut, *gvt, *gke, *guq, *gvq;
 };
 
-// NL > 0: exactly NL levels, every per-level array in registers; NL = 0:
-// a.nlev <= 64 levels at run time, the arrays in per-lane memory.
+// ROW = 0: calcgp on the grid, 64 points per block.  ROW = N (64, 128):
+// gridpointa on rows of N longitudes, one row per block; the nine tendency fields of a
+// level and gvp then leave as the Fourier coefficients of their rows (gp2fc):
+// the wave that computed a level transforms it in LDS rows of its own, two
+// real rows per complex FFT and GpCfg::NFB FFTs at a time, so the grid values
+// of those fields never reach HBM.
+template <typename R, int ROW>
+struct GpCfg {
+  static constexpr int PPL = ROW ? ROW / 64 : 1;  // points per lane
+  static constexpr int P = 64 * PPL;              // points per block
+  static constexpr int W = 8;                     // waves per block
+  // FFTs at a time: all five of a level, but two in FP64 on rows of 128, whose
+  // five would leave the level arrays too little LDS
+  static constexpr int NFB = sizeof(R) == 4 || ROW <= 64 ? 5 : 2;
+  static constexpr int NP = ROW + ROW / 32;  // padded FFT row
+  static constexpr int WPS = (sizeof(R) == 4 || ROW <= 64) ? 4 : 2;  // waves per SIMD asked for
+  static size_t lds(int nlev) {
+    return sizeof(R) * 3 * nlev * P + (ROW ? sizeof(C2<R>) * (W * NFB * NP + ROW) : 0);
+  }
+};
+
+// A wave-uniform vector of the vertical set-up, read through scalar loads
+template <typename R>
+using Uni = __attribute__((address_space(4))) const R*;
+
 // With sid (gridpointa) rcsq = 1 / cos^2 comes from the Gaussian abscissas, as
 // the model sets it up (src/plasim.f90:1897 csq = 1 - sid^2 in the real kind,
 // :205), and is written to rcsq_out; else it is read.
-template <typename R, int NL>
-__global__ __launch_bounds__(256) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, int nlev_rt,
-                                                int nhor, long mstride, int nqspec, int exp_gp,
-                                                const double* sid, int nlon, R* rcsq_out) {
-  constexpr int NA = NL > 0 ? NL : 64;
-  const int n = NL > 0 ? NL : nlev_rt;
-  const int h = blockIdx.x * 256 + threadIdx.x;
-  if (h >= nhor) return;
-  const long mo = (long)blockIdx.y * mstride;
-  auto at = [&](const R* p, int j) -> R { return p[mo + (long)j * nhor + h]; };
-  auto put = [&](R* p, int j, R x) { p[mo + (long)j * nhor + h] = x; };
-  const R gpm = f.gpm[mo + h], gpj = f.gpj[mo + h];
-  R rcsq;
-  if (sid) {
-    const double x = sid[h / nlon];
-    rcsq = R(1) / (R)(1.0 - x * x);
-    rcsq_out[mo + h] = rcsq;
-  } else {
-    rcsq = f.rcsq[mo + h];
+template <typename R, int ROW>
+__global__ __launch_bounds__(512, (GpCfg<R, ROW>::WPS)) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, int n, int nhor,
+                                                long mstride, int nqspec, int exp_gp,
+                                                const double* sid, int nlon, R* rcsq_out,
+                                                const C2<R>* tw) {
+  using C = GpCfg<R, ROW>;
+  using R2 = R __attribute__((ext_vector_type(2)));
+  constexpr int PPL = C::PPL, P = C::P, W = C::W;
+  extern __shared__ __align__(16) char smem[];
+  R2* zg = (R2*)smem;          // [level][point]: (zvgpg, gd)
+  R* cr = (R*)(zg + n * P);    // [level][point]: humidity term of the virtual temperature
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Every field is addressed by a wave-uniform base (member, level, block) and
+  // the lane's point within the block, so that the address arithmetic is
+  // scalar.  The lanes past the last point repeat it and store nothing.
+  const int h0 = blockIdx.x * P;
+  const long mo = (long)blockIdx.y * mstride + h0;
+  unsigned pt = lane;
+  bool live = true;
+  if constexpr (ROW == 0) {
+    live = h0 + lane < nhor;
+    if (!live) pt = nhor - 1 - h0;
   }
-  R gp = f.gp[mo + h];
-  if (exp_gp) {
-    gp = exp(gp);
-    f.gp[mo + h] = gp;
-  }
-  const R* __restrict__ dsig = v.dsigma;
-  const R* __restrict__ sigh = v.sigmah;
-  const R* __restrict__ c = v.c;
-  const R* __restrict__ g = v.g;
-
-  // zvgpg = rcsq (u d/dlambda + v d/dmu) ln ps; the running sums of the
-  // sigma-dot integral in the reference's order
-  R zvgpg[NA], gdl[NA], ztv1d[NA], ke[NA];
-  R zsumd = R(0), vp = R(0);
-#pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    if (j >= n) break;
-    const R gu = at(f.gu, j), gv = at(f.gv, j), gd = at(f.gd, j);
-    zvgpg[j] = rcsq * (gu * gpm + gv * gpj);
-    gdl[j] = gd;
-    zsumd = zsumd + dsig[j] * gd;
-    vp = vp + dsig[j] * zvgpg[j];
-  }
-  f.gvp[mo + h] = vp;
-  const R tot = zsumd + vp;  // zsumd + gvp at the bottom
+  auto at = [&](const R* p, int j, int i) -> R {
+    const R* b = p + (mo + (long)j * nhor + 64 * i);
+    return b[pt];
+  };
+  auto put = [&](R* p, int j, int i, R x) {
+    R* b = p + (mo + (long)j * nhor + 64 * i);
+    if (live) b[pt] = x;
+  };
+  const Uni<R> dsig = (Uni<R>)v.dsigma, sigh = (Uni<R>)v.sigmah, rdsig = (Uni<R>)v.rdsig;
+  const Uni<R> t0v = (Uni<R>)v.t0, t01 = (Uni<R>)v.t01s2, tkp = (Uni<R>)v.tkp;
   const R qfac = R(1) / v.rdbrv - R(1);
 
-  // level j: virtual temperatures, then the terms of level j that need
-  // level j + 1 (gtd, gqm, gud, gvd), carried one level on
-  R rz = R(0), rv = R(0);  // running sums again, for zsdotp(j)
-  R gtd_m = R(0), gqm_m = R(0), gud_m = R(0), gvd_m = R(0);
-  R zs2 = R(0);            // the second zsumd of the reference (:2656, :2681)
-  R gt = at(f.gt, 0), gq = at(f.gq, 0), gu = at(f.gu, 0), gv = at(f.gv, 0);
+  // ---- surface fields ----
+  R gpm[PPL], gpj[PPL], rcsq[PPL], gp[PPL];
 #pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    if (j >= n) break;
-    const R gz = at(f.gz, j);
-    R zq = (nqspec == 1) ? gq / gp : at(f.dq, j);
-    if (!(zq > R(0))) zq = R(0);
-    // The reference forms (gt + t0)(1 + (1/rdbrv - 1) zq) - t0 and then
-    // subtracts gt again for gphi (src/plasim.f90:2617-2622, 2742): t0 is
-    // large against the humidity term, and the subtractions cancel it.  The
-    // same quantities in the form without the cancellation: the virtual
-    // temperature term corr = (gt + t0)(1/rdbrv - 1) zq, ztv1 = gt + corr,
-    // ztv1 - gt = corr and ztv2 = (gt + corr - t0 adv zq) / (1 + adv zq).
-    const R t0 = v.t0[j];
-    const R corr = (gt + t0) * (qfac * zq);
-    const R ztv1 = gt + corr;
-    const R ztv2 = (gt + corr - t0 * (v.adv * zq)) / (R(1) + v.adv * zq);
-    ztv1d[j] = corr;
-    // sigma-dot and the vertical advection terms at the interface below j
-    R gtd = R(0), gqm = R(0), gud = R(0), gvd = R(0);
-    R gt1 = R(0), gq1 = R(0), gu1 = R(0), gv1 = R(0);
-    if (j < n - 1) {
-      rz = rz + dsig[j] * gdl[j];
-      rv = rv + dsig[j] * zvgpg[j];
-      const R zsdotp = sigh[j] * tot - (rz + rv);
-      gt1 = at(f.gt, j + 1);
-      gq1 = at(f.gq, j + 1);
-      gu1 = at(f.gu, j + 1);
-      gv1 = at(f.gv, j + 1);
-      gtd = zsdotp * (gt1 - gt);
-      gqm = zsdotp * (gq1 + gq);
-      gud = zsdotp * (gu1 - gu);
-      gvd = zsdotp * (gv1 - gv);
-    }
-    const R rd = v.rdsig[j];
-    R gtn, gqn, guz, gvz, dw;
-    if (j == 0) {
-      zs2 = zvgpg[0] * dsig[0];
-      gtn = gt * gdl[0] - v.akap * ztv2 * gdl[0] -
-            rd * (gtd + v.t01s2[0] * (sigh[0] * vp - zs2));
-      gqn = -rd * gqm;
-      guz = -gu * gz - gpj * ztv1 - rd * gvd;
-      gvz = gv * gz - gpm * ztv1 - rd * gud;
-      dw = gdl[0] * gp * v.psurf * v.ww;
+  for (int i = 0; i < PPL; ++i) {
+    gpm[i] = at(f.gpm, 0, i);
+    gpj[i] = at(f.gpj, 0, i);
+    gp[i] = at(f.gp, 0, i);
+    if (sid) {
+      const double x = sid[(h0 + (int)pt + 64 * i) / nlon];
+      rcsq[i] = R(1) / (R)(1.0 - x * x);
     } else {
-      // c(k, j) for k <= j: column j of c, through scalar loads
-      R ztpta = c[j * n] * zvgpg[0];
-      R ztptb = c[j * n] * (zvgpg[0] + gdl[0]);
-#pragma unroll
-      for (int k = 1; k < NA; ++k) {
-        if (k > j) break;
-        ztpta = ztpta + c[j * n + k] * zvgpg[k];
-        ztptb = ztptb + c[j * n + k] * (zvgpg[k] + gdl[k]);
-      }
-      if (j < n - 1) {
-        zs2 = zs2 + zvgpg[j] * dsig[j];
-        gtn = gt * gdl[j] + v.akap * ztv2 * (zvgpg[j] - ztptb) + v.tkp[j] * (zvgpg[j] - ztpta) -
-              rd * (gtd + gtd_m + vp * (v.t01s2[j] * sigh[j] + v.t01s2[j - 1] * sigh[j - 1]) -
-                    zs2 * (v.t01s2[j - 1] + v.t01s2[j]) + zvgpg[j] * dsig[j] * v.t01s2[j - 1]);
-        gqn = -rd * (gqm - gqm_m);
-        guz = -gu * gz - gpj * ztv1 - rd * (gvd + gvd_m);
-        gvz = gv * gz - gpm * ztv1 - rd * (gud + gud_m);
-      } else {
-        gtn = gt * gdl[j] + v.akap * ztv2 * (zvgpg[j] - ztptb) + v.tkp[j] * (zvgpg[j] - ztpta) -
-              rd * (gtd_m + v.t01s2[j - 1] * (sigh[j - 1] * vp - zs2));
-        gqn = rd * gqm_m;
-        guz = -gu * gz - gpj * ztv1 - rd * gvd_m;
-        gvz = gv * gz - gpm * ztv1 - rd * gud_m;
-      }
-      dw = (zvgpg[j] - ztptb) * gp * v.psurf * v.ww;
+      rcsq[i] = at(f.rcsq, 0, i);
     }
-    put(f.gtn, j, gtn);
-    put(f.gqn, j, gqn);
-    put(f.guz, j, guz);
-    put(f.gvz, j, gvz);
-    put(f.dw, j, dw);
-    if (f.gut) put(f.gut, j, gu * gt);
-    if (f.gvt) put(f.gvt, j, gv * gt);
-    if (nqspec == 1 && f.guq) put(f.guq, j, gu * gq);
-    if (nqspec == 1 && f.gvq) put(f.gvq, j, gv * gq);
-    ke[j] = gu * gu + gv * gv;
-    gtd_m = gtd;
-    gqm_m = gqm;
-    gud_m = gud;
-    gvd_m = gvd;
-    gt = gt1;
-    gq = gq1;
-    gu = gu1;
-    gv = gv1;
+    if (exp_gp) gp[i] = exp(gp[i]);
   }
-  // gphi(j) = 2 / rcsq * sum_k g(k, j) (ztv1 - gt)(k)
+  if constexpr (ROW > 0) {
+    C2<R>* tws = (C2<R>*)(cr + n * P) + W * C::NFB * C::NP;
+    for (int k = threadIdx.x; k < ROW; k += 512) tws[k] = C2<R>{tw[k].x, -tw[k].y};
+  }
+
+  // ---- zvgpg = rcsq (u d/dlambda + v d/dmu) ln ps, the divergence, and the
+  // virtual temperature's humidity term.  The reference forms (gt + t0)(1 +
+  // (1/rdbrv - 1) zq) - t0 and then subtracts gt again for gphi
+  // (src/plasim.f90:2617-2622, 2742): t0 is large against the humidity term,
+  // and the subtractions cancel it.  The same quantities in the form without
+  // the cancellation: corr = (gt + t0)(1/rdbrv - 1) zq, ztv1 = gt + corr, ztv1
+  // - gt = corr and ztv2 = (gt + corr - t0 adv zq) / (1 + adv zq). ----
+  for (int j = w; j < n; j += W) {
 #pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    if (j >= n) break;
-    R s = R(0);
-#pragma unroll
-    for (int k = 0; k < NA; ++k) {
-      if (k >= n) break;
-      s = s + g[j * n + k] * ztv1d[k];
+    for (int i = 0; i < PPL; ++i) {
+      const R gu = at(f.gu, j, i), gv = at(f.gv, j, i), gd = at(f.gd, j, i);
+      const R gt = at(f.gt, j, i);
+      R zq = (nqspec == 1) ? at(f.gq, j, i) / gp[i] : at(f.dq, j, i);
+      zq = zq > R(0) ? zq : R(0);
+      zg[j * P + lane + 64 * i] = R2{rcsq[i] * (gu * gpm[i] + gv * gpj[i]), gd};
+      cr[j * P + lane + 64 * i] = (gt + t0v[j]) * (qfac * zq);
     }
-    const R gphi = s * R(2) / rcsq;
-    put(f.gphi, j, gphi);
-    if (f.gke) put(f.gke, j, ke[j] + gphi);
+  }
+  __syncthreads();
+  if (w == 0) {
+    // (after the barrier: every wave has read gp)
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      if (exp_gp) put(f.gp, 0, i, gp[i]);
+      if (sid) put(rcsq_out, 0, i, rcsq[i]);
+    }
+  }
+
+  // ---- this wave's levels [j0, j1) ----
+  const int j0 = w * (n / W) + (w < n % W ? w : n % W);
+  const int j1 = j0 + n / W + (w < n % W ? 1 : 0);
+  if (j0 >= j1) return;  // no barrier follows
+  // the sums of the sigma-dot integral in the reference's order: over all
+  // levels (zsumd, vp), and over the levels above j0 (rz, rv)
+  R tot[PPL], vp[PPL], rz[PPL], rv[PPL];
+#pragma unroll
+  for (int i = 0; i < PPL; ++i) tot[i] = vp[i] = rz[i] = rv[i] = R(0);
+#pragma unroll 4
+  for (int k = 0; k < n; ++k) {
+    const R dk = dsig[k];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      if (k == j0) rz[i] = tot[i], rv[i] = vp[i];
+      const R2 x = zg[k * P + lane + 64 * i];
+      tot[i] = tot[i] + dk * x.y;
+      vp[i] = vp[i] + dk * x.x;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < PPL; ++i) tot[i] = tot[i] + vp[i];
+  if (ROW == 0 && w == 0) {
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) put(f.gvp, 0, i, vp[i]);
+  }
+  // the terms at the interface above level j (gtd, gqm, gud, gvd of level
+  // j - 1, and tim = t01s2 (sigmah gvp - the sum of zvgpg dsigma)), carried one
+  // level on; zero above the top and below the bottom
+  R gt[PPL], gq[PPL], gu[PPL], gv[PPL];
+  R gtd_m[PPL], gqm_m[PPL], gud_m[PPL], gvd_m[PPL], tim[PPL];
+  {
+    const int jm = j0 > 0 ? j0 - 1 : 0;
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      gt[i] = at(f.gt, j0, i), gq[i] = at(f.gq, j0, i);
+      gu[i] = at(f.gu, j0, i), gv[i] = at(f.gv, j0, i);
+      const R zsdotp = sigh[jm] * tot[i] - (rz[i] + rv[i]);
+      const R a = zsdotp * (gt[i] - at(f.gt, jm, i)), b = zsdotp * (gq[i] + at(f.gq, jm, i));
+      const R c = zsdotp * (gu[i] - at(f.gu, jm, i)), d = zsdotp * (gv[i] - at(f.gv, jm, i));
+      const R e = t01[jm] * (sigh[jm] * vp[i] - rv[i]);
+      gtd_m[i] = j0 > 0 ? a : R(0), gqm_m[i] = j0 > 0 ? b : R(0);
+      gud_m[i] = j0 > 0 ? c : R(0), gvd_m[i] = j0 > 0 ? d : R(0);
+      tim[i] = j0 > 0 ? e : R(0);
+    }
+  }
+  C2<R>* fb = (C2<R>*)(cr + n * P) + w * C::NFB * C::NP;  // this wave's FFT rows
+  for (int j = j0; j < j1; ++j) {
+    const bool top = j == 0, bottom = j == n - 1;
+    // this level's inputs first, so that they arrive during the sums below
+    const int jp = bottom ? j : j + 1;
+    R gz[PPL], gt1[PPL], gq1[PPL], gu1[PPL], gv1[PPL], dq[PPL];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      gz[i] = at(f.gz, j, i);
+      gt1[i] = at(f.gt, jp, i), gq1[i] = at(f.gq, jp, i);
+      gu1[i] = at(f.gu, jp, i), gv1[i] = at(f.gv, jp, i);
+      if (nqspec != 1) dq[i] = at(f.dq, j, i);
+    }
+    // c(k, j) for k <= j: column j of c; ztptb = ztpta + the same sum over the
+    // divergence
+    R ztpta[PPL], ztptb[PPL], gphi[PPL];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) ztpta[i] = ztptb[i] = gphi[i] = R(0);
+    const Uni<R> cj = (Uni<R>)v.c + j * n, gj = (Uni<R>)v.g + j * n;
+#pragma unroll 4
+    for (int k = 0; k <= j; ++k) {
+      const R ck = cj[k];
+#pragma unroll
+      for (int i = 0; i < PPL; ++i) {
+        const R2 x = zg[k * P + lane + 64 * i];
+        ztpta[i] = ztpta[i] + ck * x.x;
+        ztptb[i] = ztptb[i] + ck * x.y;
+      }
+    }
+    // gphi(j) = 2 / rcsq * sum_k g(k, j) (ztv1 - gt)(k)
+#pragma unroll 4
+    for (int k = 0; k < n; ++k) {
+      const R gk = gj[k];
+#pragma unroll
+      for (int i = 0; i < PPL; ++i) gphi[i] = gphi[i] + gk * cr[k * P + lane + 64 * i];
+    }
+    R out[10][PPL];  // gtn gqn guz gvz gut gvt guq gvq gke, and gvp at the top
+    const R rd = rdsig[j], dsj = bottom ? R(0) : dsig[j], shj = sigh[j], t01j = t01[j];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) {
+      const R2 x = zg[j * P + lane + 64 * i];
+      const R zv = x.x, gd = x.y, corr = cr[j * P + lane + 64 * i];
+      R zq = (nqspec == 1) ? gq[i] / gp[i] : dq[i];
+      zq = zq > R(0) ? zq : R(0);
+      ztptb[i] = ztpta[i] + ztptb[i];
+      const R ztv1 = gt[i] + corr;
+      const R ztv2 = (gt[i] + corr - t0v[j] * (v.adv * zq)) / (R(1) + v.adv * zq);
+      gphi[i] = gphi[i] * R(2) / rcsq[i];
+      // (sigma-dot times the differences across the interface below j)
+      rz[i] = rz[i] + dsj * gd;
+      rv[i] = rv[i] + dsj * zv;
+      const R zsdotp = shj * tot[i] - (rz[i] + rv[i]);
+      const R gtd = bottom ? R(0) : zsdotp * (gt1[i] - gt[i]);
+      const R gqm = bottom ? R(0) : zsdotp * (gq1[i] + gq[i]);
+      const R gud = bottom ? R(0) : zsdotp * (gu1[i] - gu[i]);
+      const R gvd = bottom ? R(0) : zsdotp * (gv1[i] - gv[i]);
+      const R ti = bottom ? R(0) : t01j * (shj * vp[i] - rv[i]);
+      const R za = top ? -gd : zv - ztptb[i], zt = top ? R(0) : tkp[j] * (zv - ztpta[i]);
+      const R dw = (top ? gd : za) * gp[i] * v.psurf * v.ww;
+      put(f.dw, j, i, dw);
+      put(f.gphi, j, i, gphi[i]);
+      out[0][i] = gt[i] * gd + v.akap * ztv2 * za + zt - rd * (gtd + gtd_m[i] + ti + tim[i]);
+      out[1][i] = -rd * (gqm - gqm_m[i]);
+      out[2][i] = -gu[i] * gz[i] - gpj[i] * ztv1 - rd * (gvd + gvd_m[i]);
+      out[3][i] = gv[i] * gz[i] - gpm[i] * ztv1 - rd * (gud + gud_m[i]);
+      out[4][i] = gu[i] * gt[i];
+      out[5][i] = gv[i] * gt[i];
+      out[6][i] = gu[i] * gq[i];
+      out[7][i] = gv[i] * gq[i];
+      out[8][i] = gu[i] * gu[i] + gv[i] * gv[i] + gphi[i];
+      out[9][i] = top ? vp[i] : R(0);
+      if constexpr (ROW > 0 && C::NFB == 5) {
+        // (straight into the FFT rows, one point's values in registers at a time)
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+          fb[q * C::NP + bix(lane + 64 * i)] = C2<R>{out[2 * q][i], out[2 * q + 1][i]};
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      gtd_m[i] = gtd, gqm_m[i] = gqm, gud_m[i] = gud, gvd_m[i] = gvd, tim[i] = ti;
+      gt[i] = gt1[i], gq[i] = gq1[i], gu[i] = gu1[i], gv[i] = gv1[i];
+    }
+    R* const dst[10] = {f.gtn, f.gqn, f.guz, f.gvz, f.gut, f.gvt, f.guq, f.gvq, f.gke, f.gvp};
+    if constexpr (ROW == 0) {
+#pragma unroll
+      for (int q = 0; q < 9; ++q)
+        if (dst[q] && (q < 6 || q > 7 || nqspec == 1)) {
+#pragma unroll
+          for (int i = 0; i < PPL; ++i) put(dst[q], j, i, out[q][i]);
+        }
+    } else {
+      // gp2fc: z = out[2q] + i out[2q + 1], separated by the Hermitian pair
+      constexpr int NFB = C::NFB, NP = C::NP, N = ROW;
+      const C2<R>* tws = (const C2<R>*)(cr + n * P) + W * NFB * NP;
+      const R sc = R(0.5) / R(N);
+#pragma unroll
+      for (int q0 = 0; q0 < 5; q0 += NFB) {
+        if constexpr (NFB < 5) {
+#pragma unroll
+          for (int q = q0; q < q0 + NFB && q < 5; ++q)
+#pragma unroll
+            for (int i = 0; i < PPL; ++i)
+              fb[(q - q0) * NP + bix(lane + 64 * i)] = C2<R>{out[2 * q][i], out[2 * q + 1][i]};
+        }
+        if (q0 + NFB <= 5)
+          fft_wave_rows<N, NFB, -1>(fb, tws, lane);
+        else
+          fft_wave_rows<N, (5 % NFB ? 5 % NFB : 1), -1>(fb, tws, lane);
+#pragma unroll
+        for (int q = q0; q < q0 + NFB && q < 5; ++q) {
+          if (q == 3 && nqspec != 1) continue;
+#pragma unroll
+          for (int k0 = 0; k0 < N / 2; k0 += 64) {
+            const int k = k0 + lane;
+            if (N / 2 % 64 && k >= N / 2) break;
+            const C2<R> zk = fb[(q - q0) * NP + bix(k)];
+            const C2<R> zn = fb[(q - q0) * NP + bix(k ? N - k : 0)];
+            const long o = mo + (long)j * nhor + 2 * k0;
+            ((R2*)(dst[2 * q] + o))[(unsigned)lane] = R2{(zk.x + zn.x) * sc, (zk.y - zn.y) * sc};
+            if (q < 4 || top)
+              ((R2*)(dst[2 * q + 1] + o))[(unsigned)lane] =
+                  R2{(zk.y + zn.y) * sc, (zn.x - zk.x) * sc};
+          }
+        }
+        wave_lds_sync();  // the rows are read before the next ones are written
+      }
+    }
   }
 }
 
@@ -300,7 +436,7 @@ extern "C" int exo_dyn_destroy(exo_dyn_t d) {
 template <typename R>
 static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int exp_gp,
                     const exo_calcgp_fields* f, hipStream_t s, const double* sid = nullptr,
-                    int nlon = 1, void* rcsq_out = nullptr) {
+                    int nlon = 1, void* rcsq_out = nullptr, const void* tw = nullptr) {
   CalcgpPtrs<R> p;
   p.gu = (const R*)f->gu;
   p.gv = (const R*)f->gv;
@@ -326,17 +462,37 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
   p.guq = (R*)f->guq;
   p.gvq = (R*)f->gvq;
   const DynVert<R> v = vert_of<R>(d);
-  dim3 grid((unsigned)((nhor + 255) / 256), (unsigned)nmem);
-  auto launch = [&](auto kern) {
-    kern<<<grid, 256, 0, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp, sid, nlon, (R*)rcsq_out);
+  auto launch = [&](auto kern, int points, size_t lds) -> int {
+    if (lds > 65536 &&
+        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
+      return EXO_ERR_LAUNCH;
+    const dim3 grid((unsigned)((nhor + points - 1) / points), (unsigned)nmem);
+    kern<<<grid, 512, lds, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp, sid, nlon, (R*)rcsq_out,
+                                (const C2<R>*)tw);
+    return hipGetLastError() == hipSuccess ? EXO_OK : EXO_ERR_LAUNCH;
   };
-  switch (d->nlev) {
-    case 10: launch(k_calcgp<R, 10>); break;
-    case 20: launch(k_calcgp<R, 20>); break;
-    case 40: launch(k_calcgp<R, 40>); break;
-    default: launch(k_calcgp<R, 0>); break;
+  const int n = d->nlev;
+  switch (tw ? nlon : 0) {
+    case 64: return launch(k_calcgp<R, 64>, 64, GpCfg<R, 64>::lds(n));
+    case 128: return launch(k_calcgp<R, 128>, 128, GpCfg<R, 128>::lds(n));
+    default: return launch(k_calcgp<R, 0>, 64, GpCfg<R, 0>::lds(n));
   }
-  return hipGetLastError() == hipSuccess ? EXO_OK : EXO_ERR_LAUNCH;
+}
+
+// Does gridpointa's calcgp transform its rows itself?  On rows of 64 and 128
+// whose level arrays fit a CU's LDS (all levels but FP64 above L40 on 128).
+// Three points per lane on rows of 192 spill (T63 L20, 16 members, FP32: 479 us
+// against 390 with calcgp on the grid and the row FFT as a launch; FP64, 3
+// members: 289 against 253).
+constexpr size_t GP_LDS = 160 * 1024;
+static bool calcgp_rows(int mode, int nlon, int nlev) {
+  const bool d = mode == MODE_F64;
+  switch (nlon) {
+    case 64: return (d ? GpCfg<double, 64>::lds(nlev) : GpCfg<float, 64>::lds(nlev)) <= GP_LDS;
+    case 128: return (d ? GpCfg<double, 128>::lds(nlev) : GpCfg<float, 128>::lds(nlev)) <= GP_LDS;
+    default: return false;
+  }
 }
 
 extern "C" int exo_dyn_calcgp(exo_dyn_t d, int mode, int nmem, long member_stride, int nhor,
@@ -483,15 +639,18 @@ extern "C" int exo_gridpointa(exo_sht_plan_t p, exo_dyn_t d, int mode, int nmem,
   f.gke = slot(sl.gke);
   f.guq = nqspec ? slot(sl.guq) : nullptr;
   f.gvq = nqspec ? slot(sl.gvq) : nullptr;
+  const bool rows = calcgp_rows(mode, tb.nlon, n);
+  const void* tw = !rows ? nullptr : mode == MODE_F64 ? (const void*)tb.tw64 : (const void*)tb.tw32;
   int rc = mode == MODE_F64 ? calcgp_t<double>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s,
-                                               tb.sid, tb.nlon, slot(sl.rcsq))
+                                               tb.sid, tb.nlon, slot(sl.rcsq), tw)
                             : calcgp_t<float>(d, nmem, work_stride, (int)nhor, nqspec, 1, &f, s,
-                                              tb.sid, tb.nlon, slot(sl.rcsq));
+                                              tb.sid, tb.nlon, slot(sl.rcsq), tw);
   if (rc) return rc;
 
-  // gp2fc of the nine tendency fields and gvpp, in place
-  if (launch_fft(tb, mode, -1, slot(sl.a), tb.nlon, (long)(9 * n + 1) * tb.nlat, s, nmem,
-                 work_stride))
+  // gp2fc of the nine tendency fields and gvpp, in place, where calcgp has
+  // not done it
+  if (!rows && launch_fft(tb, mode, -1, slot(sl.a), tb.nlon, (long)(9 * n + 1) * tb.nlat, s, nmem,
+                          work_stride))
     return EXO_ERR_LAUNCH;
 
   // mktend -> szt, sdt, stt; qtend -> sqt; fc2sp(gvpp) -> spt (src/plasim.f90:2473-2486)

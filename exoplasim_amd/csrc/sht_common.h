@@ -581,6 +581,52 @@ __device__ __forceinline__ void fft_wave(C2<F>* row, const C2<F>* tw, int lane, 
   wave_lds_sync();
 }
 
+// One Stockham pass (radix R, stride NS) of the NF rows of N + N/32 complex
+// values in `buf`, in place, by one wave; tw[k] = e^{S 2 pi i k / N}.
+template <int N, int R, int NS, int NF, int S, typename F>
+__device__ __forceinline__ void fft_wave_pass(C2<F>* buf, const C2<F>* tw, int lane) {
+  constexpr int NB = N / R, NP = N + N / 32, TOT = NF * NB, BPT = (TOT + 63) / 64;
+  C2<F> v[BPT][R];
+#pragma unroll
+  for (int t = 0; t < BPT; ++t) {
+    const int b = lane + 64 * t;
+    if (b < TOT) {
+      const int f = b / NB, j = b - f * NB;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[t][r] = buf[f * NP + bix(j + r * NB)];
+    }
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int t = 0; t < BPT; ++t) {
+    const int b = lane + 64 * t;
+    if (b < TOT) {
+      const int f = b / NB, j = b - f * NB, jm = j % NS;
+      if (NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[t][r] = cmul(v[t][r], tw[jm * r * (N / (NS * R))]);
+      }
+      Dft<R, S, F>::run(v[t]);
+      const int o = (j / NS) * NS * R + jm;
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf[f * NP + bix(o + r * NS)] = v[t][r];
+    }
+  }
+  wave_lds_sync();
+}
+
+// FFTs of the NF rows in `buf`, in place, by one wave (only the calling wave
+// touches them), with the radices of FftPlan<N>
+template <int N, int NF, int S, typename F>
+__device__ __forceinline__ void fft_wave_rows(C2<F>* buf, const C2<F>* tw, int lane) {
+  using P = FftPlan<N>;
+  static_assert(P::NP == 2 || P::NP == 3, "two or three passes");
+  wave_lds_sync();
+  fft_wave_pass<N, P::R[0], 1, NF, S>(buf, tw, lane);
+  fft_wave_pass<N, P::R[1], P::R[0], NF, S>(buf, tw, lane);
+  if constexpr (P::NP == 3) fft_wave_pass<N, P::R[2], P::R[0] * P::R[1], NF, S>(buf, tw, lane);
+}
+
 // ---- split-BF16 helpers ----
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));

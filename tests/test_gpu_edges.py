@@ -81,3 +81,115 @@ def test_direct_sums_edges(oracle, gpu, ntru, nlev, mode):
         for i, w in enumerate(want):
             assert rel(got[i][k], w) < (1e-12 if mode == "f64" else 1e-6), (i, k)
     p.close()
+
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
+from make_golden import (PLASIM_SCAL, gridpointa_humidity, gridpointa_state,  # noqa: E402
+                         plasim_inputs)
+
+CT = (6371220.0 * 7.292e-5) ** 2 / 287.0
+
+
+def _vertical(oracle, nlev):
+    return oracle.vertical(nlev, t0=np.linspace(220.0, 288.0, nlev) / CT)
+
+
+def _gphi(f, v, nq):
+    """the geopotential term in the form without the cancellation of (gt + t0)
+    (1 + a) - t0 - gt, a = (1/rdbrv - 1) q of 1e-4 to 1e-3, which costs the
+    oracle's form a factor 1 / a in rounding (up to 1e-12, and 1.35e-12 in the
+    divergence tendency of T127 through the Laplacian)"""
+    q = f["gq"] / f["gp"] if nq else f["dq"]
+    corr = (f["gt"] + v["t0"][:, None]) * (1.0 / PLASIM_SCAL[0] - 1.0) * np.maximum(q, 0.0)
+    return 2.0 / f["rcsq"] * (v["g"].T @ corr)
+
+
+@pytest.mark.parametrize("nlev,nhor", [(2, 1), (3, 64), (7, 65), (9, 127), (64, 200)])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+def test_calcgp_edges(oracle, gpu, nlev, nhor, mode):
+    """fewer levels than a block's waves, one more, the largest count; fewer
+    points than a block, whole and one over.  Tolerances as for the other
+    level counts: 1e-12 in FP64, 2e-5 in FP32 (the geopotential and sigma-dot
+    sums cancel to about 1/20 of their terms)."""
+    import torch
+
+    from exoplasim_amd.dynamics import CALCGP_OUT, PRODUCTS, Dynamics
+
+    print(f"calcgp L{nlev} x{nhor} {mode}", flush=True)
+    v = _vertical(oracle, nlev)
+    dyn = Dynamics.from_vertical(v, *PLASIM_SCAL)
+    dt = torch.float64 if mode == "f64" else torch.float32
+    f = {k: x[..., :nhor].copy() for k, x in plasim_inputs(nlev, 256, 5)[1].items()}
+    if mode == "f32":
+        f = {k: x.astype(np.float32).astype(np.float64) for k, x in f.items()}
+    dev = {k: torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt) for k, x in f.items()}
+    for k in CALCGP_OUT + PRODUCTS:
+        dev[k] = torch.full((nlev, nhor), float("nan"), dtype=dt, device="cuda")
+    dev["gvp"] = torch.full((nhor,), float("nan"), dtype=dt, device="cuda")
+    dyn.calcgp(mode, dev, nqspec=1)
+    got = {k: x.double().cpu().numpy() for k, x in dev.items()}
+    want = oracle.calcgp(f, v, PLASIM_SCAL, 1)
+    want["gphi"] = _gphi(f, v, 1)
+    want.update(gut=f["gu"] * f["gt"], gvt=f["gv"] * f["gt"], guq=f["gu"] * f["gq"],
+                gvq=f["gv"] * f["gq"], gke=f["gu"] ** 2 + f["gv"] ** 2 + want["gphi"])
+    for k, w in want.items():
+        assert rel(got[k], w) < (1e-12 if mode == "f64" else 2e-5), k
+    dyn.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,mode", [(21, 2, "f64"), (21, 9, "f32"), (42, 7, "f64"),
+                                            (42, 41, "f64"), (42, 33, "bf16x3"), (63, 5, "f32"),
+                                            (127, 3, "f64")])
+@pytest.mark.parametrize("nq", [1, 0])
+def test_gridpointa_edges(oracle, gpu, ntru, nlev, mode, nq):
+    """level counts around a block's 8 waves; rows transformed inside calcgp
+    and outside it (FP64 above L40 at T42, T63, T127), three members.  The
+    tendencies at 1e-12 in FP64 and 2e-5 in the FP32 modes, as for the other
+    sizes; the Fourier fields of the work array too, from the oracle's grid
+    fields through its gp2fc."""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.dynamics import Dynamics, work_slots
+
+    print(f"gridpointa T{ntru} L{nlev} {mode} nqspec={nq}", flush=True)
+    tol = 1e-12 if mode == "f64" else 2e-5
+    v = _vertical(oracle, nlev)
+    plan, dyn = sht.Plan(ntru), Dynamics.from_vertical(v, *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, 3, mode)
+    nlat, nlon, sl = plan.nlat, plan.nlon, work_slots(nlev)
+    states = [gridpointa_state(ntru, nlev, 0.9 + 0.1 * k) for k in range(3)]
+    st.copy_(torch.from_numpy(np.stack(states)).to(st.dtype))
+    hum = gridpointa_humidity(nlev, nlat * nlon)
+    if nq == 0:
+        for k, x in zip(("gq", "dq"), hum):
+            work[:, sl[k]:sl[k] + nlev] = torch.from_numpy(
+                x.reshape(nlev, nlat, nlon)).to("cuda", work.dtype)
+    dyn.gridpointa(plan, mode, st, work, tend, nqspec=nq)
+    got, wk = tend.double().cpu().numpy(), work.double().cpu().numpy()
+    cast = (lambda x: x) if mode == "f64" else (lambda x: x.astype(np.float32).astype(np.float64))
+    for k in (0, 2):
+        want, f = oracle.gridpointa(ntru, nlev, cast(states[k]), v, PLASIM_SCAL, nq,
+                                    gq=cast(hum[0]), dq=cast(hum[1]))
+        f["gphi"] = _gphi(f, v, nq)
+        f["gke"] = f["gu"] ** 2 + f["gv"] ** 2 + f["gphi"]
+        tab, one = oracle.legini(ntru, nlat), np.ones(ntru + 1)
+        four = {x: oracle.gp2fc(f[x].reshape(-1, nlat, nlon), nlon == 192)
+                for x in ("gtn", "gvz", "guz", "gke", "gut", "gvt")}
+        want[nlev:2 * nlev] = oracle.mktend(
+            ntru, nlat, nlon, nlev, tab["qc"], tab["qe"], tab["qm"], tab["qq"], one,
+            *[four[x] for x in ("gtn", "gvz", "guz", "gke", "gut", "gvt")])[0]
+        for i in range(4 if nq else 3):
+            s = slice(i * nlev, (i + 1) * nlev)
+            assert rel(got[k, s], want[s]) < tol, (k, i)
+        assert rel(got[k, 4 * nlev], want[4 * nlev]) < tol, k
+        for name in ("gtn", "gqn", "guz", "gvz", "gut", "gvt", "gke", "gvp") + (
+                ("guq", "gvq") if nq else ()):
+            rows = f[name].reshape(-1, nlat, nlon)
+            w = oracle.gp2fc(rows, nlon == 192)
+            assert rel(wk[k, sl[name]:sl[name] + len(rows)], w) < tol, (k, name)
+        for name in ("gphi", "dw", "gp", "rcsq"):
+            w = f[name].reshape(-1, nlat, nlon)
+            assert rel(wk[k, sl[name]:sl[name] + len(w)], w) < tol, (k, name)
+    dyn.close()
+    plan.close()
