@@ -193,3 +193,40 @@ def test_gridpointa_edges(oracle, gpu, ntru, nlev, mode, nq):
             assert rel(wk[k, sl[name]:sl[name] + len(w)], w) < tol, (k, name)
     dyn.close()
     plan.close()
+
+
+@pytest.mark.parametrize("nlev,ncol", [(2, 1), (5, 9), (7, 300), (31, 17), (32, 5), (63, 33)])
+@pytest.mark.parametrize("fp64", [True, False])
+def test_lwr_edges(oracle, gpu, nlev, ncol, fp64):
+    """level counts whose pairs of levels leave lanes with short, empty or
+    several-row runs, the last of 32 lanes and the first and last of 64, and
+    ragged blocks of columns.  FP64 at the bar of the other lwr tests (1e-10:
+    the layer emission cancels to 2e-11 of the flux where a transmissivity is
+    clamped).  FP32: flux sums of up to 63 terms of about 400 W/m2 round at
+    2.4e-5 each, layer differences of 0.1 W/m2 and more: 1e-3 of the heating,
+    1e-4 of the OLR."""
+    import torch
+
+    import oracle as O
+    from exoplasim_amd.radiation import LwrColumn, sigma_levels
+
+    print(f"lwr L{nlev} x{ncol} fp64={fp64}", flush=True)
+    rng = np.random.default_rng(nlev)
+    s = sigma_levels(nlev)[0]
+    t = 190.0 + 110.0 * np.sqrt(s) + rng.uniform(-2, 2, (ncol, nlev))
+    cols = {"dt": np.concatenate([t, t[:, -1:] + rng.uniform(1, 5, (ncol, 1))], axis=1),
+            "dq": np.exp(rng.uniform(np.log(1e-5), np.log(2e-2), (ncol, nlev))),
+            "dp": rng.uniform(5e4, 1.5e5, ncol),
+            "dqco2": np.repeat(np.exp(rng.uniform(3, 9, (ncol, 1))), nlev, axis=1),
+            "dqo3": 1e-6 * rng.random((ncol, nlev)), "dcc": 0.5 * rng.random((ncol, nlev)),
+            "dql": 1e-5 * rng.random((ncol, nlev)), "dls": (rng.random(ncol) < 0.5) * 1.0}
+    dt = torch.float64 if fp64 else torch.float32
+    dev = {k: torch.from_numpy(np.ascontiguousarray(x.T)).to("cuda", dt) for k, x in cols.items()}
+    heat, olr, fu, fd = LwrColumn(nlev, fp64=fp64)(dev, fluxes=True)
+    host = {k: np.ascontiguousarray(x.double().cpu().numpy().T) for k, x in dev.items()}
+    wu, wd, wh, wo = O.lwr(oracle, host, nlev)
+    tol = (1e-10, 1e-10) if fp64 else (1e-3, 1e-4)
+    assert rel(heat.double().cpu().numpy(), wh.T * 86400.0) < tol[0]
+    assert rel(olr.double().cpu().numpy(), wo) < tol[1]
+    assert rel(fu.double().cpu().numpy(), wu.T) < tol[1]
+    assert rel(fd.double().cpu().numpy(), wd.T) < tol[1]
