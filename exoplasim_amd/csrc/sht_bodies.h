@@ -119,7 +119,7 @@ __host__ __device__ inline long inv_items(const InvArgs& a) {
 // member mem, decoded from blk.  lds holds InvLds::BYTES bytes.
 template <int T, int MODE, int KIND, bool FUSED, int V>
 __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* tabA0,
-                                         const void* tabA1, long plane, const void* tabv,
+                                         const void* tabA1, const void* tabv,
                                          const void* twp, char* lds) {
   using S = TS<T>;
   using R = RealT<MODE>;
@@ -220,17 +220,31 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
   if constexpr (MODE == MODE_BF16X3 || MODE == MODE_F32MFMA || MODE == MODE_F64) {
     // GEMM per m: C[row = 2*pair + class][col] = sum_n A[row][n] B[n][col];
     // split-BF16 on v_mfma_f32_16x16x32_bf16, FP32 on v_mfma_f32_16x16x4_f32,
-    // FP64 on v_mfma_f64_16x16x4_f64 (the FP32 operand layouts in doubles);
+    // FP64 on v_mfma_f64_16x16x4_f64;
     // wave wv of NW takes m = wv, wv + NW, ...; each (m, 32-wide n block) is
     // one work item, and the operands of the items ahead are fetched before
     // the current one is multiplied.
+    // FP64: the rows are 8 pairs x the two parities h of n - m, the columns
+    // (at most 8: FB <= 4) once per parity, c = 8 h + column, and k counts the
+    // values of one parity, so that the quadrants of equal parity hold the
+    // sums over the even and over the odd n - m; the other two quadrants are
+    // not used.  Half the matrix instructions and half the table bytes of the
+    // FP32 form, whose rows hold zeros at every other n and whose columns 2 FB
+    // .. 15 are empty at FB = 4; the spectral loads use all lanes.  (Round trip
+    // of T42 L20, 32 members, 288 -> 184 us; gridpointa of T63 L20, 3 members,
+    // 272 -> 189; a T21 L10 step 43 -> 37.  The FP64 matrix rate then bounds
+    // the Legendre sums: 64 cycles per instruction, half of it used.)
     // The wave index is read into a scalar register, so that the item loop
     // (m, kb), its branches and the operand offsets are wave-uniform scalar
     // work rather than per-lane vector arithmetic.
     const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q = lane >> 4, c = lane & 15;
-    // column c of B: SCALAR field g*FB + c/2; UV level g*FB/2 + c/4 of
-    // vorticity ((c/2)&1 == 0) or divergence; component c&1
+    const int q = lane >> 4;
+    // column c of B (FP64: c = lane % 8, of parity hc = lane / 8 % 2): SCALAR
+    // field g*FB + c/2; UV level g*FB/2 + c/4 of vorticity ((c/2)&1 == 0) or
+    // divergence; component c&1
+    const int c = (MODE == MODE_F64) ? lane & 7 : lane & 15;
+    const int hc = (lane >> 3) & 1;
+    static_assert(MODE != MODE_F64 || FB <= 4, "FP64: 8 columns per parity");
     const R* bp = nullptr;  // F32MFMA, F64: the column's coefficients
     bool isvor = false;
     int pf = -1;  // field of column c
@@ -245,8 +259,12 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         isvor = (s == 0) && ((c & 1) == 0);
       }
     }
-    if constexpr (MODE != MODE_BF16X3) {
+    if constexpr (MODE == MODE_F32MFMA) {
       if (pf >= 0) bp = spm + (long)pf * S::NRSP + (c & 1);
+    } else if constexpr (MODE == MODE_F64) {
+      // columns without a field read the block's first field and use none of it
+      const int p0 = (KIND == INV_SCALAR) ? a.src0 + g * FB : a.vor0 + g * (FB / 2);
+      bp = spm + (long)(pf >= 0 ? pf : p0) * S::NRSP + (c & 1);
     }
     // Operands through buffer loads: a per-lane byte offset plus a
     // wave-uniform byte offset per item.
@@ -254,11 +272,12 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // element j = 16 kb + 8 (q & 1) .. + 7 (layouts in sht_common.h).
     // A: the table rows of pair block pb; a lane whose parity is not its
     // row's class, or whose j lies past the row, reads past the buffer,
-    // which returns the zeros.  F32MFMA, F64: item (m, kb) at ((m KB + kb)
-    // 512) elements of the block's table.
+    // which returns the zeros.  F32MFMA, F64: item (m, kb) at (m KB + kb) EPB
+    // elements of the block's table, KPL values per lane.
+    constexpr int KPL = (MODE == MODE_F64) ? 4 : 8, EPB = 64 * KPL;
     constexpr int AE = (MODE == MODE_BF16X3) ? 2 : (int)sizeof(R);  // bytes per table element
-    const long abase = (MODE == MODE_BF16X3) ? (long)pb * tab_pb(T) : (long)pb * NM * S::KB * 512;
-    const int abytes = (MODE == MODE_BF16X3) ? tab_pb(T) * 2 : (int)(plane - abase) * AE;
+    const long abase = (MODE == MODE_BF16X3) ? (long)pb * tab_pb(T) : (long)pb * NM * S::KB * EPB;
+    const int abytes = (MODE == MODE_BF16X3) ? tab_pb(T) * 2 : (NPB - pb) * NM * S::KB * EPB * AE;
     const __amdgpu_buffer_rsrc_t rsA0 = buffer_rsrc((const char*)tabA0 + abase * AE, abytes);
     const __amdgpu_buffer_rsrc_t rsA1 =
         buffer_rsrc((const char*)(NTERM == 2 ? tabA1 : tabA0) + abase * AE, abytes);
@@ -266,7 +285,7 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // does this lane hold nonzero table values (its parity is its row's class)
     const bool amine0 = hq == ((c & 1) ^ (table_is_q(KIND == INV_UV ? TQV : a.table) ? 1 : 0));
     const bool amine1 = hq == ((c & 1) ^ (table_is_q(TQU) ? 1 : 0));
-    const int avoff = (q * 16 + c) * 8 * AE;  // F32MFMA, F64: 8 values per lane
+    const int avoff = lane * KPL * AE;  // F32MFMA, F64: row lane % 16, k % 4 = q
     // B (BF16X3): the member's parity-ordered fp32 operand; columns without
     // a field read past the buffer, which returns zeros
     __amdgpu_buffer_rsrc_t rsB = rsA0;
@@ -277,12 +296,13 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     }
     const int brow = (c & 1) * 2 + hq;  // re/im, parity row of the B segment
     const R pv = (R)a.plavor;
-    // B fragment of one item: 8 values (F32MFMA, F64: f, n = 4j + q), or 8
-    // fp32 values of one parity as loaded (BF16X3: r, split into the three
+    // B fragment of one item: 8 values (F32MFMA: f, n = 4j + q), 4 of one
+    // parity (F64: f, n - m = 2 (4j + q) + hc), or 8 fp32 values of one parity
+    // as loaded (BF16X3: r, split into the three
     // bf16 planes when the item is multiplied; fix marks the lane that holds
     // the absolute vorticity at (m=0, n=1, re))
     struct BFrag {
-      R f[8];
+      R f[KPL];
       uint4 r[2];
       bool fix;
     };
@@ -293,8 +313,8 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // 1-3% slower)
     constexpr bool PAIRLOAD = (MODE == MODE_BF16X3) && T >= 63;
     // 16-byte table loads per item and term: three bf16 planes (two with
-    // PAIRLOAD), or 8 values of 4 or 8 bytes
-    constexpr int NA = (MODE == MODE_BF16X3) ? (PAIRLOAD ? 2 : 3) : (8 * AE) / 16;
+    // PAIRLOAD), or KPL values of 4 or 8 bytes
+    constexpr int NA = (MODE == MODE_BF16X3) ? (PAIRLOAD ? 2 : 3) : (KPL * AE) / 16;
     // Every step fetches, also past the last item (m > T: nothing is loaded,
     // at the offsets of m = T), so that each step issues the same loads and
     // the wait for an item's operands counts only the loads issued before
@@ -354,18 +374,32 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         // table's buffer
         const int m = mi;
         const int w0 = w0_of(T, m <= T ? m : T);
+        if constexpr (MODE == MODE_F64) {
+          // every lane loads, past the row its last value, which is not used:
+          // no branch between the loads of an item
+          const int last = m <= T ? T - m : 0, use = (pf >= 0 && m <= T) ? T - m : -1;
+          const int i0 = kb * 32 + 2 * q + hc;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int n = m + kb * 32 + j * 4 + q;
-          R x = R(0);
-          if (bp && n <= T) {
-            x = bp[2 * (w0 + n - m)];
-            if (isvor && m == 0 && n == 1) x = x - pv;
+          for (int j = 0; j < KPL; ++j) {
+            const int i = i0 + 8 * j;
+            const R x = bp[2 * (w0 + (i < last ? i : last))];
+            br.f[j] = i <= use ? x : R(0);
           }
-          br.f[j] = x;
+          br.fix = isvor && m == 0 && i0 == 1;
+        } else {
+#pragma unroll
+          for (int j = 0; j < KPL; ++j) {
+            const int n = m + kb * 32 + j * 4 + q;
+            R x = R(0);
+            if (bp && n <= T) {
+              x = bp[2 * (w0 + n - m)];
+              if (isvor && m == 0 && n == 1) x = x - pv;
+            }
+            br.f[j] = x;
+          }
         }
-        // operand stored as [q][row][8] so one lane reads its 8 values
-        const int aso = (m * S::KB + kb) * 512 * AE;
+        // operand stored as [q][row][KPL] so one lane reads its KPL values
+        const int aso = (m * S::KB + kb) * EPB * AE;
 #pragma unroll
         for (int i = 0; i < NA; ++i) a0[i] = buffer_load_x4(rsA0, avoff, aso + 16 * i);
         if (NTERM == 2) {
@@ -416,15 +450,16 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         acc2 = mfma_bf16(ah, bp[0], acc2);
       } else if constexpr (MODE == MODE_F64) {
         const double* ad = (const double*)a;
+        const double f0 = br.fix ? br.f[0] - pv : br.f[0];
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[j], br.f[j], acc, 0, 0, 0);
+        for (int j = 0; j < KPL; j += 2) {
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[j], j ? br.f[j] : f0, acc, 0, 0, 0);
           acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[j + 1], br.f[j + 1], acc2, 0, 0, 0);
         }
       } else {
         const float* af = (const float*)a;
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
+        for (int j = 0; j < KPL; j += 2) {
           acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j], br.f[j], acc, 0, 0, 0);
           acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(af[j + 1], br.f[j + 1], acc2, 0, 0, 0);
         }
@@ -463,23 +498,50 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         const int m = cur.m;
         acc1 += acc1b;
         if (NTERM == 2) acc2 += acc2b;
-        Acc out = acc1;
-        if (KIND == INV_UV) {
-          // u = qv.zeta + qu.(-i D), v = qu.(-i zeta) - qv.D: the qu product of
-          // the partner column (zeta.re <-> D.im, zeta.im <-> D.re)
-          Acc p2;
+        // this lane's latitude pairs: symmetric and antisymmetric sums
+        constexpr int NPL = (MODE == MODE_F64) ? 1 : 2;
+        R sym[NPL], anti[NPL];
+        if constexpr (MODE == MODE_F64) {
+          // items 2h, 2h + 1 of a lane of parity h hold the sums of pairs 2q,
+          // 2q + 1; lanes c and c + 8 exchange one each and keep pair 2q + hc
+          auto even_odd = [&](const Acc& x, bool isq, R& sy, R& an) {
+            const R own = hc ? x[3] : x[0];
+            const R got = row_ror8(hc ? x[2] : x[1]);
+            sy = (hc != 0) != isq ? got : own;
+            an = (hc != 0) != isq ? own : got;
+          };
+          even_odd(acc1, table_is_q(KIND == INV_UV ? TQV : a.table), sym[0], anti[0]);
+          if (KIND == INV_UV) {
+            R s2, a2;
+            even_odd(acc2, table_is_q(TQU), s2, a2);
+            const R sa = (c & 2) ? R(-1) : R(1), sb = (c & 1) ? R(-1) : R(1);
+            sym[0] = sa * sym[0] + sb * quad_perm<0x1B>(s2);
+            anti[0] = sa * anti[0] + sb * quad_perm<0x1B>(a2);
+          }
+        } else {
+          Acc out = acc1;
+          if (KIND == INV_UV) {
+            // u = qv.zeta + qu.(-i D), v = qu.(-i zeta) - qv.D: the qu product of
+            // the partner column (zeta.re <-> D.im, zeta.im <-> D.re)
+            Acc p2;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) p2[i] = quad_perm<0x1B>(acc2[i]);  // lane ^ 3
-          // column c & 3 = 0: acc1 + p2, 1: acc1 - p2, 2: p2 - acc1, 3: -p2 - acc1
-          const R sa = (c & 2) ? R(-1) : R(1), sb = (c & 1) ? R(-1) : R(1);
+            for (int i = 0; i < 4; ++i) p2[i] = quad_perm<0x1B>(acc2[i]);  // lane ^ 3
+            // column c & 3 = 0: acc1 + p2, 1: acc1 - p2, 2: p2 - acc1, 3: -p2 - acc1
+            const R sa = (c & 2) ? R(-1) : R(1), sb = (c & 1) ? R(-1) : R(1);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) out[i] = sa * acc1[i] + sb * p2[i];
+            for (int i = 0; i < 4; ++i) out[i] = sa * acc1[i] + sb * p2[i];
+          }
+#pragma unroll
+          for (int h = 0; h < NPL; ++h) {
+            sym[h] = out[2 * h];
+            anti[h] = out[2 * h + 1];
+          }
         }
         const int fl = c >> 1, ri = c & 1;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int pl = 2 * q + h;
-          const R sy = out[2 * h], an = out[2 * h + 1];
+        for (int h = 0; h < NPL; ++h) {
+          const int pl = 2 * q + ((MODE == MODE_F64) ? hc : h);
+          const R sy = sym[h], an = anti[h];
           // component ri of the northern and southern coefficient
           R nv = sy + an, sv = sy - an;
           if (KIND == INV_SCALAR && a.dlam) {

@@ -102,14 +102,15 @@ static int build_tables(Tables& t, int ntru, const double* sid, const double* gw
   HIPCK(hipGetLastError());
   k_pack_fwd4<<<(unsigned)((nf + 255) / 256), 256>>>(t.npair, t.ncsp, t.filt32, t.fwd4);
   HIPCK(hipGetLastError());
-  t.inv_elems = (long)(t.npair / 8) * (ntru + 1) * t.kbmax * 512;
+  // 512 (FP32) and 256 (FP64) elements per (pair block, m, n block)
+  const long inv_blocks = (long)(t.npair / 8) * (ntru + 1) * t.kbmax;
   const int inv_tabs[] = {TQI, TQJ, TQU, TQV};
   for (int tt : inv_tabs) {
     const long nbf = (long)(t.npair / 8) * tab_pb(ntru);
     HIPCK(hipMalloc(&t.inv_bf[tt], sizeof(uint16_t) * nbf));
-    HIPCK(hipMalloc(&t.inv_f32[tt], sizeof(float) * t.inv_elems));
-    HIPCK(hipMalloc(&t.inv_f64[tt], sizeof(double) * t.inv_elems));
-    k_pack_inv<<<(unsigned)((t.inv_elems + 255) / 256), 256>>>(
+    HIPCK(hipMalloc(&t.inv_f32[tt], sizeof(float) * 512 * inv_blocks));
+    HIPCK(hipMalloc(&t.inv_f64[tt], sizeof(double) * 256 * inv_blocks));
+    k_pack_inv<<<(unsigned)((512 * inv_blocks + 255) / 256), 256>>>(
         ntru, t.npair, t.kbmax, tt, t.filt64, t.inv_f32[tt], t.inv_f64[tt]);
     HIPCK(hipGetLastError());
     const long nth = nbf / 3;

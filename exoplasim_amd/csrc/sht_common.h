@@ -126,6 +126,15 @@ __device__ __forceinline__ double quad_perm(double x) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// x from the lane 8 away within the row of 16 (DPP row rotation)
+__device__ __forceinline__ double row_ror8(double x) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, 0x128, 0xF, 0xF, false);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), 0x128, 0xF, 0xF, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // a per-lane byte offset that no buffer covers: such a load returns 0
 constexpr int BUF_NONE = 0x7ff00000;
 

@@ -32,7 +32,6 @@ struct EnsInvJob {
   const void* A1;
   const void* tv;
   const void* tw;
-  long plane;
   int ntru, var;
 };
 struct EnsFwdJob {
@@ -75,30 +74,30 @@ __device__ __forceinline__ void ens_inv_item(const EnsInvJob& jb, int blk, char*
   if (NT == 512) {
     if (jb.a.kind == INV_UV) {
       if (jb.var == 3)
-        inv_body<T, MODE, INV_UV, true, 3>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw, lds);
+        inv_body<T, MODE, INV_UV, true, 3>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw, lds);
       else
-        inv_body<T, MODE, INV_UV, true, 2>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw, lds);
+        inv_body<T, MODE, INV_UV, true, 2>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw, lds);
     } else {
       if (jb.var == 3)
-        inv_body<T, MODE, INV_SCALAR, true, 3>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw,
+        inv_body<T, MODE, INV_SCALAR, true, 3>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw,
                                                lds);
       else
-        inv_body<T, MODE, INV_SCALAR, true, 2>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw,
+        inv_body<T, MODE, INV_SCALAR, true, 2>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw,
                                                lds);
     }
     return;
   }
   if (jb.a.kind == INV_UV) {
     if (jb.var)
-      inv_body<T, MODE, INV_UV, true, 1>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw, lds);
+      inv_body<T, MODE, INV_UV, true, 1>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw, lds);
     else
-      inv_body<T, MODE, INV_UV, true, 0>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw, lds);
+      inv_body<T, MODE, INV_UV, true, 0>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw, lds);
   } else {
     if (jb.var)
-      inv_body<T, MODE, INV_SCALAR, true, 1>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw,
+      inv_body<T, MODE, INV_SCALAR, true, 1>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw,
                                              lds);
     else
-      inv_body<T, MODE, INV_SCALAR, true, 0>(jb.a, blk, jb.A0, jb.A1, jb.plane, jb.tv, jb.tw,
+      inv_body<T, MODE, INV_SCALAR, true, 0>(jb.a, blk, jb.A0, jb.A1, jb.tv, jb.tw,
                                              lds);
   }
 }
@@ -343,7 +342,6 @@ static int ens_prepare(exo_sht_ens_s* e) {
       }
       j.tv = tv;
       j.tw = tw;
-      j.plane = tb.inv_elems;
       j.ntru = tb.ntru;
       j.var = e->inv_var[k];
       long items = 0;

@@ -42,8 +42,7 @@ struct Tables {
   double* skspgp = nullptr;
   uint16_t* inv_bf[NTAB] = {};  // split-BF16 inverse table operands (3 planes)
   float* inv_f32[NTAB] = {};    // FP32-MFMA inverse table operands
-  double* inv_f64[NTAB] = {};   // FP64-MFMA inverse table operands (same layout)
-  long inv_elems = 0;           // elements of one inv_f32 (inv_f64) table
+  double* inv_f64[NTAB] = {};   // FP64-MFMA inverse table operands
   float* dir_f32[NTAB] = {};    // MFMA direct table operands (qc, qe, qm, qq)
   int dir_rb = 0;               // row tiles of 16 per (m, parity)
   double* tw64 = nullptr;     // [nlon] complex

@@ -149,16 +149,16 @@ __device__ void split3_f64(double x, uint16_t& h, uint16_t& m, uint16_t& l) {
   l = (uint16_t)(ul >> 16);
 }
 
-// ---- table operands of the FP32- and FP64-MFMA inverse: [pb][m][kb][512]
-// with MFMA row `row` and k = n - m - 32 kb, stored [k%4][row][k/4] per
-// 512-element block so that one lane of v_mfma_f32_16x16x4_f32 (or
-// v_mfma_f64_16x16x4_f64, the same operand layout) reads its 8 values
-// contiguously; zero where n > NTRU or the class does not match.  Both
-// instructions leave D[row][col] in lane 16 q + col, but in item v = row % 4
-// of q = row / 4 (FP32) or item v = row / 4 of q = row % 4 (FP64); the rows
-// are ordered so that item v of lane q holds pair 2q + v/2, class v % 2 in
-// both: FP32 row = 2 pair + class, FP64 row = (row % 4 = pair / 2, row / 4 =
-// 2 (pair % 2) + class) ----
+// ---- table operands of the FP32- and FP64-MFMA inverse, per (pair block, m,
+// block kb of 32 total wavenumbers n) ----
+// FP32: [pb][m][kb][512] with MFMA row 2 pair + class and k = n - m - 32 kb,
+// stored [k%4][row][k/4] so that one lane of v_mfma_f32_16x16x4_f32 reads its
+// 8 values contiguously; zero where n > NTRU or the class does not match.
+// FP64: [pb][m][kb][256], a row holding the 16 values of one parity h of n - m
+// (k = (n - m - 32 kb - h) / 2) of one pair, stored [k%4][row][k/4].
+// v_mfma_f64_16x16x4_f64 leaves D[row][col] in item v = row / 4 of lane 16
+// (row % 4) + col; the rows are ordered so that item v holds parity v / 2 of
+// pair 2 (row % 4) + v % 2.  Zero where n > NTRU.
 __global__ void k_pack_inv(int ntru, int npair, int kbmax, int t, const double* filt64,
                            float* f32, double* f64) {
   const int ncsp = (ntru + 1) * (ntru + 2) / 2;
@@ -184,7 +184,11 @@ __global__ void k_pack_inv(int ntru, int npair, int kbmax, int t, const double* 
   const long blk = i - (i % 512);
   const long o = blk + ((k % 4) * 16 + row) * 8 + k / 4;
   f32[o] = (float)val(row >> 1, row & 1);
-  f64[o] = val(2 * (row % 4) + (row / 4) / 2, (row / 4) % 2);
+  const int h = k & 1, e = k >> 1;  // FP64: one thread per pair of FP32 rows
+  if (row & 1) return;
+  const int pl = row >> 1, r64 = 4 * (2 * h + (pl & 1)) + (pl >> 1);
+  f64[blk / 2 + ((e % 4) * 16 + r64) * 4 + e / 4] =
+      n <= ntru ? filt64[t * tsz + (long)(pb * 8 + pl) * ncsp + w0_of(ntru, m) + (n - m)] : 0.0;
 }
 
 // ---- table operand of the split-BF16 inverse (layout in sht_common.h):

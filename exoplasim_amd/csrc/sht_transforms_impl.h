@@ -10,10 +10,10 @@ namespace exo {
 
 template <int T, int MODE, int KIND, bool FUSED, int V>
 __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv(InvArgs a, const void* tabA0, const void* tabA1,
-                                             long plane, const void* tabv, const void* twp) {
+                                             const void* tabv, const void* twp) {
   __shared__ __align__(16) char lds[InvLds<T, MODE, FUSED, V>::BYTES];
-  inv_body<T, MODE, KIND, FUSED, V>(a, xcd_block(blockIdx.x, gridDim.x), tabA0, tabA1, plane,
-                                    tabv, twp, lds);
+  inv_body<T, MODE, KIND, FUSED, V>(a, xcd_block(blockIdx.x, gridDim.x), tabA0, tabA1, tabv,
+                                    twp, lds);
 }
 
 // The inverse transforms of a round trip or of a dynamics step in one launch:
@@ -32,7 +32,7 @@ __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv(InvArgs a, con
 template <int T, int MODE, int V>
 __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv_rt(InvArgs aq, InvArgs aj, InvArgs au, const void* tq,
                                                 InvOneJobs one, const void* tv0, const void* tu,
-                                                long plane, const void* tabv, const void* twp,
+                                                const void* tabv, const void* twp,
                                                 int gq, int gj, int gu) {
   __shared__ __align__(16) char lds[InvLds<T, MODE, true, V>::BYTES];
   constexpr int NPB = TS<T>::NPAIR / InvCfg<T, MODE, V>::LP;
@@ -59,17 +59,17 @@ __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv_rt(InvArgs aq,
     r = b - mem * per;
   }
   if (r < NPB * gq)
-    inv_body<T, MODE, INV_SCALAR, true, V>(aq, mem * NPB * gq + r, tq, tu, plane, tabv, twp, lds);
+    inv_body<T, MODE, INV_SCALAR, true, V>(aq, mem * NPB * gq + r, tq, tu, tabv, twp, lds);
   else if (r < NPB * (gq + gj)) {
     const int k = __builtin_amdgcn_readfirstlane((r - NPB * gq) / NPB);
     aj.table = one.table[k];
     aj.dst0 = one.dst0[k];
     aj.dlam = one.dlam[k];
     inv_body<T, MODE, INV_SCALAR, true, V>(aj, mem * NPB + (r - NPB * (gq + k)), one.tab[k], tu,
-                                           plane, tabv, twp, lds);
+                                           tabv, twp, lds);
   }
   else
-    inv_body<T, MODE, INV_UV, true, V>(au, mem * NPB * gu + (r - NPB * (gq + gj)), tv0, tu, plane,
+    inv_body<T, MODE, INV_UV, true, V>(au, mem * NPB * gu + (r - NPB * (gq + gj)), tv0, tu,
                                        tabv, twp, lds);
 }
 
@@ -119,14 +119,14 @@ static int inv_tv(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s)
   dim3 grid((unsigned)nblk), block(InvCfg<T, MODE, V>::NT);
   if (a.kind == INV_UV) {
     if (fused)
-      k_inv<T, MODE, INV_UV, true, V><<<grid, block, 0, s>>>(a, A0, A1, tb.inv_elems, tv, tw);
+      k_inv<T, MODE, INV_UV, true, V><<<grid, block, 0, s>>>(a, A0, A1, tv, tw);
     else
-      k_inv<T, MODE, INV_UV, false, V><<<grid, block, 0, s>>>(a, A0, A1, tb.inv_elems, tv, tw);
+      k_inv<T, MODE, INV_UV, false, V><<<grid, block, 0, s>>>(a, A0, A1, tv, tw);
   } else {
     if (fused)
-      k_inv<T, MODE, INV_SCALAR, true, V><<<grid, block, 0, s>>>(a, A0, A1, tb.inv_elems, tv, tw);
+      k_inv<T, MODE, INV_SCALAR, true, V><<<grid, block, 0, s>>>(a, A0, A1, tv, tw);
     else
-      k_inv<T, MODE, INV_SCALAR, false, V><<<grid, block, 0, s>>>(a, A0, A1, tb.inv_elems, tv, tw);
+      k_inv<T, MODE, INV_SCALAR, false, V><<<grid, block, 0, s>>>(a, A0, A1, tv, tw);
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
@@ -178,7 +178,7 @@ static int inv_rt_tv(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int
   const void* tv = (MODE == MODE_F64) ? (const void*)tb.filt64 : (const void*)tb.filt32;
   const void* tw = (MODE == MODE_F64) ? (const void*)tb.tw64 : (const void*)tb.tw32;
   k_inv_rt<T, MODE, V><<<(unsigned)nblk, C::NT, 0, s>>>(aq, aj[0], au, tq, one, tv0, tu,
-                                                       tb.inv_elems, tv, tw, gq, nj, gu);
+                                                       tv, tw, gq, nj, gu);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
