@@ -491,9 +491,8 @@ extern "C" int exo_sht_set_tiles(exo_sht_plan_t p, int mode, int inv_var, int uv
 extern "C" int exo_sht_get_tiles(exo_sht_plan_t p, int mode, int* vars) {
   if (!p || !mode_ok(mode) || !vars) return EXO_ERR_ARG;
   std::lock_guard<std::mutex> lk(p->mu);
-  vars[0] = p->inv_var[mode];
-  vars[1] = p->uv_var[mode];
-  vars[2] = p->fwd_var[mode];
+  const int v[3] = {p->inv_var[mode], p->uv_var[mode], p->fwd_var[mode]};
+  for (int k = 0; k < 3; ++k) vars[k] = v[k] < 0 ? 0 : v[k];
   return EXO_OK;
 }
 

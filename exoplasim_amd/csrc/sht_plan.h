@@ -16,8 +16,9 @@ struct exo_sht_plan_s {
   // device address of the file-scope `scratch` array on the device the
   // plan was created on (exo_sht_roundtrip_noalloc)
   char* na_scratch = nullptr;
-  // tile variants per precision mode, chosen by exo_sht_autotune
-  int inv_var[4] = {0, 0, 0, 0}, uv_var[4] = {0, 0, 0, 0}, fwd_var[4] = {0, 0, 0, 0};
+  // tile variants per precision mode, chosen by exo_sht_autotune or
+  // exo_sht_set_tiles; -1: by the size of each call
+  int inv_var[4] = {-1, -1, -1, -1}, uv_var[4] = {-1, -1, -1, -1}, fwd_var[4] = {-1, -1, -1, -1};
   std::mutex mu;
 };
 

@@ -131,12 +131,32 @@ static int inv_tv(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s)
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
+// The tile variant of a fused inverse on a plan that was not tuned, from the
+// blocks it would have with half the fields per block (V = 3).  While those fit
+// the 256 CUs (two per CU where a block's LDS and its half-filled matrix tile
+// allow it: below T63, and in the FP32 mode, which uses no matrix tiles, at
+// T63) they only engage idle CUs; above, whole blocks on 512 threads.  Round
+// trip inverses in us, V = 0, 2, 3: T42 L20 BF16X3, 1 member 17.7, 13.8, 13.2;
+// 4 members 19.1, 15.2, 18.2; T63 L20 FP64, 1 member 24.9, 21.0, 27.5; L10
+// 24.0, 20.1, 18.1; T127 L10 FP32MFMA, 4 members 272, 155, 206.  The two
+// exceptions: FP64 at T21, whose short rows keep 256 threads busy (L20, 16
+// members 18.7, 21.0, 29.9), and FP32 up to T42, whose vector sums want the
+// most waves (T42 L20, 16 members 233, 145, 111).
+template <int T, int MODE>
+static int inv_auto(long nblk3) {
+  if (MODE == MODE_F64 && T == 21) return 0;
+  if (MODE == MODE_F32 && T <= 42) return 3;
+  constexpr bool two = MODE == MODE_F32 ? T < 127 : (MODE != MODE_F64 && T <= 42);
+  return nblk3 <= (two ? 512 : 256) ? 3 : 2;
+}
+
 // the unfused (drop-in) transforms always use the default tiles
 template <int T, int MODE>
 static int inv_t(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s) {
-  if (fused && a.var == 1) return inv_tv<T, MODE, 1>(tb, fused, a, s);
-  if (fused && a.var == 2) return inv_tv<T, MODE, 2>(tb, fused, a, s);
-  if (fused && a.var == 3) return inv_tv<T, MODE, 3>(tb, fused, a, s);
+  const int v = !fused ? 0 : a.var >= 0 ? a.var : inv_auto<T, MODE>(inv_items<T, MODE, 3>(a));
+  if (v == 1) return inv_tv<T, MODE, 1>(tb, fused, a, s);
+  if (v == 2) return inv_tv<T, MODE, 2>(tb, fused, a, s);
+  if (v == 3) return inv_tv<T, MODE, 3>(tb, fused, a, s);
   return inv_tv<T, MODE, 0>(tb, fused, a, s);
 }
 
@@ -185,9 +205,13 @@ static int inv_rt_tv(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int
 template <int T, int MODE>
 static int inv_rt_t(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
                     const InvArgs& au, hipStream_t s) {
-  if (aq.var == 1) return inv_rt_tv<T, MODE, 1>(tb, aq, aj, nj, au, s);
-  if (aq.var == 2) return inv_rt_tv<T, MODE, 2>(tb, aq, aj, nj, au, s);
-  if (aq.var == 3) return inv_rt_tv<T, MODE, 3>(tb, aq, aj, nj, au, s);
+  const int v = aq.var >= 0 ? aq.var
+                            : inv_auto<T, MODE>(inv_items<T, MODE, 3>(aq) +
+                                                nj * inv_items<T, MODE, 3>(aj[0]) +
+                                                inv_items<T, MODE, 3>(au));
+  if (v == 1) return inv_rt_tv<T, MODE, 1>(tb, aq, aj, nj, au, s);
+  if (v == 2) return inv_rt_tv<T, MODE, 2>(tb, aq, aj, nj, au, s);
+  if (v == 3) return inv_rt_tv<T, MODE, 3>(tb, aq, aj, nj, au, s);
   return inv_rt_tv<T, MODE, 0>(tb, aq, aj, nj, au, s);
 }
 
@@ -223,12 +247,27 @@ static int fwd_tv(const Tables& tb, bool fused, const FwdArgs& a, void* scratch,
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
+// The tile variant of a fused direct transform on a plan that was not tuned,
+// from the blocks of V = 3 (half the fields, 512 threads): as long as those fit
+// the CUs (FP32: two per CU), a block's own time counts and the smallest block
+// is the fastest; above, 512 threads on all fields, but 256 in FP64 at T42,
+// where two such blocks share a CU's LDS and a wide one does not fit twice.
+// Round trip directs in us, V = 0, 2, 3: T42 L20 BF16X3, 1 member 15.1, 9.0,
+// 5.3; 16 members 15.4, 13.5, 16.2; FP64, 1 member 11.4, 9.6, 9.9; 16 members
+// 32.4, 41.0, 42.6; T63 L20 BF16X3, 16 members 66.9, 42.7, 43.4.
+template <int T, int MODE>
+static int fwd_auto(long nblk3) {
+  if (nblk3 <= (MODE == MODE_F64 ? 256 : 512)) return 3;
+  return (MODE == MODE_F64 && T == 42) ? 0 : 2;
+}
+
 template <int T, int MODE>
 static int fwd_t(const Tables& tb, bool fused, const FwdArgs& a, void* scratch, size_t sbytes,
                  hipStream_t s) {
-  if (fused && a.var == 1) return fwd_tv<T, MODE, 1>(tb, fused, a, scratch, sbytes, s);
-  if (fused && a.var == 2) return fwd_tv<T, MODE, 2>(tb, fused, a, scratch, sbytes, s);
-  if (fused && a.var == 3) return fwd_tv<T, MODE, 3>(tb, fused, a, scratch, sbytes, s);
+  const int v = !fused ? 0 : a.var >= 0 ? a.var : fwd_auto<T, MODE>(fwd_items<T, MODE, 3>(a));
+  if (v == 1) return fwd_tv<T, MODE, 1>(tb, fused, a, scratch, sbytes, s);
+  if (v == 2) return fwd_tv<T, MODE, 2>(tb, fused, a, scratch, sbytes, s);
+  if (v == 3) return fwd_tv<T, MODE, 3>(tb, fused, a, scratch, sbytes, s);
   return fwd_tv<T, MODE, 0>(tb, fused, a, scratch, sbytes, s);
 }
 

@@ -230,3 +230,32 @@ def test_lwr_edges(oracle, gpu, nlev, ncol, fp64):
     assert rel(olr.double().cpu().numpy(), wo) < tol[1]
     assert rel(fu.double().cpu().numpy(), wu.T) < tol[1]
     assert rel(fd.double().cpu().numpy(), wd.T) < tol[1]
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 5, 1), (21, 20, 40), (42, 10, 2), (42, 10, 5),
+                                            (63, 7, 1), (63, 5, 4), (127, 6, 1), (127, 5, 3)])
+@pytest.mark.parametrize("mode", ["f64", "f32", "bf16x3"])
+def test_untuned_tiles(oracle, gpu, ntru, nlev, nmem, mode):
+    """a plan that was not tuned chooses its tiles by the size of the call:
+    below and above the sizes where the choice changes, against the oracle.
+    The tolerances of the round trips at the default tiles: sums of <= 192
+    terms and three FFT passes leave about 1e-15 and 2e-7 relative in the
+    norm; 1e-12 and 1e-6."""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.synth import ensemble
+
+    print(f"untuned T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    sp = ensemble(ntru, nlev, nmem, cfg=1)
+    p = sht.Plan(ntru)
+    x, gp, y = p.alloc_roundtrip(nmem, nlev, mode)
+    x.copy_(torch.from_numpy(sp).to(x.dtype))
+    p.roundtrip(mode, x, gp, y, nlev)
+    torch.cuda.synchronize()
+    tol = 1e-12 if mode == "f64" else 1e-6
+    for k in (0, nmem - 1):
+        want_g, want_s = oracle.roundtrip(ntru, nlev, x[k].double().cpu().numpy())
+        assert rel(gp[k].double().cpu().numpy(), want_g) < tol
+        assert rel(y[k].double().cpu().numpy(), want_s) < tol
+    p.close()
