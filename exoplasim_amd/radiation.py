@@ -7,9 +7,9 @@
   its heating-rate error.
 * ``LwEmulator``: a 43 -> 256 -> 256 -> 256 -> 21 GELU MLP whose forward and
   backward passes run on this package's own BF16 MFMA kernels
-  (exo_mlp_forward / exo_mlp_backward_dx / exo_mlp_backward_dw), registered
-  as torch operators (exoplasim_amd::lw_mlp_forward / lw_mlp_backward) with
-  autograd; FP32 master weights, Adam.  Inputs per column: 20-level
+  (exo_mlp_train_forward / exo_mlp_train_backward), registered as torch
+  operators (exoplasim_amd::lw_mlp_forward / lw_mlp_backward) with autograd;
+  FP32 master weights, Adam.  Inputs per column: 20-level
   temperature, 20-level specific humidity, surface temperature, surface
   pressure, CO2; outputs: 20-level heating rates (K/day) and OLR (W/m2).
 
@@ -20,7 +20,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from ctypes import POINTER, c_double, c_int, c_void_p
+from ctypes import POINTER, c_double, c_int, c_long, c_void_p
 
 import numpy as np
 
@@ -61,17 +61,14 @@ def _proto():
         L.exo_lwr.argtypes = [POINTER(_Params), c_int, c_int, POINTER(_Cols), POINTER(_Out),
                               c_void_p]
         vp, fp = c_void_p, c_void_p
-        L.exo_mlp_forward.restype = c_int
-        L.exo_mlp_forward.argtypes = [vp, vp, fp, c_int, c_int, c_int, c_int, c_int, fp, vp, fp,
-                                      vp]
-        L.exo_mlp_backward_dx.restype = c_int
-        L.exo_mlp_backward_dx.argtypes = [vp, vp, fp, c_int, c_int, c_int, c_int, vp, fp, vp]
-        L.exo_mlp_backward_dw.restype = c_int
-        L.exo_mlp_backward_dw.argtypes = [vp, vp, fp, c_int, c_int, c_int, c_int, fp, fp, fp, vp]
+        L.exo_mlp_train_work.restype = c_long
+        L.exo_mlp_train_work.argtypes = [c_int, c_int]
+        L.exo_mlp_train_forward.restype = c_int
+        L.exo_mlp_train_forward.argtypes = [c_int, fp, vp, vp, vp, vp, vp, fp, vp, vp]
+        L.exo_mlp_train_backward.restype = c_int
+        L.exo_mlp_train_backward.argtypes = [c_int, fp, vp, vp, vp, vp, vp, vp, vp, vp]
         L.exo_mlp_cast_weights.restype = c_int
         L.exo_mlp_cast_weights.argtypes = [fp, c_int, c_int, c_int, c_int, vp, vp, vp]
-        L.exo_mlp_cast_rows.restype = c_int
-        L.exo_mlp_cast_rows.argtypes = [fp, c_int, c_int, c_int, vp, vp]
         L.exo_lw_emulate.restype = c_int
         L.exo_lw_emulate.argtypes = [POINTER(_Net), c_int, fp, fp, fp, fp, fp, fp, vp]
         L.exo_lw_emulate_guarded.restype = c_int
@@ -178,25 +175,6 @@ def features(cols: dict, nlev: int = 20):
     return torch.cat(f, dim=0).t().contiguous()
 
 
-class _MLP:
-    """Buffers and raw kernel calls of one batch size."""
-
-    def __init__(self, M: int, device):
-        import torch
-
-        bf = torch.bfloat16
-        self.M = M
-        self.x0 = torch.empty((M, KIN), dtype=bf, device=device)
-        self.z = [torch.empty((M, NHID), dtype=torch.float32, device=device) for _ in range(3)]
-        self.h = [torch.empty((M, NHID), dtype=bf, device=device) for _ in range(3)]
-        self.y = torch.empty((M, NOUTP), dtype=torch.float32, device=device)
-        self.dz = [torch.empty((M, NHID), dtype=bf, device=device) for _ in range(3)]
-        self.dz32 = [torch.empty((M, NHID), dtype=torch.float32, device=device) for _ in range(3)]
-        self.dy = torch.empty((M, NOUTP), dtype=bf, device=device)
-        self.nsplit = max(1, min(64, M // 256))
-        self.part = torch.empty(self.nsplit * NHID * NHID, dtype=torch.float32, device=device)
-
-
 def _ptr(t):
     return t.data_ptr()
 
@@ -209,18 +187,10 @@ def _register_ops():
     ``(x, W1, b1, ..., W4, b4) -> y`` is differentiable in the parameters."""
     import torch
 
-    def _weights(params, dev):
-        L, s = _proto(), _stream()
-        wb, wtb = [], []
-        for li, ((nin, nout), (K, N)) in enumerate(zip(LAYERS, PADDED)):
-            w = params[li].contiguous()
-            W = torch.empty((N, K), dtype=torch.bfloat16, device=dev)
-            Wt = torch.empty((K, N), dtype=torch.bfloat16, device=dev)
-            _chk(L.exo_mlp_cast_weights(_ptr(w), nout, nin, N, K, _ptr(W), _ptr(Wt), s),
-                 "cast_weights")
-            wb.append(W)
-            wtb.append(Wt)
-        return wb, wtb
+    f32, bf16 = torch.float32, torch.bfloat16
+
+    def _ptrs(ts):
+        return (c_void_p * len(ts))(*[t.data_ptr() for t in ts])
 
     t8 = "(" + ", ".join(["Tensor"] * 8) + ")"
 
@@ -232,22 +202,18 @@ def _register_ops():
         inputs x0, the pre-activations z1..z3 (fp32) and the bf16 hidden
         layers h1..h3"""
         L, s = _proto(), _stream()
-        bias = (b1, b2, b3, b4)
-        M = x.shape[0]
-        buf = _MLP(M, x.device)
-        wb, _ = _weights((w1, w2, w3, w4), x.device)
+        M, dev = x.shape[0], x.device
+        ws = [w.contiguous() for w in (w1, w2, w3, w4)]
         xf = x.float().contiguous()
-        _chk(L.exo_mlp_cast_rows(_ptr(xf), M, NIN, KIN, _ptr(buf.x0), s), "cast_rows")
-        inp = buf.x0
-        for li in range(3):
-            K, N = PADDED[li]
-            _chk(L.exo_mlp_forward(_ptr(inp), _ptr(wb[li]), _ptr(bias[li]), M, K, N,
-                                   LAYERS[li][1], 1, _ptr(buf.z[li]), _ptr(buf.h[li]), None,
-                                   s), "mlp_forward")
-            inp = buf.h[li]
-        _chk(L.exo_mlp_forward(_ptr(inp), _ptr(wb[3]), _ptr(b4), M, NHID, NOUTP, NOUT, 0, None,
-                               None, _ptr(buf.y), s), "mlp_forward")
-        return (buf.y[:, :NOUT].clone(), buf.x0, *buf.z, *buf.h)
+        y = torch.empty((M, NOUT), dtype=f32, device=dev)
+        x0 = torch.empty((M, KIN), dtype=bf16, device=dev)
+        z = [torch.empty((M, NHID), dtype=f32, device=dev) for _ in range(3)]
+        h = [torch.empty((M, NHID), dtype=bf16, device=dev) for _ in range(3)]
+        work = torch.empty(L.exo_mlp_train_work(M, 0), dtype=torch.uint8, device=dev)
+        _chk(L.exo_mlp_train_forward(M, _ptr(xf), _ptrs(ws), _ptrs((b1, b2, b3, b4)), _ptr(x0),
+                                     _ptrs(z), _ptrs(h), _ptr(y), _ptr(work), s),
+             "mlp_train_forward")
+        return (y, x0, *z, *h)
 
     @lw_mlp_forward.register_fake
     def _(x, w1, b1, w2, b2, w3, b3, w4, b4):
@@ -264,34 +230,16 @@ def _register_ops():
     def lw_mlp_backward(gy, x0, z1, z2, z3, h1, h2, h3, w1, w2, w3, w4):
         """gradients (dW1, db1, ..., dW4, db4) for the output gradient gy"""
         L, s = _proto(), _stream()
-        M = gy.shape[0]
-        dev = gy.device
-        buf = _MLP(M, dev)
-        z, h = (z1, z2, z3), (h1, h2, h3)
-        _, wtb = _weights((w1, w2, w3, w4), dev)
-        gy32 = torch.zeros((M, NOUTP), dtype=torch.float32, device=dev)
-        gy32[:, :NOUT] = gy
-        _chk(L.exo_mlp_cast_rows(_ptr(gy32), M, NOUTP, NOUTP, _ptr(buf.dy), s), "cast_rows")
-        grads = [None] * 8
-        dz, dz32 = buf.dy, gy32
-        for li in (3, 2, 1, 0):
-            K, N = PADDED[li]
-            nin, nout = LAYERS[li]
-            xin = h[li - 1] if li > 0 else x0
-            dW = torch.empty((N, K), dtype=torch.float32, device=dev)
-            db = torch.empty(N, dtype=torch.float32, device=dev)
-            _chk(L.exo_mlp_backward_dw(_ptr(dz), _ptr(xin), _ptr(dz32), M, N, K, buf.nsplit,
-                                       _ptr(buf.part), _ptr(dW), _ptr(db), s),
-                 "mlp_backward_dw")
-            grads[2 * li] = dW[:nout, :nin].contiguous()
-            grads[2 * li + 1] = db[:nout].contiguous()
-            if li > 0:
-                Kp = PADDED[li - 1][1]
-                _chk(L.exo_mlp_backward_dx(_ptr(dz), _ptr(wtb[li]), _ptr(z[li - 1]), M, N, Kp,
-                                           LAYERS[li - 1][1], _ptr(buf.dz[li - 1]),
-                                           _ptr(buf.dz32[li - 1]), s), "mlp_backward_dx")
-                dz, dz32 = buf.dz[li - 1], buf.dz32[li - 1]
-        return tuple(grads)
+        M, dev = gy.shape[0], gy.device
+        ws = [w.contiguous() for w in (w1, w2, w3, w4)]
+        g = gy.float().contiguous()
+        dw = [torch.empty((nout, nin), dtype=f32, device=dev) for nin, nout in LAYERS]
+        db = [torch.empty(nout, dtype=f32, device=dev) for _, nout in LAYERS]
+        work = torch.empty(L.exo_mlp_train_work(M, 1), dtype=torch.uint8, device=dev)
+        _chk(L.exo_mlp_train_backward(M, _ptr(g), _ptr(x0), _ptrs((z1, z2, z3)),
+                                      _ptrs((h1, h2, h3)), _ptrs(ws), _ptrs(dw), _ptrs(db),
+                                      _ptr(work), s), "mlp_train_backward")
+        return (dw[0], db[0], dw[1], db[1], dw[2], db[2], dw[3], db[3])
 
     @lw_mlp_backward.register_fake
     def _(gy, x0, z1, z2, z3, h1, h2, h3, w1, w2, w3, w4):
@@ -441,7 +389,7 @@ class LwEmulator:
         return heat, olr, n
 
     def predict_layers(self, cols):
-        """the same through the per-layer training kernels (features in torch)"""
+        """the same through the training kernels (features in torch)"""
         import torch
 
         with torch.no_grad():

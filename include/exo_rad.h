@@ -68,6 +68,22 @@ int exo_mlp_cast_weights(const float *w, int nout, int nin, int N, int K, void *
 /* fp32 rows src[M][nin] -> zero-padded bf16 dst[M][K] */
 int exo_mlp_cast_rows(const float *src, int M, int nin, int K, void *dst, void *stream);
 
+/* The training passes of the whole network (layers 43 -> 256 -> 256 -> 256 ->
+ * 21).  w[l] and b[l] are the fp32 master weights and biases, unpadded.
+ * forward: y[M][21] of the inputs x[M][43], and what the backward pass reads:
+ * x0[M][64] (the inputs in bf16, zero padded), z[l][M][256] (fp32
+ * pre-activations) and h[l][M][256] (bf16 activations) of layers l = 0..2.
+ * backward: the gradients dw[l] (as w[l]) and db[l] for the output gradient
+ * gy[M][21], M >= 1.  work holds exo_mlp_train_work(M, backward) bytes and
+ * is free again once the call's kernels have run. */
+long exo_mlp_train_work(int M, int backward);
+int exo_mlp_train_forward(int M, const float *x, const float *const *w, const float *const *b,
+                          void *x0, float *const *z, void *const *h, float *y, void *work,
+                          void *stream);
+int exo_mlp_train_backward(int M, const float *gy, const void *x0, const float *const *z,
+                           const void *const *h, const float *const *w, float *const *dw,
+                           float *const *db, void *work, void *stream);
+
 /* A trained emulator for inference: bf16 weights W1[256][64], W2[256][256],
  * W3[256][256], W4[32][256] (zero padded, as exo_mlp_cast_weights writes
  * them), fp32 biases, and the output normalisation ymean/ystd (21 values).

@@ -259,3 +259,38 @@ def test_untuned_tiles(oracle, gpu, ntru, nlev, nmem, mode):
         assert rel(gp[k].double().cpu().numpy(), want_g) < tol
         assert rel(y[k].double().cpu().numpy(), want_s) < tol
     p.close()
+
+
+@pytest.mark.parametrize("nbatch", [1, 15, 17, 256, 321, 1000, 4096, 4097, 4129])
+def test_mlp_training_edges(gpu, nbatch):
+    """the emulator's output and all gradients at ragged rows of a block, one
+    and several batch splits, and both sides of the change from 16 to 32 rows
+    per block, against the FP64 oracle with the kernels' bf16 roundings.
+    What is left is FP32 accumulation and the bf16 values it flips to their
+    neighbour: at most 2^-8 of a value, below 2^-9 = 2e-3 in the norm."""
+    import sys as _sys
+
+    _sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(__file__)), "oracle"))
+    import mlp_oracle as MO
+    import torch
+
+    from exoplasim_amd.radiation import LwEmulator
+
+    print(f"mlp training {nbatch}", flush=True)
+    em = LwEmulator(seed=3)
+    g = torch.Generator(device="cpu").manual_seed(nbatch)
+    with torch.no_grad():
+        for b in em.params[1::2]:
+            b.copy_(0.1 * torch.randn(b.shape, generator=g))
+    x = torch.randn(nbatch, 43, generator=g)
+    gy = torch.randn(nbatch, 21, generator=g)
+    y = em.raw(x.cuda())
+    y.backward(gy.cuda())
+    torch.cuda.synchronize()
+    ps = [p.detach().double().cpu().numpy() for p in em.params]
+    want, saved = MO.forward(x.double().numpy(), ps)
+    grads = MO.backward(gy.double().numpy(), ps, saved)
+    assert rel(y.detach().double().cpu().numpy(), want) < 2e-3
+    for i, (p, w) in enumerate(zip(em.params, grads)):
+        assert p.grad.shape == p.shape
+        assert rel(p.grad.double().cpu().numpy(), w) < 2e-3, i
