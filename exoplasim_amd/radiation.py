@@ -249,10 +249,15 @@ def _register_ops():
         return tuple(out)
 
     def setup_context(ctx, inputs, output):
+        # no zero gradients of the seven saved outputs, which autograd would
+        # otherwise allocate and fill on every backward pass
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(*output[1:], inputs[1], inputs[3], inputs[5], inputs[7])
 
     def backward(ctx, gy, *unused):
         x0, z1, z2, z3, h1, h2, h3, w1, w2, w3, w4 = ctx.saved_tensors
+        if gy is None:  # only saved outputs were used: no gradient flows through them
+            gy = x0.new_zeros((x0.shape[0], NOUT), dtype=f32)
         g = torch.ops.exoplasim_amd.lw_mlp_backward(gy.contiguous(), x0, z1, z2, z3, h1, h2, h3,
                                                     w1, w2, w3, w4)
         return (None, *g)

@@ -294,3 +294,17 @@ def test_mlp_training_edges(gpu, nbatch):
     for i, (p, w) in enumerate(zip(em.params, grads)):
         assert p.grad.shape == p.shape
         assert rel(p.grad.double().cpu().numpy(), w) < 2e-3, i
+
+
+def test_mlp_saved_outputs_have_no_gradient(gpu):
+    """a loss on a saved output alone reaches the backward pass without an
+    output gradient: every parameter's gradient is zero"""
+    import torch
+
+    from exoplasim_amd.radiation import LwEmulator
+
+    em = LwEmulator(seed=3)
+    em.raw(torch.randn(20, 43, device="cuda"))
+    out = torch.ops.exoplasim_amd.lw_mlp_forward(torch.randn(20, 43, device="cuda"), *em.params)
+    out[2].sum().backward()
+    assert all(p.grad is not None and not bool(p.grad.any()) for p in em.params)
