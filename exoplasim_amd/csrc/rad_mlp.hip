@@ -216,113 +216,100 @@ inline unsigned nb(long n, int b) { return (unsigned)((n + b - 1) / b); }
 
 // ---------------------------------------------------------------------------
 // fused inference: features -> 4 layers -> heating rates and OLR, one block
-// of 8 waves per 32 columns, activations in LDS, weights streamed from L2.
+// of 8 waves per MT columns, activations in LDS, weights streamed from L2.
 // Each layer is computed transposed, C^T[n][m] = W[n][:] . H[m][:], so that a
 // lane's four accumulator values (consecutive n of one column m) go to LDS
 // as one 8-byte store of the row-major activations.
+//
+// A block is a chain of dependent layers, bound in turn by the latency of its
+// inputs and weights and by the vector work of features and GELUs (about 2000
+// vector instructions per wave at MT = 32, some 8 of its 10 us).
+// MT = 16 halves that work per block, and is taken while it leaves no CU more
+// than one block (4096 columns: 7.4 us against 10.9); above, MT = 32 halves the
+// weight traffic (8192 columns 10.0 against 12.5).
 // ---------------------------------------------------------------------------
-constexpr int EM_NLEV = 20, EM_KIN = 64, EM_NH = 256, EM_NOUT = 21, EM_NOUTP = 32;
+constexpr int EM_NLEV = 20, EM_KIN = 64, EM_NH = 256, EM_NOUT = 21;
 constexpr int EM_NIN = 2 * EM_NLEV + 3;  // features: T, ln q, T_s, ln p_s, ln CO2
-constexpr int EM_MT = 32;             // columns per block
 constexpr int EM_NT = 512;            // threads per block (8 waves)
 constexpr int EM_LDH = EM_NH + 8;     // padded LDS row (bf16) of a hidden layer
 constexpr int EM_LDX = EM_KIN + 8;
 
-// one hidden layer: Hout[32][256] = gelu(Hin[32][K] W^T + b); wave w owns
-// output features [32w, 32w + 32)
-template <int K, int LDI>
-__device__ __forceinline__ void em_hidden(const uint16_t* hin, const V8 (&wa)[K / 32][2],
-                                          const float* b, uint16_t* hout) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int q = lane >> 4, c = lane & 15;
-  const int n0 = wv * 32;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < K / 32; ++ks) {
-    V8 h[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      h[j].q = *(const uint4*)(hin + (j * 16 + c) * LDI + ks * 32 + q * 8);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma(wa[ks][i], h[j], acc[i][j]);
-  }
+// bias and GELU of a hidden layer: hout[MT][256], wave w the features [32w, 32w + 32)
+template <int MT>
+__device__ __forceinline__ void em_act(const f32x4 (&acc)[2][MT / 16], const float4 (&bias)[2],
+                                       uint16_t* hout) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int nb = n0 + i * 16 + 4 * q;  // this lane's 4 consecutive features
-    const float4 bn = *(const float4*)(b + nb);
+    const float4 bn = bias[i];  // this lane's 4 consecutive features
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int m = j * 16 + c;
-      uint2 pk;
-      pk.x = (uint32_t)f2bf(gelu(acc[i][j][0] + bn.x)) |
-             ((uint32_t)f2bf(gelu(acc[i][j][1] + bn.y)) << 16);
-      pk.y = (uint32_t)f2bf(gelu(acc[i][j][2] + bn.z)) |
-             ((uint32_t)f2bf(gelu(acc[i][j][3] + bn.w)) << 16);
-      *(uint2*)(hout + m * EM_LDH + nb) = pk;
+    for (int j = 0; j < MT / 16; ++j) {
+      const f32x4 z = acc[i][j];
+      const uint2 pk = {f2bf2(gelu(z[0] + bn.x), gelu(z[1] + bn.y)),
+                        f2bf2(gelu(z[2] + bn.z), gelu(z[3] + bn.w))};
+      *(uint2*)(hout + (j * 16 + c) * EM_LDH + wv * 32 + i * 16 + 4 * q) = pk;
     }
   }
 }
 
 // GUARD: also flag (outside[col] = 1) every column with a feature outside
-// [flo, fhi] (or not a number): the columns the network was not trained on
-template <bool GUARD>
-__global__ __launch_bounds__(EM_NT) void k_emulate(exo_lw_net net, int ncol, const float* dt,
-                                                   const float* dq, const float* dp,
-                                                   const float* co2, float* heat, float* olr,
-                                                   const float* flo, const float* fhi,
-                                                   int* outside) {
-  __shared__ __align__(16) uint16_t sx[EM_MT * EM_LDX];
-  __shared__ __align__(16) uint16_t sh0[EM_MT * EM_LDH];
-  __shared__ __align__(16) uint16_t sh1[EM_MT * EM_LDH];
-  __shared__ int sflag[EM_MT];
+// [flo, fhi] (or not a number): the columns the network was not trained on.
+// PACKED: net.w in fragment order, else row-major.
+template <int MT, bool GUARD, bool PACKED>
+__global__ __launch_bounds__(EM_NT, 2) void k_emulate(exo_lw_net net, int ncol, const float* dt,
+                                                      const float* dq, const float* dp,
+                                                      const float* co2, float* heat, float* olr,
+                                                      const float* flo, const float* fhi,
+                                                      int* outside) {
+  __shared__ __align__(16) uint16_t sx[MT * EM_LDX];
+  __shared__ __align__(16) uint16_t sh0[MT * EM_LDH];
+  __shared__ __align__(16) uint16_t sh1[MT * EM_LDH];
+  __shared__ int sflag[MT];
   const int tid = threadIdx.x;
-  const int col0 = blockIdx.x * EM_MT;
+  const int col0 = blockIdx.x * MT;
   if (GUARD) {
-    if (tid < EM_MT) sflag[tid] = 0;
+    if (tid < MT) sflag[tid] = 0;
     __syncthreads();
   }
-  // every layer's weights are on their way while the features are computed
-  // (one block per CU at a model step's 8192 columns: nothing else would
-  // hide a later request's latency)
-  const int lane = tid & 63, wv = tid >> 6;
-  const int q = lane >> 4, c = lane & 15;
-  const int nt = wv & 1, mt = (wv >> 1) & 1;
-  V8 w1[EM_KIN / 32][2], w2[EM_NH / 32][2], w3[EM_NH / 32][2], w4[EM_NH / 32];
-  em_load<EM_KIN>((const uint16_t*)net.w[0], w1);
-  em_load<EM_NH>((const uint16_t*)net.w[1], w2);
-  em_load<EM_NH>((const uint16_t*)net.w[2], w3);
-  if (wv < 4) {
-    const uint16_t* W4 = (const uint16_t*)net.w[3] + (long)(nt * 16 + c) * EM_NH + q * 8;
-#pragma unroll
-    for (int k = 0; k < EM_NH / 32; ++k) w4[k].q = *(const uint4*)(W4 + 32 * k);
-  }
   // features (exoplasim_amd.radiation.features), column index fastest: all
-  // of a thread's inputs are requested before any is used
-  constexpr int NIT = EM_MT * EM_KIN / EM_NT;
-  static_assert(EM_MT * EM_KIN % EM_NT == 0, "feature items per thread");
+  // of a thread's inputs are requested first, without a branch, so that the
+  // wait for them does not include the weights behind them
+  constexpr int NIT = MT * EM_KIN / EM_NT;
+  static_assert(MT * EM_KIN % EM_NT == 0, "feature items per thread");
   float raw[NIT];
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int idx = tid + EM_NT * it;
-    const int m = idx % EM_MT, f = idx / EM_MT;
+    const int m = idx % MT, f = idx / MT;
     const int col = min(col0 + m, ncol - 1);
     const float* src = (f < EM_NLEV)           ? dt + (long)f * ncol
                        : (f < 2 * EM_NLEV)     ? dq + (long)(f - EM_NLEV) * ncol
                        : (f == 2 * EM_NLEV)    ? dt + (long)EM_NLEV * ncol
                        : (f == 2 * EM_NLEV + 1) ? dp
                                                 : co2;
-    raw[it] = (f < EM_NIN) ? src[col] : 0.f;
+    raw[it] = src[col];  // past the features: CO2, not used
   }
+  __builtin_amdgcn_sched_barrier(0);
+  // the first two layers' weights and biases are on their way while the
+  // features are computed, a later layer's during the GELUs of one before
+  const int lane = tid & 63, wv = tid >> 6;
+  const int q = lane >> 4, c = lane & 15;
+  V8 w1[2][EM_KIN / 32], w2[2][EM_NH / 32], w3[2][EM_NH / 32], w4[EM_NH / 32];
+  float4 bias[3][2];
+  auto load_w = [&](int l, auto& w) {
+    constexpr int K = 32 * (sizeof(w[0]) / sizeof(V8));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      load_tile<K, PACKED>((const uint16_t*)net.w[l], 2 * wv + i, w[i]);
+      bias[l][i] = *(const float4*)(net.b[l] + wv * 32 + i * 16 + 4 * q);
+    }
+  };
+  load_w(0, w1);
+  load_w(1, w2);
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
     const int idx = tid + EM_NT * it;
-    const int m = idx % EM_MT, f = idx / EM_MT;
+    const int m = idx % MT, f = idx / MT;
     const float x = raw[it];
     float v = 0.f;
     if (f < EM_NLEV)
@@ -339,36 +326,88 @@ __global__ __launch_bounds__(EM_NT) void k_emulate(exo_lw_net net, int ncol, con
     if (GUARD && f < EM_NIN && !(v >= flo[f] && v <= fhi[f])) atomicOr(&sflag[m], 1);
   }
   __syncthreads();
-  if (GUARD && tid < EM_MT && col0 + tid < ncol) outside[col0 + tid] = sflag[tid];
-  em_hidden<EM_KIN, EM_LDX>(sx, w1, net.b[0], sh0);
+  if (GUARD && tid < MT && col0 + tid < ncol) outside[col0 + tid] = sflag[tid];
+  f32x4 acc[2][MT / 16];
+  layer<EM_KIN, EM_LDX, MT>(sx, w1, acc);
+  load_w(2, w3);
+  __builtin_amdgcn_sched_barrier(0);
+  em_act<MT>(acc, bias[0], sh0);
   __syncthreads();
-  em_hidden<EM_NH, EM_LDH>(sh0, w2, net.b[1], sh1);
+  layer<EM_NH, EM_LDH, MT>(sh0, w2, acc);
+  // output layer, transposed: waves 0 .. MT / 8 - 1 take feature tile wv & 1
+  // (n) and column tile wv >> 1 (m)
+  const int nt = wv & 1, mt = wv >> 1;
+  const int col = col0 + mt * 16 + c;
+  float b4[4], ys[4], ym[4], psurf = 0.f;
+  if (mt < MT / 16) {
+    load_tile<EM_NH, PACKED>((const uint16_t*)net.w[3], nt, w4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = min(nt * 16 + 4 * q + r, EM_NOUT - 1);
+      b4[r] = net.b[3][n], ys[r] = net.ystd[n], ym[r] = net.ymean[n];
+    }
+    psurf = dp[min(col, ncol - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  em_act<MT>(acc, bias[1], sh1);
   __syncthreads();
-  em_hidden<EM_NH, EM_LDH>(sh1, w3, net.b[2], sh0);
+  layer<EM_NH, EM_LDH, MT>(sh1, w3, acc);
+  em_act<MT>(acc, bias[2], sh0);
   __syncthreads();
-  // output layer, transposed: waves 0..3 take feature tile wv&1 (n) and
-  // column tile wv>>1 (m)
-  if (wv >= 4) return;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (mt >= MT / 16) return;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < EM_NH / 32; ++k) {
     V8 h;
     h.q = *(const uint4*)(sh0 + (mt * 16 + c) * EM_LDH + 32 * k + q * 8);
-    acc = mfma(w4[k], h, acc);
+    o = mfma(w4[k], h, o);
   }
-  const int col = col0 + mt * 16 + c;
   if (col >= ncol) return;
-  const float ps = dp[col] / 1e5f;
+  const float ps = psurf / 1e5f;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int n = nt * 16 + 4 * q + r;
     if (n >= EM_NOUT) continue;
-    const float y = (acc[r] + net.b[3][n]) * net.ystd[n] + net.ymean[n];
+    const float y = (o[r] + b4[r]) * ys[r] + ym[r];
     if (n < EM_NLEV)
       heat[(long)n * ncol + col] = y / ps;
     else
       olr[col] = y;
   }
+}
+
+template <bool PACKED>
+int emulate(const exo_lw_net* net, const float* flo, const float* fhi, int ncol, const float* dt,
+            const float* dq, const float* dp, const float* co2, float* heat, float* olr,
+            int* outside, hipStream_t s) {
+  if (!net || ncol < 0 || net->nlev != EM_NLEV) return EXO_RAD_ERR_ARG;
+  if (ncol == 0) return EXO_RAD_OK;
+  if (!dt || !dq || !dp || !co2 || !heat || !olr || !net->ymean || !net->ystd)
+    return EXO_RAD_ERR_ARG;
+  for (int l = 0; l < 4; ++l)
+    if (!net->w[l] || !net->b[l]) return EXO_RAD_ERR_ARG;
+  auto launch = [&](auto kern, int mt) {
+    kern<<<nb(ncol, mt), EM_NT, 0, s>>>(*net, ncol, dt, dq, dp, co2, heat, olr, flo, fhi, outside);
+  };
+  const bool small = ncol <= 16 * 256;
+  if (outside && small)
+    launch(k_emulate<16, true, PACKED>, 16);
+  else if (outside)
+    launch(k_emulate<32, true, PACKED>, 32);
+  else if (small)
+    launch(k_emulate<16, false, PACKED>, 16);
+  else
+    launch(k_emulate<32, false, PACKED>, 32);
+  return hipGetLastError() == hipSuccess ? EXO_RAD_OK : EXO_RAD_ERR_HIP;
+}
+
+// FP32 master W[nout][nin] -> padded bf16 W[N][K] in fragment order
+__global__ void k_cast_frag(const float* w, int nout, int nin, int N, int K, uint16_t* out) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= N * K) return;
+  int n, k;
+  frag_nk(e, K, n, k);
+  out[e] = (n < nout && k < nin) ? f2bf(w[(long)n * nin + k]) : (uint16_t)0;
 }
 
 }  // namespace
@@ -428,30 +467,34 @@ extern "C" int exo_mlp_cast_weights(const float* w, int nout, int nin, int N, in
 extern "C" int exo_lw_emulate(const exo_lw_net* net, int ncol, const float* dt, const float* dq,
                               const float* dp, const float* dqco2, float* heat, float* olr,
                               void* stream) {
-  if (!net || ncol < 0 || net->nlev != EM_NLEV) return EXO_RAD_ERR_ARG;
-  if (ncol == 0) return EXO_RAD_OK;
-  if (!dt || !dq || !dp || !dqco2 || !heat || !olr || !net->ymean || !net->ystd)
-    return EXO_RAD_ERR_ARG;
-  for (int l = 0; l < 4; ++l)
-    if (!net->w[l] || !net->b[l]) return EXO_RAD_ERR_ARG;
-  k_emulate<false><<<nb(ncol, EM_MT), EM_NT, 0, (hipStream_t)stream>>>(
-      *net, ncol, dt, dq, dp, dqco2, heat, olr, nullptr, nullptr, nullptr);
-  return hipGetLastError() == hipSuccess ? EXO_RAD_OK : EXO_RAD_ERR_HIP;
+  return emulate<false>(net, nullptr, nullptr, ncol, dt, dq, dp, dqco2, heat, olr, nullptr,
+                        (hipStream_t)stream);
 }
 
 extern "C" int exo_lw_emulate_guarded(const exo_lw_net* net, const float* flo, const float* fhi,
                                       int ncol, const float* dt, const float* dq,
                                       const float* dp, const float* dqco2, float* heat,
                                       float* olr, int* outside, void* stream) {
-  if (!net || ncol < 0 || net->nlev != EM_NLEV) return EXO_RAD_ERR_ARG;
-  if (ncol == 0) return EXO_RAD_OK;
-  if (!dt || !dq || !dp || !dqco2 || !heat || !olr || !net->ymean || !net->ystd || !flo ||
-      !fhi || !outside)
+  if (ncol > 0 && (!flo || !fhi || !outside)) return EXO_RAD_ERR_ARG;
+  return emulate<false>(net, flo, fhi, ncol, dt, dq, dp, dqco2, heat, olr, outside,
+                        (hipStream_t)stream);
+}
+
+extern "C" int exo_lw_emulate_packed(const exo_lw_net* net, const float* flo, const float* fhi,
+                                     int ncol, const float* dt, const float* dq, const float* dp,
+                                     const float* dqco2, float* heat, float* olr, int* outside,
+                                     void* stream) {
+  if (outside && (!flo || !fhi)) return EXO_RAD_ERR_ARG;
+  return emulate<true>(net, flo, fhi, ncol, dt, dq, dp, dqco2, heat, olr, outside,
+                       (hipStream_t)stream);
+}
+
+extern "C" int exo_mlp_pack_weights(const float* w, int nout, int nin, int N, int K, void* packed,
+                                    void* stream) {
+  if (!w || !packed || nout > N || nin > K || N < 16 || N % 16 || K < 32 || K % 32)
     return EXO_RAD_ERR_ARG;
-  for (int l = 0; l < 4; ++l)
-    if (!net->w[l] || !net->b[l]) return EXO_RAD_ERR_ARG;
-  k_emulate<true><<<nb(ncol, EM_MT), EM_NT, 0, (hipStream_t)stream>>>(
-      *net, ncol, dt, dq, dp, dqco2, heat, olr, flo, fhi, outside);
+  k_cast_frag<<<nb((long)N * K, 256), 256, 0, (hipStream_t)stream>>>(w, nout, nin, N, K,
+                                                                     (uint16_t*)packed);
   return hipGetLastError() == hipSuccess ? EXO_RAD_OK : EXO_RAD_ERR_HIP;
 }
 

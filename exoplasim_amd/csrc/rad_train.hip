@@ -17,7 +17,7 @@
 // dependences allow: 2 and 4 launches and one workspace, where a kernel per
 // layer and operand took 9 and 25 launches with the padded copies and fills
 // between them.  (4096 rows, forward and backward pass with loss: 658 us per
-// step with a kernel per layer, 376 us with these; kernel time 287 -> 57
+// step with a kernel per layer, 340-360 us with these; kernel time 287 -> 45
 // us.)  Every product and sum runs in the order of the per-layer kernels
 // (rad_mlp.hip); only the bias sums are regrouped.
 #include "../../include/exo_rad.h"
@@ -38,8 +38,8 @@ struct TrainW {
   const float* w[4];
 };
 
-// padded W[N][K] bf16 of layer l at element `at` of the concatenated layers;
-// with TR the transpose Wt[K][N] (same offsets)
+// padded bf16 weights of layer l in fragment order, the layers one after the
+// other: W[N][K], with TR its transpose Wt[K][N]
 template <bool TR>
 __global__ __launch_bounds__(256) void k_cast_net(TrainW p, uint16_t* out) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -48,31 +48,20 @@ __global__ __launch_bounds__(256) void k_cast_net(TrainW p, uint16_t* out) {
   const int e = i - (l == 0 ? TW1 : l == 1 ? TW2 : l == 2 ? TW3 : TW4);
   const int N = l == 3 ? TNOUTP : TNH, K = l == 0 ? TKIN : TNH;
   const int nout = l == 3 ? TNOUT : TNH, nin = l == 0 ? TNIN : TNH;
-  const int n = TR ? e % N : e / K, k = TR ? e / N : e % K;
+  int n, k;
+  if (TR)
+    frag_nk(e, N, k, n);
+  else
+    frag_nk(e, K, n, k);
   out[i] = (n < nout && k < nin) ? f2bf(p.w[l][n * nin + k]) : (uint16_t)0;
 }
 
-// the wave's 32 output features x MT rows of one layer, transposed:
-// acc[i][j] holds features 32 wv + 16 i + 4 q .. + 3 of row 16 j + c
-template <int K, int LDI, int MT>
-__device__ __forceinline__ void layer(const uint16_t* in, const V8 (&w)[K / 32][2],
-                                      f32x4 (&acc)[2][MT / 16]) {
-  const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < MT / 16; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < K / 32; ++ks) {
-    V8 h[MT / 16];
-#pragma unroll
-    for (int j = 0; j < MT / 16; ++j)
-      h[j].q = *(const uint4*)(in + (j * 16 + c) * LDI + ks * 32 + q * 8);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < MT / 16; ++j) acc[i][j] = mfma(w[ks][i], h[j], acc[i][j]);
-  }
+// the wave's two row tiles of one layer
+template <int K>
+__device__ __forceinline__ void load_pair(const uint16_t* W, V8 (&w)[2][K / 32]) {
+  const int wv = threadIdx.x >> 6;
+  load_tile<K>(W, 2 * wv, w[0]);
+  load_tile<K>(W, 2 * wv + 1, w[1]);
 }
 
 // sum over the 16 lanes of a row, in every lane (DPP row rotations)
@@ -85,8 +74,7 @@ __device__ __forceinline__ float row16_sum(float x) {
 }
 
 __device__ __forceinline__ uint2 pack4(const float (&v)[4]) {
-  return uint2{(uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16),
-               (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16)};
+  return uint2{f2bf2(v[0], v[1]), f2bf2(v[2], v[3])};
 }
 
 // the block's MT rows of 256 bf16 values, LDS -> global, whole lines
@@ -115,17 +103,35 @@ __global__ __launch_bounds__(TNT, 2) void k_train_fwd(TrainFwd a, int M) {
   __shared__ __align__(16) uint16_t sh[2][MT * TLD];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, q = lane >> 4, c = lane & 15;
   const int row0 = blockIdx.x * MT;
-  // the weights of the layers ahead are on their way while one is computed
-  V8 w1[TKIN / 32][2], w2[TNH / 32][2], w3[TNH / 32][2], w4[TNH / 32];
-  em_load<TKIN>(a.wb + TW1, w1);
-  em_load<TNH>(a.wb + TW2, w2);
+  // the inputs first, without a branch, so that the wait for them does not
+  // include the weights; the weights of the layers ahead are on their way while
+  // one is computed
+  float xv[MT / 16][2];
+#pragma unroll
+  for (int it = 0; it < MT / 16; ++it) {
+    const int e = tid + TNT * it, m = e >> 5, k = (e & 31) * 2;
+    const float* xr = a.x + (long)min(row0 + m, M - 1) * TNIN;
+    xv[it][0] = xr[min(k, TNIN - 1)];
+    xv[it][1] = xr[min(k + 1, TNIN - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  V8 w1[2][TKIN / 32], w2[2][TNH / 32], w3[2][TNH / 32], w4[TNH / 32];
+  load_pair<TKIN>(a.wb + TW1, w1);
+  load_pair<TNH>(a.wb + TW2, w2);
+  float bias[3][2][4];
+#pragma unroll
+  for (int l = 0; l < 3; ++l)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bias[l][i][r] = a.b[l][wv * 32 + i * 16 + 4 * q + r];
 #pragma unroll
   for (int it = 0; it < MT / 16; ++it) {
     const int e = tid + TNT * it, m = e >> 5, k = (e & 31) * 2;
     const long row = row0 + m;
-    const float v0 = row < M && k < TNIN ? a.x[row * TNIN + k] : 0.f;
-    const float v1 = row < M && k + 1 < TNIN ? a.x[row * TNIN + k + 1] : 0.f;
-    const uint32_t p = (uint32_t)f2bf(v0) | ((uint32_t)f2bf(v1) << 16);
+    const float v0 = row < M && k < TNIN ? xv[it][0] : 0.f;
+    const float v1 = row < M && k + 1 < TNIN ? xv[it][1] : 0.f;
+    const uint32_t p = f2bf2(v0, v1);
     *(uint32_t*)(sx + m * TLDX + k) = p;
     if (row < M) *(uint32_t*)(a.x0 + row * TKIN + k) = p;
   }
@@ -135,13 +141,11 @@ __global__ __launch_bounds__(TNT, 2) void k_train_fwd(TrainFwd a, int M) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int n = wv * 32 + i * 16 + 4 * q;
-      const float* b = a.b[l] + n;
-      const float4 bn = {b[0], b[1], b[2], b[3]};
 #pragma unroll
       for (int j = 0; j < MT / 16; ++j) {
         const int m = j * 16 + c;
-        const float z[4] = {acc[i][j][0] + bn.x, acc[i][j][1] + bn.y, acc[i][j][2] + bn.z,
-                            acc[i][j][3] + bn.w};
+        const float z[4] = {acc[i][j][0] + bias[l][i][0], acc[i][j][1] + bias[l][i][1],
+                            acc[i][j][2] + bias[l][i][2], acc[i][j][3] + bias[l][i][3]};
         const float g[4] = {gelu(z[0]), gelu(z[1]), gelu(z[2]), gelu(z[3])};
         *(uint2*)(hout + m * TLD + n) = pack4(g);
         if (row0 + m < M)
@@ -152,15 +156,11 @@ __global__ __launch_bounds__(TNT, 2) void k_train_fwd(TrainFwd a, int M) {
     rows_out<MT>(hout, a.h[l], row0, M);
   };
   layer<TKIN, TLDX, MT>(sx, w1, acc);
-  em_load<TNH>(a.wb + TW3, w3);
+  load_pair<TNH>(a.wb + TW3, w3);
   finish(0, sh[0]);
   layer<TNH, TLD, MT>(sh[0], w2, acc);
   const int nt = wv & 1, mt = wv >> 1;  // output layer: feature tile, row tile
-  if (mt < MT / 16) {
-    const uint16_t* wr = a.wb + TW4 + (nt * 16 + c) * TNH + q * 8;
-#pragma unroll
-    for (int k = 0; k < TNH / 32; ++k) w4[k].q = *(const uint4*)(wr + 32 * k);
-  }
+  if (mt < MT / 16) load_tile<TNH>(a.wb + TW4, nt, w4);
   finish(1, sh[1]);
   layer<TNH, TLD, MT>(sh[1], w3, acc);
   finish(2, sh[0]);
@@ -197,26 +197,32 @@ __global__ __launch_bounds__(TNT, 2) void k_train_dx(TrainDx a, int M) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, q = lane >> 4, c = lane & 15;
   const int row0 = blockIdx.x * MT;
   float* bp = a.bpart + (long)blockIdx.x * TBALL;
-  V8 w4[1][2], w3[TNH / 32][2], w2[TNH / 32][2];
-  em_load<TNOUTP>(a.wt + TW4, w4);
-  em_load<TNH>(a.wt + TW3, w3);
-  float4 zv[2][MT / 16];
-  auto load_z = [&](int l) {
+  float gv[MT / 16];
+#pragma unroll
+  for (int it = 0; it < MT / 16; ++it) {
+    const int e = tid + TNT * it, m = e >> 5, n = e & 31;
+    gv[it] = a.gy[(long)min(row0 + m, M - 1) * TNOUT + min(n, TNOUT - 1)];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  V8 w4[2][1], w3[2][TNH / 32], w2[2][TNH / 32];
+  load_pair<TNOUTP>(a.wt + TW4, w4);
+  load_pair<TNH>(a.wt + TW3, w3);
+  float4 zv[3][2][MT / 16];
+#pragma unroll
+  for (int l = 2; l >= 0; --l)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < MT / 16; ++j) {
         const int row = row0 + j * 16 + c;
-        zv[i][j] = *(const float4*)(a.z[l] + (long)(row < M ? row : M - 1) * TNH + wv * 32 +
-                                    i * 16 + 4 * q);
+        zv[l][i][j] = *(const float4*)(a.z[l] + (long)(row < M ? row : M - 1) * TNH + wv * 32 +
+                                       i * 16 + 4 * q);
       }
-  };
-  load_z(2);
 #pragma unroll
   for (int it = 0; it < MT / 16; ++it) {
     const int e = tid + TNT * it, m = e >> 5, n = e & 31;
     const long row = row0 + m;
-    const float v = row < M && n < TNOUT ? a.gy[row * TNOUT + n] : 0.f;
+    const float v = row < M && n < TNOUT ? gv[it] : 0.f;
     const uint16_t p = f2bf(v);
     sy[m * TLDY + n] = p;
     sg[m][n] = v;
@@ -240,7 +246,7 @@ __global__ __launch_bounds__(TNT, 2) void k_train_dx(TrainDx a, int M) {
       for (int j = 0; j < MT / 16; ++j) {
         const int m = j * 16 + c;
         const bool in = row0 + m < M;
-        const float4 z = zv[i][j];
+        const float4 z = zv[l][i][j];
         const float g[4] = {in ? acc[i][j][0] * gelu_d(z.x) : 0.f,
                             in ? acc[i][j][1] * gelu_d(z.y) : 0.f,
                             in ? acc[i][j][2] * gelu_d(z.z) : 0.f,
@@ -258,12 +264,10 @@ __global__ __launch_bounds__(TNT, 2) void k_train_dx(TrainDx a, int M) {
     rows_out<MT>(out, a.dz[l], row0, M);
   };
   layer<TNOUTP, TLDY, MT>(sy, w4, acc);
-  em_load<TNH>(a.wt + TW2, w2);
+  load_pair<TNH>(a.wt + TW2, w2);
   finish(2, sd[0]);
-  load_z(1);
   layer<TNH, TLD, MT>(sd[0], w3, acc);
   finish(1, sd[1]);
-  load_z(0);
   layer<TNH, TLD, MT>(sd[1], w2, acc);
   finish(0, sd[0]);
 }

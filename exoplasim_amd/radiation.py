@@ -67,13 +67,11 @@ def _proto():
         L.exo_mlp_train_forward.argtypes = [c_int, fp, vp, vp, vp, vp, vp, fp, vp, vp]
         L.exo_mlp_train_backward.restype = c_int
         L.exo_mlp_train_backward.argtypes = [c_int, fp, vp, vp, vp, vp, vp, vp, vp, vp]
-        L.exo_mlp_cast_weights.restype = c_int
-        L.exo_mlp_cast_weights.argtypes = [fp, c_int, c_int, c_int, c_int, vp, vp, vp]
-        L.exo_lw_emulate.restype = c_int
-        L.exo_lw_emulate.argtypes = [POINTER(_Net), c_int, fp, fp, fp, fp, fp, fp, vp]
-        L.exo_lw_emulate_guarded.restype = c_int
-        L.exo_lw_emulate_guarded.argtypes = [POINTER(_Net), fp, fp, c_int, fp, fp, fp, fp, fp,
-                                             fp, vp, vp]
+        L.exo_mlp_pack_weights.restype = c_int
+        L.exo_mlp_pack_weights.argtypes = [fp, c_int, c_int, c_int, c_int, vp, vp]
+        L.exo_lw_emulate_packed.restype = c_int
+        L.exo_lw_emulate_packed.argtypes = [POINTER(_Net), fp, fp, c_int, fp, fp, fp, fp, fp, fp,
+                                            vp, vp]
         L._rad_proto = True
     return L
 
@@ -316,17 +314,16 @@ class LwEmulator:
         return emulator_op()(x, *self.params)
 
     def _freeze(self):
-        """bf16 padded copies of the weights for the fused inference kernel"""
+        """bf16 padded copies of the weights, in the inference kernel's order"""
         import torch
 
         L = _proto()
         s = _stream()
         ws = []
         for (nin, nout), (K, N), w in zip(LAYERS, PADDED, self.params[0::2]):
-            W = torch.empty((N, K), dtype=torch.bfloat16, device="cuda")
-            Wt = torch.empty((K, N), dtype=torch.bfloat16, device="cuda")
-            _chk(L.exo_mlp_cast_weights(_ptr(w.detach().contiguous()), nout, nin, N, K, _ptr(W),
-                                        _ptr(Wt), s), "cast_weights")
+            W = torch.empty(N * K, dtype=torch.bfloat16, device="cuda")
+            _chk(L.exo_mlp_pack_weights(_ptr(w.detach().contiguous()), nout, nin, N, K, _ptr(W),
+                                        s), "pack_weights")
             ws.append(W)
         bs = [b.detach().float().contiguous() for b in self.params[1::2]]
         ym, ys = self.ymean.float().contiguous(), self.ystd.float().contiguous()
@@ -334,11 +331,11 @@ class LwEmulator:
                    (c_void_p * 4)(*[_ptr(b) for b in bs]), _ptr(ym), _ptr(ys))
         self._net = (net, ws, bs, ym, ys)  # keeps the buffers alive
         self._net_ref = ctypes.byref(net)
-        self._emulate = L.exo_lw_emulate
+        self._emulate = L.exo_lw_emulate_packed
 
     def predict(self, cols, out=None):
         """heating (nlev, ncol) K/day and OLR (ncol) of device columns, in
-        one kernel (exo_lw_emulate).  out=(heat, olr) reuses fp32 buffers."""
+        one kernel (exo_lw_emulate_packed).  out=(heat, olr) reuses fp32 buffers."""
         import torch
 
         if self._net is None:
@@ -354,9 +351,9 @@ class LwEmulator:
             olr = torch.empty(ncol, dtype=torch.float32, device=dp.device)
         else:
             heat, olr = out
-        _chk(self._emulate(self._net_ref, ncol, dt.data_ptr(), dq.data_ptr(), dp.data_ptr(),
-                           co2.data_ptr(), heat.data_ptr(), olr.data_ptr(), _stream()),
-             "exo_lw_emulate")
+        _chk(self._emulate(self._net_ref, None, None, ncol, dt.data_ptr(), dq.data_ptr(),
+                           dp.data_ptr(), co2.data_ptr(), heat.data_ptr(), olr.data_ptr(), None,
+                           _stream()), "exo_lw_emulate")
         return heat, olr
 
     def predict_guarded(self, cols, column: "LwrColumn"):
@@ -378,10 +375,9 @@ class LwEmulator:
         olr = torch.empty(ncol, dtype=torch.float32, device=dp.device)
         outside = torch.empty(ncol, dtype=torch.int32, device=dp.device)
         flo, fhi = self.flo.float().contiguous(), self.fhi.float().contiguous()
-        _chk(_proto().exo_lw_emulate_guarded(self._net_ref, flo.data_ptr(), fhi.data_ptr(), ncol,
-                                             dt.data_ptr(), dq.data_ptr(), dp.data_ptr(),
-                                             co2.data_ptr(), heat.data_ptr(), olr.data_ptr(),
-                                             outside.data_ptr(), _stream()),
+        _chk(self._emulate(self._net_ref, flo.data_ptr(), fhi.data_ptr(), ncol, dt.data_ptr(),
+                           dq.data_ptr(), dp.data_ptr(), co2.data_ptr(), heat.data_ptr(),
+                           olr.data_ptr(), outside.data_ptr(), _stream()),
              "exo_lw_emulate_guarded")
         idx = torch.nonzero(outside, as_tuple=True)[0]
         n = int(idx.numel())

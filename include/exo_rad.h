@@ -100,7 +100,7 @@ typedef struct {
  * (nlev+1 rows, the last the surface), dq (nlev rows), dp (1 row), dqco2 (its
  * first row) -- to heat (nlev rows, K/day) and olr (1 row, W/m2).  Features,
  * the four layers (bf16 MFMA, fp32 accumulate) and the output scaling run
- * per block of 32 columns with the activations in LDS. */
+ * per block of 16 or 32 columns with the activations in LDS. */
 int exo_lw_emulate(const exo_lw_net *net, int ncol, const float *dt, const float *dq,
                    const float *dp, const float *dqco2, float *heat, float *olr, void *stream);
 /* The same, and outside[col] = 1 for every column with one of its 43
@@ -111,6 +111,16 @@ int exo_lw_emulate_guarded(const exo_lw_net *net, const float *flo, const float 
                            const float *dt, const float *dq, const float *dp,
                            const float *dqco2, float *heat, float *olr, int *outside,
                            void *stream);
+/* The same with the weights of net in fragment order, each W[N][K] as
+ * exo_mlp_pack_weights writes it from the fp32 master w[nout][nin] (bf16, zero
+ * padded; N a multiple of 16, K of 32): the order in which the kernel's matrix
+ * instructions hold them, which it loads faster than rows.  outside == NULL:
+ * no guard, flo and fhi are not read. */
+int exo_mlp_pack_weights(const float *w, int nout, int nin, int N, int K, void *packed,
+                         void *stream);
+int exo_lw_emulate_packed(const exo_lw_net *net, const float *flo, const float *fhi, int ncol,
+                          const float *dt, const float *dq, const float *dp, const float *dqco2,
+                          float *heat, float *olr, int *outside, void *stream);
 
 #ifdef __cplusplus
 }

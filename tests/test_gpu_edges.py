@@ -308,3 +308,51 @@ def test_mlp_saved_outputs_have_no_gradient(gpu):
     out = torch.ops.exoplasim_amd.lw_mlp_forward(torch.randn(20, 43, device="cuda"), *em.params)
     out[2].sum().backward()
     assert all(p.grad is not None and not bool(p.grad.any()) for p in em.params)
+
+
+@pytest.mark.parametrize("ncol", [1, 17, 4096, 4097])
+def test_emulate_row_major_weights(gpu, ncol):
+    """inference from row-major weights (exo_lw_emulate, guarded or not)
+    against the fragment order that the class keeps, on both sides of the
+    change from 16 to 32 columns per block: the same products in the same
+    order, so equal to the last bit; and both guards flag the same columns"""
+    import ctypes
+
+    import torch
+
+    from exoplasim_amd import radiation as R
+    from exoplasim_amd._lib import lib
+    from exoplasim_amd.columns import make_columns
+
+    print(f"row-major emulate {ncol}", flush=True)
+    em = R.LwEmulator(seed=5)
+    cols = R.columns_to_device(make_columns(ncol, 20, 3), torch.float32)
+    heat, olr = em.predict(cols)
+    L, vp, ci = lib(), ctypes.c_void_p, ctypes.c_int
+    ws = []
+    for (nin, nout), (K, N), w in zip(R.LAYERS, R.PADDED, em.params[0::2]):
+        W = torch.empty((N, K), dtype=torch.bfloat16, device="cuda")
+        Wt = torch.empty((K, N), dtype=torch.bfloat16, device="cuda")
+        assert L.exo_mlp_cast_weights(vp(w.data_ptr()), ci(nout), ci(nin), ci(N), ci(K),
+                                      vp(W.data_ptr()), vp(Wt.data_ptr()), None) == 0
+        ws.append((W, Wt))
+    net = R._Net(20, (vp * 4)(*[W.data_ptr() for W, _ in ws]),
+                 (vp * 4)(*[b.data_ptr() for b in em.params[1::2]]), em.ymean.data_ptr(),
+                 em.ystd.data_ptr())
+    x = [vp(cols[k].data_ptr()) for k in ("dt", "dq", "dp", "dqco2")]
+    h, o = torch.empty_like(heat), torch.empty_like(olr)
+    assert L.exo_lw_emulate(ctypes.byref(net), ci(ncol), *x, vp(h.data_ptr()), vp(o.data_ptr()),
+                            None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(h, heat) and torch.equal(o, olr)
+    f = R.features(cols)
+    lo, hi = f.quantile(0.02, dim=0), f.quantile(0.98, dim=0)
+    flags = [torch.empty(ncol, dtype=torch.int32, device="cuda") for _ in range(2)]
+    assert L.exo_lw_emulate_guarded(ctypes.byref(net), vp(lo.data_ptr()), vp(hi.data_ptr()),
+                                    ci(ncol), *x, vp(h.data_ptr()), vp(o.data_ptr()),
+                                    vp(flags[0].data_ptr()), None) == 0
+    assert L.exo_lw_emulate_packed(em._net_ref, vp(lo.data_ptr()), vp(hi.data_ptr()), ci(ncol),
+                                   *x, vp(h.data_ptr()), vp(o.data_ptr()),
+                                   vp(flags[1].data_ptr()), None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(h, heat) and torch.equal(o, olr) and torch.equal(*flags)
