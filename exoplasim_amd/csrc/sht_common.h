@@ -135,6 +135,14 @@ __device__ __forceinline__ double row_ror8(double x) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// x, or -x where sign = 0x80000000 (else 0)
+__device__ __forceinline__ float flip_sign(float x, uint32_t sign) {
+  return __uint_as_float(__float_as_uint(x) ^ sign);
+}
+__device__ __forceinline__ double flip_sign(double x, uint32_t sign) {
+  return __longlong_as_double(__double_as_longlong(x) ^ ((long long)(unsigned long long)sign << 32));
+}
+
 // a per-lane byte offset that no buffer covers: such a load returns 0
 constexpr int BUF_NONE = 0x7ff00000;
 

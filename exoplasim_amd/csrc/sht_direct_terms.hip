@@ -51,10 +51,8 @@ struct DirxCfg {
   // the LDS.
   static constexpr int KC = (sizeof(R) == 8) ? ((NIN == 1) ? 8 : 4)
                             : (NIN == 1)     ? ((T == 127) ? 8 : 16)
-                            : (T == 127)     ? ((NIN == 2) ? 8 : 4)
-                            : (NIN == 3)     ? 8
-                            : (T == 63)      ? 16
-                                             : 8;
+                            : (NIN == 2 && T == 63) ? 16
+                                                    : 8;
   static constexpr int KS = DIRX_LG * 2 * DIRX_MR + 2;  // reals per (input, class, pair), padded
   static constexpr size_t LDS = sizeof(R) * NIN * 2 * KC * KS;
 };
@@ -79,7 +77,8 @@ struct DirxJobs {
   DirxJob<R> job[DIRX_JOBS];
 };
 
-template <int T, typename R, int NIN, int NOUT>
+// RB: row tiles of 16 per parity that the block's wavenumbers need (dirx_run)
+template <int T, typename R, int NIN, int NOUT, int RB>
 __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, int mr,
                                           char* lds) {
   using S = TS<T>;
@@ -87,7 +86,7 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
   using R2 = R __attribute__((ext_vector_type(2)));
   using Acc = typename std::conditional<sizeof(R) == 8, f64x4, f32x4>::type;
   constexpr bool F64 = sizeof(R) == 8;
-  constexpr int N = S::NLON, NLAT = S::NLAT, NPAIR = S::NPAIR, RB = S::RB, NCSP = S::NCSP;
+  constexpr int N = S::NLON, NLAT = S::NLAT, NPAIR = S::NPAIR, NCSP = S::NCSP;
   constexpr int MR = DIRX_MR, LG = DIRX_LG, KC = C::KC, KS = C::KS, NT = DIRX_NT;
   constexpr int NKS = KC / 4;  // MFMA K steps (4 pairs each) per staged step
   constexpr int NJ = 2 * MR;   // reals of one staged row segment
@@ -102,46 +101,41 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = mr * MR, lev0 = lg * LG;
-  const int nj = (S::NM - m0 < MR ? S::NM - m0 : MR) * 2;  // reals below the truncation
   const int nl = a.nlev - lev0 < LG ? a.nlev - lev0 : LG;  // levels of this block
 
-  // each input's levels of this block as one buffer (2 m0 + NJ <= N: the
-  // 16-byte runs stay inside their rows; reals past the truncation are
-  // zeroed)
-  __amdgpu_buffer_rsrc_t rsi[NIN];
-#pragma unroll
-  for (int i = 0; i < NIN; ++i)
-    rsi[i] = buffer_rsrc(a.in[i] + mem * a.in_stride + (long)lev0 * NLAT * N,
-                         nl * NLAT * N * (int)sizeof(R));
+  // A wave stages items of one input: its levels of this block as one buffer,
+  // so that levels past the last load zeros (2 m0 + NJ <= N: the 16-byte runs
+  // stay inside their rows; reals past the truncation are staged and not used).
+  // The loads have no branch and no arithmetic on their results, which would
+  // wait for them here instead of at the next step's fold.
+  static_assert(NJ4 * KC * LG % 64 == 0, "one input per wave");
   static_assert(2 * ((TS<T>::NM - 1) / MR * MR) + NJ <= N, "staged runs inside a row");
-  auto quad = [&](__amdgpu_buffer_rsrc_t rs, int off, R* v) {
+  constexpr int ES = (int)sizeof(R), NC = NPAIR / KC;
+  __amdgpu_buffer_rsrc_t rsi[MAXIT];
+  int vn[MAXIT], vs[MAXIT];  // byte offsets of the northern run of step 0, the southern of step NC - 1
+#pragma unroll
+  for (int it = 0; it < MAXIT; ++it) {
+    const int e = tid + NT * it;
+    const int j4 = e % NJ4, k = (e / NJ4) % KC, l = (e / (NJ4 * KC)) % LG;
+    const int i = (64 * wv + NT * it) / (NJ4 * KC * LG);
+    const R* in = NIN > 2 && i == 2 ? a.in[NIN > 2 ? 2 : 0] : NIN > 1 && i == 1 ? a.in[1] : a.in[0];
+    rsi[it] = buffer_rsrc(in + mem * a.in_stride + (long)lev0 * NLAT * N, nl * NLAT * N * ES);
+    const int o = l * NLAT * N + 2 * m0 + 4 * j4;
+    vn[it] = e < NITEM ? (o + k * N) * ES : BUF_NONE;
+    vs[it] = e < NITEM ? (o + (NLAT - NPAIR + KC - 1 - k) * N) * ES : BUF_NONE;
+  }
+  auto quad = [&](__amdgpu_buffer_rsrc_t rs, int off, int soff, R* v) {
     uint4 u[sizeof(R) / 4];
 #pragma unroll
-    for (int h = 0; h < (int)sizeof(R) / 4; ++h) u[h] = buffer_load_x4(rs, off + 16 * h, 0);
+    for (int h = 0; h < (int)sizeof(R) / 4; ++h) u[h] = buffer_load_x4(rs, off + 16 * h, soff);
     __builtin_memcpy(v, u, 4 * sizeof(R));
   };
   R rn[MAXIT][4], rs[MAXIT][4];
   auto load = [&](int c) {
 #pragma unroll
     for (int it = 0; it < MAXIT; ++it) {
-      const int e = tid + NT * it;
-      const int j4 = e % NJ4, k = (e / NJ4) % KC, l = (e / (NJ4 * KC)) % LG,
-                i = e / (NJ4 * KC * LG);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) rn[it][q] = rs[it][q] = R(0);
-      if (e < NITEM && l < nl && 4 * j4 < nj) {
-        const int pair = c * KC + k;
-        const int off = (l * NLAT * N + 2 * m0 + 4 * j4) * (int)sizeof(R);
-        R vn[4], vs[4];
-        quad(rsi[i], off + pair * N * (int)sizeof(R), vn);
-        quad(rsi[i], off + (NLAT - 1 - pair) * N * (int)sizeof(R), vs);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (4 * j4 + q < nj) {
-            rn[it][q] = vn[q];
-            rs[it][q] = vs[q];
-          }
-      }
+      quad(rsi[it], vn[it], c * KC * N * ES, rn[it]);
+      quad(rsi[it], vs[it], (NC - 1 - c) * KC * N * ES, rs[it]);
     }
   };
   // fold into E = N + S (class 0) and O = N - S (class 1)
@@ -149,7 +143,7 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
 #pragma unroll
     for (int it = 0; it < MAXIT; ++it) {
       const int e = tid + NT * it;
-      if (e < NITEM) {
+      if (64 * wv + NT * it < NITEM) {
         const int j4 = e % NJ4, k = (e / NJ4) % KC, l = (e / (NJ4 * KC)) % LG,
                   i = e / (NJ4 * KC * LG);
         const int o = l * NJ + 4 * j4;  // even, and KS is even: pairs of reals are aligned
@@ -166,14 +160,10 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
   // A operand: row r = lane & 15, pair 4 ks + (lane >> 4) of the step; B
   // operand: column lane & 15 = (level l, component oc), the same pair
   const int r = lane & 15, kq = lane >> 4, l = (lane & 15) >> 1, oc = lane & 1;
-  const int m = m0 + wv;
-  const bool live = m <= T;  // the last range of wavenumbers may end early
-  const int w0 = w0_of(T, live ? m : T);
-  auto ntile = [](int mm, int p) {
-    const int d = T - mm - p;
-    return d < 0 ? 0 : (d / 2 + 16) / 16;
-  };
-  const int nt0 = live ? ntile(m, 0) : 0, nt1 = live ? ntile(m, 1) : 0;
+  // (the waves past the truncation repeat the last wavenumber's tables and
+  // store nothing)
+  const int m = m0 + wv < T ? m0 + wv : T;
+  const int w0 = w0_of(T, m);
   Acc acc[NOUT][2][RB];
 #pragma unroll
   for (int o = 0; o < NOUT; ++o)
@@ -181,20 +171,24 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int rt = 0; rt < RB; ++rt) acc[o][p][rt] = Acc{0, 0, 0, 0};
-  // this lane's B source per output and slot: offset of (input, class 0,
-  // pair kq, level l, component ic) in X and the sign (0: no term for
-  // component oc); has: does the output have a term with the slot's table
-  int boff[NOUT][NIN];
-  R bsg[NOUT][NIN];
-  bool has[NOUT][NIN];
+  // this lane's B source per output, slot and parity: offset of (input, class,
+  // pair kq, level l, component ic) in X, and the sign bit.  Of the folded
+  // input the symmetric class (E) iff (n - m even) != Q-type table.
+  auto term = [](int o, int s) { return !(NIN == 3 && NOUT == 2 && o == 1 && s == 0); };
+  int boff[NOUT][NIN][2];
+  uint32_t bsg[NOUT][NIN];
 #pragma unroll
   for (int o = 0; o < NOUT; ++o)
 #pragma unroll
     for (int s = 0; s < NIN; ++s) {
-      boff[o][s] = ((oc ? a.src[o][s][1] : a.src[o][s][0]) * 2 * KC + kq) * KS + l * NJ +
-                   (oc ? a.ic[o][s][1] : a.ic[o][s][0]) + 2 * wv;
-      bsg[o][s] = (R)(oc ? a.sign[o][s][1] : a.sign[o][s][0]);
-      has[o][s] = a.sign[o][s][0] != 0 || a.sign[o][s][1] != 0;
+      const int src = oc ? a.src[o][s][1] : a.src[o][s][0];
+      const int ic = oc ? a.ic[o][s][1] : a.ic[o][s][0];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int cls = (p == 0) == (a.isq[s] != 0) ? 1 : 0;
+        boff[o][s][p] = ((src * 2 + cls) * KC + kq) * KS + l * NJ + ic + 2 * wv;
+      }
+      bsg[o][s] = (oc ? a.sign[o][s][1] : a.sign[o][s][0]) < 0 ? 0x80000000u : 0u;
     }
   // FP64 tables are read as they are, [pair][w]: the pair of reals at w0 +
   // 2 (16 rt + r) holds the rows n of both parities, so one 16-byte load
@@ -206,7 +200,6 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
     for (int s = 0; s < NIN; ++s) rst[s] = buffer_rsrc(a.tab[s], NPAIR * NCSP * 8);
   }
 
-  constexpr int NC = NPAIR / KC;
   load(0);
   for (int c = 0; c < NC; ++c) {
     __syncthreads();  // the previous step's MFMAs have read X
@@ -216,72 +209,59 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
     // then the next step's inputs, whose loads stay in flight through the
     // MFMAs
     R av[NIN][2][RB][NKS];
-    if (live) {
 #pragma unroll
-      for (int s = 0; s < NIN; ++s) {
+    for (int s = 0; s < NIN; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RB; ++rt) {
         if constexpr (F64) {
 #pragma unroll
-          for (int rt = 0; rt < RB; ++rt)
-            if (rt < nt0) {
-#pragma unroll
-              for (int ks = 0; ks < NKS; ++ks) {
-                const uint4 v = buffer_load_x4(rst[s], (kq * NCSP + 2 * r) * 8,
-                                               ((c * KC + 4 * ks) * NCSP + w0 + 32 * rt) * 8);
-                R d[2];
-                __builtin_memcpy(d, &v, 16);
-                av[s][0][rt][ks] = d[0];
-                av[s][1][rt][ks] = d[1];
-              }
-            }
+          for (int ks = 0; ks < NKS; ++ks) {
+            const uint4 v = buffer_load_x4(rst[s], (kq * NCSP + 2 * r) * 8,
+                                           ((c * KC + 4 * ks) * NCSP + w0 + 32 * rt) * 8);
+            R d[2];
+            __builtin_memcpy(d, &v, 16);
+            av[s][0][rt][ks] = d[0];
+            av[s][1][rt][ks] = d[1];
+          }
         } else {
-          const R* tp = a.tab[s] + ((long)(m * 2) * RB * NPAIR + c * KC + kq) * 16 + r;
+          // one 16-byte load per 8 pairs and row tile: 2 K steps of both parities
 #pragma unroll
-          for (int p = 0; p < 2; ++p)
+          for (int g = 0; g < KC / 8; ++g) {
+            const f32x4 v = ((const f32x4*)a.tab[s])[((m * S::RB + rt) * (NPAIR / 8) +
+                                                      c * (KC / 8) + g) * 64 + lane];
 #pragma unroll
-            for (int rt = 0; rt < RB; ++rt)
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-              for (int ks = 0; ks < NKS; ++ks)
-                av[s][p][rt][ks] = tp[(((long)p * RB + rt) * NPAIR + 4 * ks) * 16];
+              for (int h = 0; h < 2; ++h) av[s][p][rt][2 * g + h] = v[2 * p + h];
+          }
         }
       }
-    }
     if (c + 1 < NC) load(c + 1);
-    if (!live) continue;
 #pragma unroll
     for (int s = 0; s < NIN; ++s)
 #pragma unroll
       for (int o = 0; o < NOUT; ++o) {
-        if (NOUT > 1 && !has[o][s]) continue;
+        if (!term(o, s)) continue;
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          R b[2];
-#pragma unroll
-          for (int cls = 0; cls < 2; ++cls) {
-            const R x = X[boff[o][s] + (cls * KC + 4 * ks) * KS];
-            b[cls] = bsg[o][s] == R(0) ? R(0) : bsg[o][s] * x;
-          }
+        for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
           for (int p = 0; p < 2; ++p) {
-            // class of the folded input: symmetric (E) iff (n - m even) != Q-type table
-            const R bv = b[(p == 0) == (a.isq[s] != 0) ? 1 : 0];
-            const int nt = p ? nt1 : nt0;
+            const R bv = flip_sign(X[boff[o][s][p] + 4 * ks * KS], bsg[o][s]);
 #pragma unroll
-            for (int rt = 0; rt < RB; ++rt)
-              if (rt < nt) {
-                if constexpr (F64)
-                  acc[o][p][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][p][rt][ks], bv,
-                                                                       acc[o][p][rt], 0, 0, 0);
-                else
-                  acc[o][p][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][p][rt][ks], bv,
-                                                                       acc[o][p][rt], 0, 0, 0);
-              }
+            for (int rt = 0; rt < RB; ++rt) {
+              if constexpr (F64)
+                acc[o][p][rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][p][rt][ks], bv,
+                                                                     acc[o][p][rt], 0, 0, 0);
+              else
+                acc[o][p][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][p][rt][ks], bv,
+                                                                     acc[o][p][rt], 0, 0, 0);
+            }
           }
-        }
       }
   }
   // item v of a lane is row 4 kq + v of column (l, oc); in the FP64 form row
   // 4 v + kq
-  if (l >= nl || !live) return;
+  if (l >= nl || m0 + wv > T) return;
 #pragma unroll
   for (int o = 0; o < NOUT; ++o) {
     R* out = a.out[o] + mem * a.out_stride + (long)(lev0 + l) * S::NRSP;
@@ -295,6 +275,24 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
           if (m + dn <= T) out[2 * (w0 + dn) + oc] = acc[o][p][rt][v];
         }
   }
+}
+
+// The block's wavenumbers m0 .. m0 + 7 need the row tiles of m0 (n - m = 0 .. T
+// - m0); the tile count is a template argument of the body, so that its products
+// have no branches between them.  (A branch per product, on the wavenumber's
+// own tile count, and one per operand for terms that a list does not have, kept
+// the compiler from overlapping any of a step's loads: T42 L20, 32 members,
+// gridpointa 241 us against 258, T21 L10 FP64, one member, 28.5 against 31.9, T127
+// L40 round trip of 8 members 722 against 736.)
+template <int T, typename R, int NIN, int NOUT, int RB = 1>
+__device__ __forceinline__ void dirx_run(const DirxJob<R>& a, int mem, int lg, int mr, char* lds) {
+  if constexpr (RB < TS<T>::RB) {
+    if ((T - mr * DIRX_MR) / 2 >= 16 * RB) {
+      dirx_run<T, R, NIN, NOUT, RB + 1>(a, mem, lg, mr, lds);
+      return;
+    }
+  }
+  dirx_body<T, R, NIN, NOUT, RB>(a, mem, lg, mr, lds);
 }
 
 // Minimum waves per SIMD asked of the compiler: two blocks per CU instead of
@@ -319,7 +317,7 @@ __global__ __launch_bounds__(DIRX_NT, (dirx_waves<T, R, NOUT, NIN>())) void k_di
   // lines of a Fourier row: renumbered so that they run on one XCD's L2
   const int b = xcd_block(blockIdx.x, gridDim.x);
   const int mem = b / per, i = b - mem * per;
-  dirx_body<T, R, NIN, NOUT>(a, mem, i / NMR, i % NMR, lds);
+  dirx_run<T, R, NIN, NOUT>(a, mem, i / NMR, i % NMR, lds);
 }
 
 // mktend, gridpointa: jobs of three inputs and one or two outputs, and of one
@@ -342,11 +340,11 @@ __global__ __launch_bounds__(DIRX_NT, (dirx_waves<T, R, 2, 3>())) void k_dirx_mf
   const int i = q - j.start[k];
   const int mr = i % NMR, lg = i / NMR;
   if (a.nin == 1)
-    dirx_body<T, R, 1, 1>(a, mem, lg, mr, lds);
+    dirx_run<T, R, 1, 1>(a, mem, lg, mr, lds);
   else if (a.nout == 1)
-    dirx_body<T, R, 3, 1>(a, mem, lg, mr, lds);
+    dirx_run<T, R, 3, 1>(a, mem, lg, mr, lds);
   else
-    dirx_body<T, R, 3, 2>(a, mem, lg, mr, lds);
+    dirx_run<T, R, 3, 2>(a, mem, lg, mr, lds);
 }
 
 template <int T, typename R>
@@ -384,6 +382,12 @@ static int dirx_t(const Tables& tb, const DirxArgs* args, int njob, hipStream_t 
     }
     if (nslot != a.nin) return -2;  // one table per input
     if (a.nin < 3 && a.nin != a.nout) return -2;
+    // every output has a term of every table, but the second of three inputs'
+    // (mktend's vorticity) none of the first
+    for (int o = 0; o < a.nout; ++o)
+      for (int i = 0; i < a.nin; ++i)
+        for (int c = 0; c < 2; ++c)
+          if ((g.sign[o][i][c] != 0) != !(a.nin == 3 && a.nout == 2 && o == 1 && i == 0)) return -2;
     wide = wide || a.nin == 3;
     for (int i = 0; i < a.nin; ++i) g.in[i] = (const R*)a.in[i];
     for (int o = 0; o < a.nout; ++o) g.out[o] = (R*)a.out[o];
