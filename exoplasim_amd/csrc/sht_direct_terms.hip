@@ -18,11 +18,11 @@
 // A block owns one member, 8 levels and MR wavenumbers of one job: up to 3
 // inputs (one table each) and up to 2 outputs that share them.  It walks the
 // latitude pairs KC at a time: the folded Fourier values of those pairs
-// (all inputs, its levels and wavenumbers) are staged in LDS, every table
-// operand of the step is requested, then the next pairs' values, and the
-// MFMAs run while those are in flight; every (output, m, p, row tile)
-// accumulates in registers across all pairs, so the sum over latitudes is
-// complete in the block (no partial sums).  Wave w takes m = m0 + w.
+// (all inputs, its levels and wavenumbers) are staged in LDS, and the tables
+// and inputs of the steps ahead are in flight through the MFMAs; every
+// (output, m, p, row tile) accumulates in registers across all pairs, so the
+// sum over latitudes is complete in the block (no partial sums).  Wave w takes
+// m = m0 + w.
 //
 // What bounds it is the latency of those steps (stage, barrier, tables), not
 // bytes or flops, so the jobs of one call run in one launch: the blocks of
@@ -54,7 +54,11 @@ struct DirxCfg {
                             : (NIN == 2 && T == 63) ? 16
                                                     : 8;
   static constexpr int KS = DIRX_LG * 2 * DIRX_MR + 2;  // reals per (input, class, pair), padded
-  static constexpr size_t LDS = sizeof(R) * NIN * 2 * KC * KS;
+  // FP32: two staged steps in LDS and two steps' tables in registers; FP64's
+  // registers leave no room for the second (T127 L10 gridpointa 233 -> 283 us)
+  static constexpr bool AHEAD = sizeof(R) == 4;
+  static constexpr int STEP = NIN * 2 * KC * KS;  // reals of one staged step
+  static constexpr size_t LDS = sizeof(R) * STEP * (AHEAD ? 2 : 1);
 };
 
 // one job: the term list regrouped by table.  Slot s multiplies table tab[s]
@@ -97,7 +101,7 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
   constexpr int NJ4 = NJ / 4;
   constexpr int NITEM = NIN * LG * KC * NJ4;
   constexpr int MAXIT = (NITEM + NT - 1) / NT;
-  R* X = (R*)lds;  // [input][class][pair][level][m][re/im]
+  R* const X0 = (R*)lds;  // [step % 2 (AHEAD)][input][class][pair][level][m][re/im]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = mr * MR, lev0 = lg * LG;
@@ -139,7 +143,7 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
     }
   };
   // fold into E = N + S (class 0) and O = N - S (class 1)
-  auto store = [&]() {
+  auto store = [&](R* X) {
 #pragma unroll
     for (int it = 0; it < MAXIT; ++it) {
       const int e = tid + NT * it;
@@ -200,15 +204,7 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
     for (int s = 0; s < NIN; ++s) rst[s] = buffer_rsrc(a.tab[s], NPAIR * NCSP * 8);
   }
 
-  load(0);
-  for (int c = 0; c < NC; ++c) {
-    __syncthreads();  // the previous step's MFMAs have read X
-    store();
-    __syncthreads();
-    // every A operand of this step first, so that their latencies overlap;
-    // then the next step's inputs, whose loads stay in flight through the
-    // MFMAs
-    R av[NIN][2][RB][NKS];
+  auto tables = [&](int c, R (&av)[NIN][2][RB][NKS]) {
 #pragma unroll
     for (int s = 0; s < NIN; ++s)
 #pragma unroll
@@ -236,7 +232,8 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
           }
         }
       }
-    if (c + 1 < NC) load(c + 1);
+  };
+  auto products = [&](const R* X, const R (&av)[NIN][2][RB][NKS]) {
 #pragma unroll
     for (int s = 0; s < NIN; ++s)
 #pragma unroll
@@ -258,6 +255,43 @@ __device__ __forceinline__ void dirx_body(const DirxJob<R>& a, int mem, int lg, 
             }
           }
       }
+  };
+  load(0);
+  if constexpr (C::AHEAD) {
+    // While step c is multiplied, the tables of step c + 1 and the inputs of
+    // step c + 2 are on their way, and the inputs of step c + 1 are folded into
+    // the other half of LDS.  One barrier per step: behind it the half of step c
+    // is complete, and that of step c - 1 no longer read.  (One step and two
+    // barriers: T42 L20, 32 members, gridpointa 241 us against 237, T127 L20, 2
+    // members, 312 against 290, the T127 round trip 722 against 713.)
+    R av[2][NIN][2][RB][NKS];
+    tables(0, av[0]);
+    store(X0);
+    if (NC > 1) load(1);
+    auto step = [&](int c, const R (&cur)[NIN][2][RB][NKS], R (&next)[NIN][2][RB][NKS]) {
+      __syncthreads();
+      if (c + 1 < NC) tables(c + 1, next);
+      products(X0 + (c & 1) * C::STEP, cur);
+      if (c + 1 < NC) store(X0 + ((c + 1) & 1) * C::STEP);
+      if (c + 2 < NC) load(c + 2);
+    };
+    for (int c = 0; c < NC; c += 2) {
+      step(c, av[0], av[1]);
+      if (NC % 2 == 0 || c + 1 < NC) step(c + 1, av[1], av[0]);
+    }
+  } else {
+    for (int c = 0; c < NC; ++c) {
+      __syncthreads();  // the previous step's MFMAs have read X
+      store(X0);
+      __syncthreads();
+      // every A operand of this step first, so that their latencies overlap;
+      // then the next step's inputs, whose loads stay in flight through the
+      // MFMAs
+      R av[NIN][2][RB][NKS];
+      tables(c, av);
+      if (c + 1 < NC) load(c + 1);
+      products(X0, av);
+    }
   }
   // item v of a lane is row 4 kq + v of column (l, oc); in the FP64 form row
   // 4 v + kq
