@@ -292,9 +292,9 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     int bvoff = BUF_NONE;
     if constexpr (MODE == MODE_BF16X3) {
       rsB = buffer_rsrc((const float*)a.bpk + mem * a.bpk_stride, (int)a.bpk_stride * 4);
-      if (pf >= 0) bvoff = ((pf - a.bpk_f0) * pk_field(T) + jq) * 4;
+      if (pf >= 0)
+        bvoff = (pf - a.bpk_f0) * pk_field(T) * 4 + ((q & 1) * 4 + hq * 2 + (c & 1)) * 16;
     }
-    const int brow = (c & 1) * 2 + hq;  // re/im, parity row of the B segment
     const R pv = (R)a.plavor;
     // B fragment of one item: 8 values (F32MFMA: f, n = 4j + q), 4 of one
     // parity (F64: f, n - m = 2 (4j + q) + hc), or 8 fp32 values of one parity
@@ -327,10 +327,10 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         // lanes whose j lies past the row would read n > NTRU, where the
         // table operand is zero: they load nothing
         const bool inrow = live && 16 * kb + jq < rw;
-        const int bso = (pk_seg(T, m) + 16 * kb) * 4;
-        const int bv = inrow ? bvoff + brow * rw * 4 : BUF_NONE;
+        const int bso = (pk_seg(T, m) + 64 * kb) * 4;
+        const int bv = inrow ? bvoff : BUF_NONE;
         br.r[0] = buffer_load_x4(rsB, bv, bso);
-        br.r[1] = buffer_load_x4(rsB, bv, bso + 16);
+        br.r[1] = buffer_load_x4(rsB, bv, bso + (16 * kb + 8 < rw ? 128 : 64));
         // absolute -> relative vorticity at (m=0, n=1, re), the first odd
         // value (subtracted when the item is multiplied)
         br.fix = live && m == 0 && kb == 0 && isvor && q == 2;
@@ -342,21 +342,22 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         // multiplied: two 16-byte loads per term instead of three (a wave's
         // load costs the same however many of its lanes read).  Else each
         // lane loads its three planes, the other class's lanes nothing.
-        const int aso = (tab_seg(T, m) + 16 * kb) * 2;
-        const int av = (c * rw + jq) * 2;                          // own row, hi plane
+        const int aso = (tab_seg(T, m) + 768 * kb) * 2;
+        const int w = rw - 16 * kb < 16 ? rw - 16 * kb : 16;  // values per row
+        const int av = (c * w + jq) * 2;                          // own row, hi plane
         if constexpr (!PAIRLOAD) {
           const int av0 = (amine0 && inrow) ? av : BUF_NONE;
 #pragma unroll
-          for (int p = 0; p < 3; ++p) a0[p] = buffer_load_x4(rsA0, av0, aso + p * rw * 32);
+          for (int p = 0; p < 3; ++p) a0[p] = buffer_load_x4(rsA0, av0, aso + p * w * 32);
           if (NTERM == 2) {
             const int av1 = (amine1 && inrow) ? av : BUF_NONE;
 #pragma unroll
-            for (int p = 0; p < 3; ++p) a1[p] = buffer_load_x4(rsA1, av1, aso + p * rw * 32);
+            for (int p = 0; p < 3; ++p) a1[p] = buffer_load_x4(rsA1, av1, aso + p * w * 32);
           }
           return;
         }
-        const int avp = ((c ^ 1) * rw + jq) * 2 + rw * 32;         // partner's row, mid plane
-        const int avl = av + rw * 64;                              // own row, lo plane
+        const int avp = ((c ^ 1) * w + jq) * 2 + w * 32;         // partner's row, mid plane
+        const int avl = av + w * 64;                              // own row, lo plane
         {
           const int v1 = inrow ? (amine0 ? av : avp) : BUF_NONE;
           const int v2 = (amine0 && inrow) ? avl : BUF_NONE;

@@ -74,16 +74,20 @@ __host__ __device__ constexpr int pk_c16(int x) {
   const unsigned a = (unsigned)x >> 4, b = (unsigned)x & 15u;
   return (int)(64u * a * (a + 1u) + 8u * b * (a + 1u));
 }
-// spectral operand: per field, for each m, [re/im][h][pk_rw] fp32 values in
-// parity order (the inverse splits them into bf16 planes in registers)
+// spectral operand: per field, for each m, the fp32 values (which the inverse
+// splits into bf16 planes in registers) in the order in which a wave loads
+// them: blocks of 32 total wavenumbers (16 j) as [j / 4 % 2][j / 8][h][re/im][j %
+// 4], so that each of the two 16-byte loads of a lane takes one whole 128-byte
+// line per field; a last block of 8 j as [j / 4][h][re/im][j % 4]
 __host__ __device__ constexpr int pk_field(int ntru) { return 4 * pk_c16(ntru + 1); }
 __host__ __device__ constexpr int pk_seg(int ntru, int m) {
   return 4 * (pk_c16(ntru + 1) - pk_c16(ntru + 1 - m));
 }
-// table operand: per block of 8 latitude pairs, for each m,
-// [plane][row = 2 pair + class][pk_rw]; the row holds the parity of its
-// class (h = class for P-type tables, 1 - class for Q-type), the other
-// parity being zero and not stored
+// table operand: per block of 8 latitude pairs, for each m and each block of 32
+// total wavenumbers (16 j, the last 16 or 8), [plane][row = 2 pair +
+// class][j], so that one plane of a block is one run of 256 or 512 bytes; the
+// row holds the parity of its class (h = class for P-type tables, 1 - class for
+// Q-type), the other parity being zero and not stored
 __host__ __device__ constexpr int tab_pb(int ntru) { return 48 * pk_c16(ntru + 1); }
 __host__ __device__ constexpr int tab_seg(int ntru, int m) {
   return 48 * (pk_c16(ntru + 1) - pk_c16(ntru + 1 - m));

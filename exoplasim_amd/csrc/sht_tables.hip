@@ -209,8 +209,10 @@ __global__ void k_pack_inv_bf(int ntru, int npair, int t, const double* filt64, 
       hi = mid - 1;
   }
   const int m = lo, rw = pk_rw(ntru, m);
-  const int r = e - tab_seg(ntru, m) / 3;
-  const int row = r / rw, j = r - row * rw;
+  // one plane of block kb of m's segment: 16 rows of w values
+  const int r = e - tab_seg(ntru, m) / 3, kb = r >> 8;
+  const int w = rw - 16 * kb < 16 ? rw - 16 * kb : 16;
+  const int row = (r & 255) / w, j = 16 * kb + (r & 255) % w;
   const int pl = row >> 1, cls = row & 1;
   const int h = cls ^ (table_is_q(t) ? 1 : 0);
   const int n = m + 2 * j + h;
@@ -218,10 +220,10 @@ __global__ void k_pack_inv_bf(int ntru, int npair, int t, const double* filt64, 
       (n <= ntru) ? filt64[t * tsz + (long)(pb * 8 + pl) * ncsp + w0_of(ntru, m) + (n - m)] : 0.0;
   uint16_t hh, mm, ll;
   split3_f64(v, hh, mm, ll);
-  uint16_t* o = bf + (long)pb * tab_pb(ntru) + tab_seg(ntru, m) + row * rw + j;
+  uint16_t* o = bf + (long)pb * tab_pb(ntru) + tab_seg(ntru, m) + 768 * kb + (r & 255);
   o[0] = hh;
-  o[16 * rw] = mm;
-  o[32 * rw] = ll;
+  o[16 * w] = mm;
+  o[32 * w] = ll;
 }
 
 // ---- table operand of the MFMA direct transforms (k_dirx_mf): per (m, row

@@ -194,62 +194,62 @@ static int fft_t(const void* tw, int dir, R* a, long lot, int nmem, long mstride
 
 // ---------------------------------------------------------------------------
 // parity-ordered spectral operand of the split-BF16 inverse (layout in
-// sht_common.h): one thread per 4 consecutive coefficients n - m = 4g ..
-// 4g + 3 of one (member, field, m), read as two contiguous 16-byte loads
-// (consecutive threads read consecutive runs) and written as 8 bytes, the
-// values j = 2g, 2g + 1, into each of the m's four rows (re/im x parity),
-// so a wave writes 512 contiguous bytes of each row.  Coefficients past the
-// truncation are zeros.  (Each thread reading 8 values of one row at a
-// 16-byte stride put a wave's loads on 64 cache lines each.)
+// sht_common.h): one thread per 8 consecutive coefficients n - m = 8g ..
+// 8g + 7 of one (member, field, m), 64 contiguous bytes read and written.
+// Coefficients past the truncation are zeros.
 // ---------------------------------------------------------------------------
 template <int T>
 __global__ __launch_bounds__(256) void k_pack_sp(const float* sp, long sp_stride, int f0, int nf,
                                                  int nmem, float* out) {
   using S = TS<T>;
-  constexpr int NC = pk_c16(T + 1) / 2;  // threads per field: sum over m of rw(m) / 2
+  constexpr int NC = pk_field(T) / 16;  // threads per field: sum over m of rw(m) / 4
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)nmem * nf * NC) return;
   const int u = (int)(i % NC);
   const long fm = i / NC;
   const int field = (int)(fm % nf), mem = (int)(fm / nf);
   // the largest m whose segment starts at or before thread u (segment of m:
-  // threads pk_seg(m) / 8 .. + rw(m) / 2)
+  // threads pk_seg(m) / 16 .. + rw(m) / 4)
   int lo = 0, hi = T;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (pk_seg(T, mid) / 8 <= u)
+    if (pk_seg(T, mid) / 16 <= u)
       lo = mid;
     else
       hi = mid - 1;
   }
   const int m = lo, rw = pk_rw(T, m);
-  const int g = u - pk_seg(T, m) / 8;  // coefficients n - m = 4g .. 4g + 3
+  const int g = u - pk_seg(T, m) / 16;  // coefficients n - m = 8g .. 8g + 7
   // the member's fields as one buffer: a run past its end reads zeros, one
   // past the truncation (into the next m or field) is zeroed below
   const float* base = sp + mem * sp_stride;
   const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(base, (int)((f0 + nf) * (long)S::NRSP * 4));
-  const int off = (int)(((long)(f0 + field) * S::NRSP + 2 * (w0_of(T, m) + 4 * g)) * 4);
-  const uint4 a0 = buffer_load_x4(rs, off, 0), a1 = buffer_load_x4(rs, off, 16);
-  float x[8] = {__uint_as_float(a0.x), __uint_as_float(a0.y), __uint_as_float(a0.z),
-                __uint_as_float(a0.w), __uint_as_float(a1.x), __uint_as_float(a1.y),
-                __uint_as_float(a1.z), __uint_as_float(a1.w)};
+  const int off = (int)(((long)(f0 + field) * S::NRSP + 2 * (w0_of(T, m) + 8 * g)) * 4);
+  uint4 a[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    if (m + 4 * g + q > T) x[2 * q] = x[2 * q + 1] = 0.f;
-  // rows (re/im ri, parity h) = 2 ri + h; values j = 2g (n - m = 4g + h) and
-  // 2g + 1 (4g + 2 + h)
-  float* dst = out + fm * pk_field(T) + pk_seg(T, m) + 2 * g;
+  for (int q = 0; q < 4; ++q) a[q] = buffer_load_x4(rs, off, 16 * q);
+  float x[16];
+  __builtin_memcpy(x, a, sizeof(x));
 #pragma unroll
-  for (int ri = 0; ri < 2; ++ri)
+  for (int q = 0; q < 8; ++q)
+    if (m + 8 * g + q > T) x[2 * q] = x[2 * q + 1] = 0.f;
+  // j = 4g .. 4g + 3: block kb = g / 4; within a whole block j / 4 % 2 = g % 2,
+  // j / 8 = g / 2 % 2, else the two groups of four one after the other
+  const int kb = g >> 2;
+  const int o = (16 * kb + 8 < rw) ? 32 * (g & 1) + 16 * ((g >> 1) & 1) : 16 * (g & 1);
+  float4* dst = (float4*)(out + fm * pk_field(T) + pk_seg(T, m) + 64 * kb + o);
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      *(float2*)(dst + (2 * ri + h) * rw) = make_float2(x[2 * h + ri], x[2 * (2 + h) + ri]);
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int ri = 0; ri < 2; ++ri)  // values n - m = 8g + 2t + h
+      dst[2 * h + ri] = make_float4(x[2 * h + ri], x[4 + 2 * h + ri], x[8 + 2 * h + ri],
+                                    x[12 + 2 * h + ri]);
 }
 
 template <int T>
 static int pack_t(const float* sp, long sps, int f0, int nf, int nmem, float* out,
                   hipStream_t s) {
-  const long total = (long)nmem * nf * (pk_c16(T + 1) / 2);
+  const long total = (long)nmem * nf * (pk_field(T) / 16);
   if (total <= 0) return 0;
   k_pack_sp<T><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(sp, sps, f0, nf, nmem, out);
   return hipGetLastError() == hipSuccess ? 0 : -3;
