@@ -276,11 +276,13 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // elements of the block's table, KPL values per lane.
     constexpr int KPL = (MODE == MODE_F64) ? 4 : 8, EPB = 64 * KPL;
     constexpr int AE = (MODE == MODE_BF16X3) ? 2 : (int)sizeof(R);  // bytes per table element
-    const long abase = (MODE == MODE_BF16X3) ? (long)pb * tab_pb(T) : (long)pb * NM * S::KB * EPB;
-    const int abytes = (MODE == MODE_BF16X3) ? tab_pb(T) * 2 : (NPB - pb) * NM * S::KB * EPB * AE;
+    constexpr int NH = (KIND == INV_UV) ? 2 : 1;  // BF16X3: tables per operand
+    const long abase =
+        (MODE == MODE_BF16X3) ? (long)pb * tab_pb(T) * NH : (long)pb * NM * S::KB * EPB;
+    const int abytes = (MODE == MODE_BF16X3) ? tab_pb(T) * NH * 2 : (NPB - pb) * NM * S::KB * EPB * AE;
     const __amdgpu_buffer_rsrc_t rsA0 = buffer_rsrc((const char*)tabA0 + abase * AE, abytes);
-    const __amdgpu_buffer_rsrc_t rsA1 =
-        buffer_rsrc((const char*)(NTERM == 2 ? tabA1 : tabA0) + abase * AE, abytes);
+    const __amdgpu_buffer_rsrc_t rsA1 = buffer_rsrc(
+        (const char*)(NTERM == 2 && MODE != MODE_BF16X3 ? tabA1 : tabA0) + abase * AE, abytes);
     const int hq = q >> 1, jq = 8 * (q & 1);
     // does this lane hold nonzero table values (its parity is its row's class)
     const bool amine0 = hq == ((c & 1) ^ (table_is_q(KIND == INV_UV ? TQV : a.table) ? 1 : 0));
@@ -311,7 +313,7 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // Legendre phase (T63 inverse 5% faster); at T21 and T42 the pair
     // exchange's VALU work cost more than the load it saves (T42 inverse
     // 1-3% slower)
-    constexpr bool PAIRLOAD = (MODE == MODE_BF16X3) && T >= 63;
+    constexpr bool PAIRLOAD = (MODE == MODE_BF16X3) && KIND == INV_SCALAR && T >= 63;
     // 16-byte table loads per item and term: three bf16 planes (two with
     // PAIRLOAD), or KPL values of 4 or 8 bytes
     constexpr int NA = (MODE == MODE_BF16X3) ? (PAIRLOAD ? 2 : 3) : (KPL * AE) / 16;
@@ -342,18 +344,23 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         // multiplied: two 16-byte loads per term instead of three (a wave's
         // load costs the same however many of its lanes read).  Else each
         // lane loads its three planes, the other class's lanes nothing.
-        const int aso = (tab_seg(T, m) + 768 * kb) * 2;
-        const int w = rw - 16 * kb < 16 ? rw - 16 * kb : 16;  // values per row
+        const int aso = (tab_seg(T, m) + 768 * kb) * NH * 2;
+        const int w = rw - 16 * kb < 16 ? rw - 16 * kb : 16;  // values per row and parity
+        if constexpr (KIND == INV_UV) {
+          // every lane holds values of one of the two tables: three loads that
+          // use all lanes instead of four or six that use half of them (round
+          // trips: T127 L40, 8 members, 625 -> 621 us; T63 L20, 16 members,
+          // 127.4 -> 125.9; T42 unchanged)
+          const int av = inrow ? ((2 * c + hq) * w + jq) * 2 : BUF_NONE;
+#pragma unroll
+          for (int p = 0; p < 3; ++p) a0[p] = buffer_load_x4(rsA0, av, aso + p * w * 64);
+          return;
+        }
         const int av = (c * w + jq) * 2;                          // own row, hi plane
         if constexpr (!PAIRLOAD) {
           const int av0 = (amine0 && inrow) ? av : BUF_NONE;
 #pragma unroll
           for (int p = 0; p < 3; ++p) a0[p] = buffer_load_x4(rsA0, av0, aso + p * w * 32);
-          if (NTERM == 2) {
-            const int av1 = (amine1 && inrow) ? av : BUF_NONE;
-#pragma unroll
-            for (int p = 0; p < 3; ++p) a1[p] = buffer_load_x4(rsA1, av1, aso + p * w * 32);
-          }
           return;
         }
         const int avp = ((c ^ 1) * w + jq) * 2 + w * 32;         // partner's row, mid plane
@@ -363,12 +370,6 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
           const int v2 = (amine0 && inrow) ? avl : BUF_NONE;
           a0[0] = buffer_load_x4(rsA0, v1, aso);
           a0[1] = buffer_load_x4(rsA0, v2, aso);
-        }
-        if (NTERM == 2) {
-          const int v1 = inrow ? (amine1 ? av : avp) : BUF_NONE;
-          const int v2 = (amine1 && inrow) ? avl : BUF_NONE;
-          a1[0] = buffer_load_x4(rsA1, v1, aso);
-          a1[1] = buffer_load_x4(rsA1, v2, aso);
         }
       } else {
         // m > T: n > T loads nothing, and the table offset lies past the
@@ -431,8 +432,12 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
         // the lane holding its row's values: hi and lo as loaded, mid from
         // the partner lane (lane ^ 1); the other lane: zeros
         BF8 ah, am, al;
-        if constexpr (PAIRLOAD) {
-          const uint4 z = {0u, 0u, 0u, 0u};
+        const uint4 z = {0u, 0u, 0u, 0u};
+        if constexpr (KIND == INV_UV) {
+          ah.q = amine ? a[0] : z;
+          am.q = amine ? a[1] : z;
+          al.q = amine ? a[NA - 1] : z;
+        } else if constexpr (PAIRLOAD) {
           const uint4 pm = {quad_perm_u<0xB1>(a[0].x), quad_perm_u<0xB1>(a[0].y),
                             quad_perm_u<0xB1>(a[0].z), quad_perm_u<0xB1>(a[0].w)};
           ah.q = amine ? a[0] : z;
@@ -469,7 +474,7 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // operands of one work item (m, kb)
     struct Frag {
       BFrag b;
-      uint4 a0[NA], a1[NA];
+      uint4 a0[NA], a1[MODE == MODE_BF16X3 ? 1 : NA];
     };
     struct Item {
       int m, kb;
@@ -492,7 +497,8 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
       BF8 bp[3];
       split(use.b, bp);
       mul(use.b, bp, use.a0, amine0, acc1, acc1b);
-      if (NTERM == 2) mul(use.b, bp, use.a1, amine1, acc2, acc2b);
+      if (NTERM == 2)
+        mul(use.b, bp, MODE == MODE_BF16X3 ? use.a0 : use.a1, amine1, acc2, acc2b);
       // (a step past the wave's last item multiplies the zeros it loaded
       // and stores nothing)
       if (next_item(cur).kb == 0 && cur.m <= T) {

@@ -106,16 +106,16 @@ static int build_tables(Tables& t, int ntru, const double* sid, const double* gw
   const long inv_blocks = (long)(t.npair / 8) * (ntru + 1) * t.kbmax;
   const int inv_tabs[] = {TQI, TQJ, TQU, TQV};
   for (int tt : inv_tabs) {
-    const long nbf = (long)(t.npair / 8) * tab_pb(ntru);
-    HIPCK(hipMalloc(&t.inv_bf[tt], sizeof(uint16_t) * nbf));
     HIPCK(hipMalloc(&t.inv_f32[tt], sizeof(float) * 512 * inv_blocks));
     HIPCK(hipMalloc(&t.inv_f64[tt], sizeof(double) * 256 * inv_blocks));
     k_pack_inv<<<(unsigned)((512 * inv_blocks + 255) / 256), 256>>>(
         ntru, t.npair, t.kbmax, tt, t.filt64, t.inv_f32[tt], t.inv_f64[tt]);
     HIPCK(hipGetLastError());
-    const long nth = nbf / 3;
-    k_pack_inv_bf<<<(unsigned)((nth + 255) / 256), 256>>>(ntru, t.npair, tt, t.filt64,
-                                                          t.inv_bf[tt]);
+    if (tt == TQU) continue;
+    const long nbf = (long)(t.npair / 8) * tab_pb(ntru) * (tt == TQV ? 2 : 1);
+    HIPCK(hipMalloc(&t.inv_bf[tt], sizeof(uint16_t) * nbf));
+    k_pack_inv_bf<<<(unsigned)((nbf / 3 + 255) / 256), 256>>>(ntru, t.npair, tt, t.filt64,
+                                                              t.inv_bf[tt]);
     HIPCK(hipGetLastError());
   }
   t.dir_rb = ((ntru + 2) / 2 + 15) / 16;

@@ -78,7 +78,11 @@ __host__ __device__ constexpr int pk_c16(int x) {
 // splits into bf16 planes in registers) in the order in which a wave loads
 // them: blocks of 32 total wavenumbers (16 j) as [j / 4 % 2][j / 8][h][re/im][j %
 // 4], so that each of the two 16-byte loads of a lane takes one whole 128-byte
-// line per field; a last block of 8 j as [j / 4][h][re/im][j % 4]
+// line per field; a last block of 8 j as [j / 4][h][re/im][j % 4].  (As rows of
+// one component and parity a load touched 32 half-used lines: the round trip of
+// T127 L40, 8 members, 715 us against 680, and with the table operand below in
+// load order too 625.  The bf16 planes themselves in memory are one load more
+// per item and slower: 670 against 623.)
 __host__ __device__ constexpr int pk_field(int ntru) { return 4 * pk_c16(ntru + 1); }
 __host__ __device__ constexpr int pk_seg(int ntru, int m) {
   return 4 * (pk_c16(ntru + 1) - pk_c16(ntru + 1 - m));
@@ -87,7 +91,9 @@ __host__ __device__ constexpr int pk_seg(int ntru, int m) {
 // total wavenumbers (16 j, the last 16 or 8), [plane][row = 2 pair +
 // class][j], so that one plane of a block is one run of 256 or 512 bytes; the
 // row holds the parity of its class (h = class for P-type tables, 1 - class for
-// Q-type), the other parity being zero and not stored
+// Q-type), the other parity being zero and not stored.  dv2uv's two tables, qv
+// (Q-type) and qu (P-type), fill each other's zeros: one operand of twice the
+// size, [plane][row][parity h][j], with qu where h = class and qv elsewhere
 __host__ __device__ constexpr int tab_pb(int ntru) { return 48 * pk_c16(ntru + 1); }
 __host__ __device__ constexpr int tab_seg(int ntru, int m) {
   return 48 * (pk_c16(ntru + 1) - pk_c16(ntru + 1 - m));

@@ -40,7 +40,9 @@ struct Tables {
   float* fwd4 = nullptr;      // [8][npair/4][ncsp][4]: filt32 with 4 pairs side by side
   double* skgpsp = nullptr;   // [ntru+1]
   double* skspgp = nullptr;
-  uint16_t* inv_bf[NTAB] = {};  // split-BF16 inverse table operands (3 planes)
+  // split-BF16 inverse table operands (3 planes): qi, qj, and under TQV qv and
+  // qu together
+  uint16_t* inv_bf[NTAB] = {};
   float* inv_f32[NTAB] = {};    // FP32-MFMA inverse table operands
   double* inv_f64[NTAB] = {};   // FP64-MFMA inverse table operands
   float* dir_f32[NTAB] = {};    // MFMA direct table operands (qc, qe, qm, qq)

@@ -192,38 +192,41 @@ __global__ void k_pack_inv(int ntru, int npair, int kbmax, int t, const double* 
 }
 
 // ---- table operand of the split-BF16 inverse (layout in sht_common.h):
-// one thread per (pair block, m, row, j) writing the three planes ----
+// one thread per (pair block, m, row[, parity], j) writing the three planes;
+// t = TQV: both parities of each row, qv's and qu's ----
 __global__ void k_pack_inv_bf(int ntru, int npair, int t, const double* filt64, uint16_t* bf) {
   const int ncsp = (ntru + 1) * (ntru + 2) / 2;
   const long tsz = (long)npair * ncsp;
-  const int per = 16 * pk_c16(ntru + 1);  // (row, j) per pair block
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  const int nh = t == TQV ? 2 : 1;              // parities per row
+  const int per = nh * 16 * pk_c16(ntru + 1);   // (row, parity, j) per pair block
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (long)(npair / 8) * per) return;
   const int pb = (int)(i / per), e = (int)(i % per);
   int lo = 0, hi = ntru;  // the largest m whose segment starts at or before e
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (tab_seg(ntru, mid) / 3 <= e)
+    if (nh * (tab_seg(ntru, mid) / 3) <= e)
       lo = mid;
     else
       hi = mid - 1;
   }
   const int m = lo, rw = pk_rw(ntru, m);
-  // one plane of block kb of m's segment: 16 rows of w values
-  const int r = e - tab_seg(ntru, m) / 3, kb = r >> 8;
+  // one plane of block kb of m's segment: 16 rows of nh w values
+  const int r = e - nh * (tab_seg(ntru, m) / 3), kb = r / (256 * nh), rr = r % (256 * nh);
   const int w = rw - 16 * kb < 16 ? rw - 16 * kb : 16;
-  const int row = (r & 255) / w, j = 16 * kb + (r & 255) % w;
+  const int row = rr / (nh * w), j = 16 * kb + rr % w;
   const int pl = row >> 1, cls = row & 1;
-  const int h = cls ^ (table_is_q(t) ? 1 : 0);
+  const int h = nh == 2 ? (rr / w) & 1 : cls ^ (table_is_q(t) ? 1 : 0);
+  const int tt = nh == 1 ? t : h == cls ? TQU : TQV;
   const int n = m + 2 * j + h;
   const double v =
-      (n <= ntru) ? filt64[t * tsz + (long)(pb * 8 + pl) * ncsp + w0_of(ntru, m) + (n - m)] : 0.0;
+      (n <= ntru) ? filt64[tt * tsz + (long)(pb * 8 + pl) * ncsp + w0_of(ntru, m) + (n - m)] : 0.0;
   uint16_t hh, mm, ll;
   split3_f64(v, hh, mm, ll);
-  uint16_t* o = bf + (long)pb * tab_pb(ntru) + tab_seg(ntru, m) + 768 * kb + (r & 255);
+  uint16_t* o = bf + nh * ((long)pb * tab_pb(ntru) + tab_seg(ntru, m) + 768 * kb) + rr;
   o[0] = hh;
-  o[16 * w] = mm;
-  o[32 * w] = ll;
+  o[16 * nh * w] = mm;
+  o[32 * nh * w] = ll;
 }
 
 // ---- table operand of the MFMA direct transforms (k_dirx_mf): per (m, row
