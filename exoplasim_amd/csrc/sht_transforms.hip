@@ -194,62 +194,73 @@ static int fft_t(const void* tw, int dir, R* a, long lot, int nmem, long mstride
 
 // ---------------------------------------------------------------------------
 // parity-ordered spectral operand of the split-BF16 inverse (layout in
-// sht_common.h): one thread per 8 consecutive coefficients n - m = 8g ..
-// 8g + 7 of one (member, field, m), 64 contiguous bytes read and written.
-// Coefficients past the truncation are zeros.
+// sht_common.h): one thread per 16 bytes, coefficients n - m = 8g + 2t and the
+// next, of which the four lanes t of a quad transpose their 4 x 4 values into
+// the four runs (h, re/im) of j = 4g .. 4g + 3.  Consecutive lanes read
+// consecutive bytes and write whole 64-byte groups; the wavenumber of a group
+// comes from a table.  Coefficients past the truncation are zeros.  (128
+// members of T42 L20: 22.1 us, against 32.7 with 64 bytes per thread, whose loads
+// and stores touch a line per lane, and 23.2 for rows of one component and
+// parity, 32 bytes per thread and m found by bisection.)
 // ---------------------------------------------------------------------------
+template <int T>
+struct PkWave {  // m of each 32 values of a field's operand
+  uint8_t m[pk_field(T) / 32];
+  constexpr PkWave() : m() {
+    for (int k = 0, e = 0; k <= T; ++k)
+      for (int i = 0; i < pk_rw(T, k) / 8; ++i) m[e++] = (uint8_t)k;
+  }
+};
+template <int T>
+__device__ const PkWave<T> pk_wave{};
+
 template <int T>
 __global__ __launch_bounds__(256) void k_pack_sp(const float* sp, long sp_stride, int f0, int nf,
                                                  int nmem, float* out) {
   using S = TS<T>;
-  constexpr int NC = pk_field(T) / 16;  // threads per field: sum over m of rw(m) / 4
+  constexpr int NC = pk_field(T) / 4;  // threads per field
+  static_assert(NC % 4 == 0, "whole quads");
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)nmem * nf * NC) return;
-  const int u = (int)(i % NC);
+  const int u = (int)(i % NC), t = u & 3;
   const long fm = i / NC;
   const int field = (int)(fm % nf), mem = (int)(fm / nf);
-  // the largest m whose segment starts at or before thread u (segment of m:
-  // threads pk_seg(m) / 16 .. + rw(m) / 4)
-  int lo = 0, hi = T;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (pk_seg(T, mid) / 16 <= u)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  const int m = lo, rw = pk_rw(T, m);
-  const int g = u - pk_seg(T, m) / 16;  // coefficients n - m = 8g .. 8g + 7
+  const int m = pk_wave<T>.m[u >> 3], rw = pk_rw(T, m);
+  const int g = (u >> 2) - pk_seg(T, m) / 16;
   // the member's fields as one buffer: a run past its end reads zeros, one
   // past the truncation (into the next m or field) is zeroed below
   const float* base = sp + mem * sp_stride;
   const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(base, (int)((f0 + nf) * (long)S::NRSP * 4));
-  const int off = (int)(((long)(f0 + field) * S::NRSP + 2 * (w0_of(T, m) + 8 * g)) * 4);
-  uint4 a[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) a[q] = buffer_load_x4(rs, off, 16 * q);
-  float x[16];
-  __builtin_memcpy(x, a, sizeof(x));
-#pragma unroll
-  for (int q = 0; q < 8; ++q)
-    if (m + 8 * g + q > T) x[2 * q] = x[2 * q + 1] = 0.f;
-  // j = 4g .. 4g + 3: block kb = g / 4; within a whole block j / 4 % 2 = g % 2,
-  // j / 8 = g / 2 % 2, else the two groups of four one after the other
+  const int n = m + 8 * g + 2 * t;
+  const int off = (int)(((long)(f0 + field) * S::NRSP + 2 * (w0_of(T, m) + n - m)) * 4);
+  const uint4 a = buffer_load_x4(rs, off, 0);
+  unsigned x0 = a.x, x1 = a.y, x2 = a.z, x3 = a.w;
+  if (n > T) x0 = x1 = 0u;
+  if (n + 1 > T) x2 = x3 = 0u;
+  // 4 x 4 transpose over the quad: lanes t ^ 1, then t ^ 2
+  {
+    const bool o = t & 1;
+    const unsigned s0 = quad_perm_u<0xB1>(o ? x0 : x1), s1 = quad_perm_u<0xB1>(o ? x2 : x3);
+    x0 = o ? s0 : x0, x1 = o ? x1 : s0;
+    x2 = o ? s1 : x2, x3 = o ? x3 : s1;
+  }
+  {
+    const bool o = t & 2;
+    const unsigned s0 = quad_perm_u<0x4E>(o ? x0 : x2), s1 = quad_perm_u<0x4E>(o ? x1 : x3);
+    x0 = o ? s0 : x0, x2 = o ? x2 : s0;
+    x1 = o ? s1 : x1, x3 = o ? x3 : s1;
+  }
+  // block kb = g / 4; within a whole block j / 4 % 2 = g % 2, j / 8 = g / 2 % 2,
+  // else the two groups of four one after the other
   const int kb = g >> 2;
   const int o = (16 * kb + 8 < rw) ? 32 * (g & 1) + 16 * ((g >> 1) & 1) : 16 * (g & 1);
-  float4* dst = (float4*)(out + fm * pk_field(T) + pk_seg(T, m) + 64 * kb + o);
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int ri = 0; ri < 2; ++ri)  // values n - m = 8g + 2t + h
-      dst[2 * h + ri] = make_float4(x[2 * h + ri], x[4 + 2 * h + ri], x[8 + 2 * h + ri],
-                                    x[12 + 2 * h + ri]);
+  *(uint4*)(out + fm * pk_field(T) + pk_seg(T, m) + 64 * kb + o + 4 * t) = uint4{x0, x1, x2, x3};
 }
 
 template <int T>
 static int pack_t(const float* sp, long sps, int f0, int nf, int nmem, float* out,
                   hipStream_t s) {
-  const long total = (long)nmem * nf * (pk_field(T) / 16);
+  const long total = (long)nmem * nf * (pk_field(T) / 4);
   if (total <= 0) return 0;
   k_pack_sp<T><<<(unsigned)((total + 255) / 256), 256, 0, s>>>(sp, sps, f0, nf, nmem, out);
   return hipGetLastError() == hipSuccess ? 0 : -3;
