@@ -12,7 +12,7 @@
 //
 // calcgp is a column computation of pointwise terms, prefix sums over the
 // levels and two matrix products over the levels (c and g).  A block takes 64
-// grid points, or one latitude row in gridpointa, and all levels; its 8 waves
+// grid points, or one latitude row in gridpointa, and all levels; its 4 to 10 waves
 // share the levels, a lane owning the same points at each.  What a level needs
 // of the others -- v . grad ln ps, the divergence and the humidity term --
 // meets in LDS, and c and g are read through scalar loads (a wave's lanes all
@@ -52,16 +52,17 @@ struct CalcgpPtrs {
 // the wave that computed a level transforms it in LDS rows of its own, two
 // real rows per complex FFT and GpCfg::NFB FFTs at a time, so the grid values
 // of those fields never reach HBM.
-template <typename R, int ROW>
+template <typename R, int ROW, int WAVES = 8>
 struct GpCfg {
   static constexpr int PPL = ROW ? ROW / 64 : 1;  // points per lane
   static constexpr int P = 64 * PPL;              // points per block
-  static constexpr int W = 8;                     // waves per block
+  static constexpr int W = WAVES;                 // waves per block
   // FFTs at a time: all five of a level, but two in FP64 on rows of 128, whose
   // five would leave the level arrays too little LDS
   static constexpr int NFB = sizeof(R) == 4 || ROW <= 64 ? 5 : 2;
   static constexpr int NP = ROW + ROW / 32;  // padded FFT row
-  static constexpr int WPS = (sizeof(R) == 4 || ROW <= 64) ? 4 : 2;  // waves per SIMD asked for
+  // waves per SIMD asked for
+  static constexpr int WPS = W > 8 ? 3 : (sizeof(R) == 4 || ROW <= 64) ? 4 : 2;
   static size_t lds(int nlev) {
     return sizeof(R) * 3 * nlev * P + (ROW ? sizeof(C2<R>) * (W * NFB * NP + ROW) : 0);
   }
@@ -74,12 +75,12 @@ using Uni = __attribute__((address_space(4))) const R*;
 // With sid (gridpointa) rcsq = 1 / cos^2 comes from the Gaussian abscissas, as
 // the model sets it up (src/plasim.f90:1897 csq = 1 - sid^2 in the real kind,
 // :205), and is written to rcsq_out; else it is read.
-template <typename R, int ROW>
-__global__ __launch_bounds__(512, (GpCfg<R, ROW>::WPS)) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, int n, int nhor,
+template <typename R, int ROW, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_calcgp(CalcgpPtrs<R> f, DynVert<R> v, int n, int nhor,
                                                 long mstride, int nqspec, int exp_gp,
                                                 const double* sid, int nlon, R* rcsq_out,
                                                 const C2<R>* tw) {
-  using C = GpCfg<R, ROW>;
+  using C = GpCfg<R, ROW, WAVES>;
   using R2 = R __attribute__((ext_vector_type(2)));
   constexpr int PPL = C::PPL, P = C::P, W = C::W;
   extern __shared__ __align__(16) char smem[];
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(512, (GpCfg<R, ROW>::WPS)) void k_calcgp(CalcgpPtrs
   }
   if constexpr (ROW > 0) {
     C2<R>* tws = (C2<R>*)(cr + n * P) + W * C::NFB * C::NP;
-    for (int k = threadIdx.x; k < ROW; k += 512) tws[k] = C2<R>{tw[k].x, -tw[k].y};
+    for (int k = threadIdx.x; k < ROW; k += 64 * W) tws[k] = C2<R>{tw[k].x, -tw[k].y};
   }
 
   // ---- zvgpg = rcsq (u d/dlambda + v d/dmu) ln ps, the divergence, and the
@@ -462,21 +463,40 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
   p.guq = (R*)f->guq;
   p.gvq = (R*)f->gvq;
   const DynVert<R> v = vert_of<R>(d);
-  auto launch = [&](auto kern, int points, size_t lds) -> int {
+  auto launch = [&](auto kern, int points, int waves, size_t lds) -> int {
     if (lds > 65536 &&
         hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
       return EXO_ERR_LAUNCH;
     const dim3 grid((unsigned)((nhor + points - 1) / points), (unsigned)nmem);
-    kern<<<grid, 512, lds, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp, sid, nlon, (R*)rcsq_out,
+    kern<<<grid, 64 * waves, lds, s>>>(p, v, d->nlev, nhor, ms, nqspec, exp_gp, sid, nlon, (R*)rcsq_out,
                                 (const C2<R>*)tw);
     return hipGetLastError() == hipSuccess ? EXO_OK : EXO_ERR_LAUNCH;
   };
   const int n = d->nlev;
+  // Waves per block of a row kernel.  Up to one block per CU its own chain of
+  // levels is the time, and 10 waves shorten it (T21 L10 FP64, one member,
+  // gridpointa 28.8 -> 26.6 us; T42 L13 FP32 42.9 -> 40.9), but in FP64 on rows
+  // of 128, whose registers do not allow it (T42 L10 49 -> 62).  Above, FP64
+  // takes 4: twice the blocks fit a CU's LDS, and the levels come out evenly
+  // (T42 L20, 8 members, 133.5 -> 125.4; T21 L10, 32 members, 73.4 -> 67.1; FP32
+  // T42 L20, 32 members, 235.6 against 244.4).
+  const bool few = (long)(nhor / (nlon > 0 ? nlon : 1)) * nmem <= 256;
   switch (tw ? nlon : 0) {
-    case 64: return launch(k_calcgp<R, 64>, 64, GpCfg<R, 64>::lds(n));
-    case 128: return launch(k_calcgp<R, 128>, 128, GpCfg<R, 128>::lds(n));
-    default: return launch(k_calcgp<R, 0>, 64, GpCfg<R, 0>::lds(n));
+    case 64:
+      if (few) return launch(k_calcgp<R, 64, 10>, 64, 10, GpCfg<R, 64, 10>::lds(n));
+      if constexpr (sizeof(R) == 8)
+        return launch(k_calcgp<R, 64, 4>, 64, 4, GpCfg<R, 64, 4>::lds(n));
+      else
+        return launch(k_calcgp<R, 64, 8>, 64, 8, GpCfg<R, 64>::lds(n));
+    case 128:
+      if constexpr (sizeof(R) == 4) {
+        if (few) return launch(k_calcgp<R, 128, 10>, 128, 10, GpCfg<R, 128, 10>::lds(n));
+      } else {
+        if (!few) return launch(k_calcgp<R, 128, 4>, 128, 4, GpCfg<R, 128, 4>::lds(n));
+      }
+      return launch(k_calcgp<R, 128, 8>, 128, 8, GpCfg<R, 128>::lds(n));
+    default: return launch(k_calcgp<R, 0, 8>, 64, 8, GpCfg<R, 0>::lds(n));
   }
 }
 

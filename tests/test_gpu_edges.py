@@ -356,3 +356,35 @@ def test_emulate_row_major_weights(gpu, ncol):
                                    vp(flags[1].data_ptr()), None) == 0
     torch.cuda.synchronize()
     assert torch.equal(h, heat) and torch.equal(o, olr) and torch.equal(*flags)
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 3, 9), (21, 11, 10), (42, 4, 5), (42, 21, 6)])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+def test_gridpointa_many_members(oracle, gpu, ntru, nlev, nmem, mode):
+    """grids of more than one block per CU, whose levels a block shares among
+    fewer waves, against each member alone (more waves, against the oracle
+    above): the same sums in the same order, so that only the contraction of
+    products and sums can differ, an ulp per term of sums that cancel by less
+    than 1e2: 1e-12 and 2e-5."""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.dynamics import Dynamics
+
+    print(f"gridpointa T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    plan = sht.Plan(ntru)
+    dyn = Dynamics.from_vertical(_vertical(oracle, nlev), *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, nmem, mode)
+    st.copy_(torch.from_numpy(np.stack([gridpointa_state(ntru, nlev, 0.9 + 0.02 * k)
+                                        for k in range(nmem)])).to(st.dtype))
+    dyn.gridpointa(plan, mode, st, work, tend)
+    st1, work1, tend1 = dyn.alloc_gridpointa(plan, 1, mode)
+    tol = 1e-12 if mode == "f64" else 2e-5
+    for k in (0, nmem - 1):
+        st1.copy_(st[k:k + 1])
+        dyn.gridpointa(plan, mode, st1, work1, tend1)
+        torch.cuda.synchronize()
+        for a, b in ((tend[k], tend1[0]), (work[k], work1[0])):
+            assert rel(a.double().cpu().numpy(), b.double().cpu().numpy()) < tol
+    dyn.close()
+    plan.close()
