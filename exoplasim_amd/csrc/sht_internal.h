@@ -19,7 +19,8 @@ __global__ void k_pack_inv(int ntru, int npair, int kbmax, int t, const double* 
                            float* f32, double* f64);
 __global__ void k_pack_inv_bf(int ntru, int npair, int t, const double* filt64, uint16_t* bf);
 __global__ void k_pack_dir(int ntru, int npair, int rb, int t, const double* filt64, float* out);
-__global__ void k_pack_fwd4(int npair, int ncsp, const float* filt32, float* fwd4);
+template <typename R>
+__global__ void k_pack_fwd(int npair, int ncsp, const R* filt, R* out);
 __global__ void k_twiddle(int n, double* tw64, float* tw32);
 
 // Which inverse transform a launch performs.
@@ -38,6 +39,7 @@ struct Tables {
   double* filt64 = nullptr;   // [8][npair][ncsp] filter folded in
   float* filt32 = nullptr;
   float* fwd4 = nullptr;      // [8][npair/4][ncsp][4]: filt32 with 4 pairs side by side
+  double* fwd2 = nullptr;     // [8][npair/2][ncsp][2]: filt64 with 2 pairs side by side
   double* skgpsp = nullptr;   // [ntru+1]
   double* skspgp = nullptr;
   // split-BF16 inverse table operands (3 planes): qi, qj, and under TQV qv and

@@ -250,21 +250,25 @@ __global__ void k_pack_dir(int ntru, int npair, int rb, int t, const double* fil
                        : 0.0f;
 }
 
-// ---- the FP32 tables of the fused direct transform (k_fwd): 4 latitude
-// pairs side by side, [t][pair / 4][w][pair % 4], so that a lane summing
-// coefficient w reads 4 pairs in one 16-byte load and the lanes of a wave
-// (consecutive w) read one contiguous run ----
-__global__ void k_pack_fwd4(int npair, int ncsp, const float* filt32, float* fwd4) {
+// ---- the tables of the direct transform (k_fwd): G latitude pairs of 16
+// bytes together side by side (FP32: 4, FP64: 2), [t][pair / G][w][pair % G],
+// so that a lane summing coefficient w reads G pairs in one 16-byte load and
+// the lanes of a wave (consecutive w) read one contiguous run ----
+template <typename R>
+__global__ void k_pack_fwd(int npair, int ncsp, const R* filt, R* out) {
+  constexpr int G = 16 / sizeof(R);
   const long total = (long)NTAB * npair * ncsp;
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (i >= total) return;
-  const int u = (int)(i % 4);
-  const int w = (int)((i / 4) % ncsp);
-  const long tg = i / (4L * ncsp);  // t * (npair / 4) + pair group
-  const int g = (int)(tg % (npair / 4));
-  const int t = (int)(tg / (npair / 4));
-  fwd4[i] = filt32[((long)t * npair + 4 * g + u) * ncsp + w];
+  const int u = (int)(i % G);
+  const int w = (int)((i / G) % ncsp);
+  const long tg = i / ((long)G * ncsp);  // t * (npair / G) + pair group
+  const int g = (int)(tg % (npair / G));
+  const int t = (int)(tg / (npair / G));
+  out[i] = filt[((long)t * npair + G * g + u) * ncsp + w];
 }
+template __global__ void k_pack_fwd<float>(int, int, const float*, float*);
+template __global__ void k_pack_fwd<double>(int, int, const double*, double*);
 
 // twiddles e^{+2 pi i k/N} in FP64 and FP32
 __global__ void k_twiddle(int n, double* tw64, float* tw32) {
