@@ -1,4 +1,4 @@
-// rad_mlp.hip -- forward and backward kernels of the long-wave emulator MLP
+// rad_mlp.hip -- inference and per-layer training kernels of the long-wave emulator MLP
 // (43 -> 256 -> 256 -> 256 -> 21, GELU), BF16 operands on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation.
 //

@@ -364,8 +364,9 @@ extern "C" int exo_sht_inverse_uv(exo_sht_plan_t p, int mode, int nmem, const vo
 // truncations, or null for the plan's own, grown as needed)
 static int direct_impl(exo_sht_plan_t p, int mode, bool fused, int nmem, const void* in,
                        long in_stride, int src0, void* sp, long sp_stride, int dst0, int nfield,
-                       hipStream_t s, void* scr = nullptr, size_t sbytes = 0) {
+                       hipStream_t s, void* scr = nullptr, size_t sbytes = 0, int nrule = 0) {
   FwdArgs a{};
+  a.nrule = nrule;
   a.in = in;
   a.sp = sp;
   a.in_stride = in_stride;
@@ -396,7 +397,7 @@ extern "C" int exo_sht_direct(exo_sht_plan_t p, int mode, int nmem, const void* 
 }
 
 static int inverse_all_impl(exo_sht_plan_t p, int mode, int nmem, int nlev, const void* sp_in,
-                            void* gp, hipStream_t s, void* pkbuf = nullptr);
+                            void* gp, hipStream_t s, void* pkbuf = nullptr, int nrule = 0);
 
 extern "C" int exo_sht_roundtrip(exo_sht_plan_t p, int mode, int nmem, int nlev, const void* sp_in,
                                  void* gp, void* sp_out, void* stream) {
@@ -470,9 +471,9 @@ extern "C" int exo_sht_roundtrip_noalloc(exo_sht_plan_t p, int mode, int nmem, i
     char* pk = p->na_scratch;
     char* fwd = p->na_scratch + na_pk_off(t, mode, nfl, c);
     const size_t fwd_bytes = EXO_NOALLOC_SCRATCH_BYTES - na_pk_off(t, mode, nfl, c);
-    int rc = inverse_all_impl(p, mode, c, nlev, spi, g, s, pk);
+    int rc = inverse_all_impl(p, mode, c, nlev, spi, g, s, pk, nmem);
     if (rc) return rc;
-    rc = direct_impl(p, mode, true, c, g, gps, 0, spo, sps, 0, nfl, s, fwd, fwd_bytes);
+    rc = direct_impl(p, mode, true, c, g, gps, 0, spo, sps, 0, nfl, s, fwd, fwd_bytes, nmem);
     if (rc) return rc;
   }
   return EXO_OK;
@@ -501,7 +502,7 @@ extern "C" int exo_sht_get_tiles(exo_sht_plan_t p, int mode, int* vars) {
 // the inverse half of exo_sht_roundtrip: pre-split (split-BF16) and the
 // three inverse transforms in one launch
 static int inverse_all_impl(exo_sht_plan_t p, int mode, int nmem, int nlev, const void* sp_in,
-                            void* gp, hipStream_t s, void* pkbuf) {
+                            void* gp, hipStream_t s, void* pkbuf, int nrule) {
   const Tables& t = p->tb;
   const int nfl = 3 * nlev + 1;
   const long sps = (long)nfl * 2 * t.ncsp;
@@ -517,6 +518,7 @@ static int inverse_all_impl(exo_sht_plan_t p, int mode, int nmem, int nlev, cons
   aq.nmem = nmem;
   aq.plavor = t.plavor;
   aq.var = p->inv_var[mode];
+  aq.nrule = nrule;
   aq.bpk = pk.bpk;
   aq.bpk_stride = pk.bpk_stride;
   aq.bpk_f0 = pk.bpk_f0;

@@ -66,6 +66,7 @@ struct InvArgs {
   int vor0, div0, u0, v0, nlev;         // INV_UV
   double plavor;
   int var;          // tile variant (InvCfg / FwdCfg), -1: by the size of the call
+  int nrule;        // members of the whole call, of which this launch runs nmem (0: nmem)
   int dlam;         // INV_SCALAR: times i m before the FFT (d/dlambda)
   // MODE_BF16X3: the parity-ordered spectral operand (launch_pack) of
   // fields [bpk_f0, ...), bpk_stride floats per member
@@ -89,6 +90,7 @@ struct FwdArgs {
   int src0, dst0, nfield;
   int table;        // TQC
   int var;          // tile variant (InvCfg / FwdCfg), -1: by the size of the call
+  int nrule;        // members of the whole call, of which this launch runs nmem (0: nmem)
 };
 
 // One term of a multi-input direct transform: out_o[oc] += sign * t * X_in[ic]

@@ -150,10 +150,24 @@ static int inv_auto(long nblk3) {
   return nblk3 <= (two ? 512 : 256) ? 3 : 2;
 }
 
+// blocks at V = 3 of the call that a launch belongs to: a call that runs its
+// members in chunks uses the same tiles, and returns the same bits, as one
+// launch of them all
+template <int T, int MODE>
+static long inv_rule(InvArgs a) {
+  if (a.nrule > 0) a.nmem = a.nrule;
+  return inv_items<T, MODE, 3>(a);
+}
+template <int T, int MODE>
+static long fwd_rule(FwdArgs a) {
+  if (a.nrule > 0) a.nmem = a.nrule;
+  return fwd_items<T, MODE, 3>(a);
+}
+
 // the unfused (drop-in) transforms always use the default tiles
 template <int T, int MODE>
 static int inv_t(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s) {
-  const int v = !fused ? 0 : a.var >= 0 ? a.var : inv_auto<T, MODE>(inv_items<T, MODE, 3>(a));
+  const int v = !fused ? 0 : a.var >= 0 ? a.var : inv_auto<T, MODE>(inv_rule<T, MODE>(a));
   if (v == 1) return inv_tv<T, MODE, 1>(tb, fused, a, s);
   if (v == 2) return inv_tv<T, MODE, 2>(tb, fused, a, s);
   if (v == 3) return inv_tv<T, MODE, 3>(tb, fused, a, s);
@@ -206,9 +220,9 @@ template <int T, int MODE>
 static int inv_rt_t(const Tables& tb, const InvArgs& aq, const InvArgs* aj, int nj,
                     const InvArgs& au, hipStream_t s) {
   const int v = aq.var >= 0 ? aq.var
-                            : inv_auto<T, MODE>(inv_items<T, MODE, 3>(aq) +
-                                                nj * inv_items<T, MODE, 3>(aj[0]) +
-                                                inv_items<T, MODE, 3>(au));
+                            : inv_auto<T, MODE>(inv_rule<T, MODE>(aq) +
+                                                nj * inv_rule<T, MODE>(aj[0]) +
+                                                inv_rule<T, MODE>(au));
   if (v == 1) return inv_rt_tv<T, MODE, 1>(tb, aq, aj, nj, au, s);
   if (v == 2) return inv_rt_tv<T, MODE, 2>(tb, aq, aj, nj, au, s);
   if (v == 3) return inv_rt_tv<T, MODE, 3>(tb, aq, aj, nj, au, s);
@@ -264,7 +278,7 @@ static int fwd_auto(long nblk3) {
 template <int T, int MODE>
 static int fwd_t(const Tables& tb, bool fused, const FwdArgs& a, void* scratch, size_t sbytes,
                  hipStream_t s) {
-  const int v = !fused ? 0 : a.var >= 0 ? a.var : fwd_auto<T, MODE>(fwd_items<T, MODE, 3>(a));
+  const int v = !fused ? 0 : a.var >= 0 ? a.var : fwd_auto<T, MODE>(fwd_rule<T, MODE>(a));
   if (v == 1) return fwd_tv<T, MODE, 1>(tb, fused, a, scratch, sbytes, s);
   if (v == 2) return fwd_tv<T, MODE, 2>(tb, fused, a, scratch, sbytes, s);
   if (v == 3) return fwd_tv<T, MODE, 3>(tb, fused, a, scratch, sbytes, s);

@@ -388,3 +388,24 @@ def test_gridpointa_many_members(oracle, gpu, ntru, nlev, nmem, mode):
             assert rel(a.double().cpu().numpy(), b.double().cpu().numpy()) < tol
     dyn.close()
     plan.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem,mode", [(63, 10, 33, "f64"), (42, 7, 300, "bf16x3")])
+def test_noalloc_last_chunk(gpu, ntru, nlev, nmem, mode):
+    """the no-allocation round trip of an untuned plan where the last chunk of
+    members is small enough for other tiles than the whole call's: it uses
+    the call's, so its outputs are the round trip's to the last bit"""
+    import torch
+
+    from exoplasim_amd import sht
+
+    print(f"noalloc T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    plan = sht.Plan(ntru)
+    x, gp, y = plan.alloc_roundtrip(nmem, nlev, mode)
+    x.normal_()
+    plan.roundtrip(mode, x, gp, y, nlev)
+    gp2, y2 = torch.full_like(gp, float("nan")), torch.full_like(y, float("nan"))
+    plan.roundtrip_noalloc(mode, x, gp2, y2, nlev)
+    torch.cuda.synchronize()
+    assert torch.equal(gp, gp2) and torch.equal(y, y2)
+    plan.close()
