@@ -2,7 +2,7 @@
 
 Forward and backward of the 43 -> 256 -> 256 -> 256 -> 21 GELU network in
 numpy float64, rounding to bfloat16 exactly where the GPU kernels
-(exoplasim_amd/csrc/rad_mlp.hip) hold bf16 values: the layer inputs, the
+(exoplasim_amd/csrc/rad_mlp.hip, rad_train.hip) hold bf16 values: the layer inputs, the
 weights, the activations and the back-propagated pre-activation gradients.
 Sums are exact-order-independent FP64, so the comparison measures the
 kernels' FP32 accumulation plus any bf16 rounding flips.
