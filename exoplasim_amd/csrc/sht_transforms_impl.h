@@ -53,6 +53,19 @@ __global__ __launch_bounds__((InvCfg<T, MODE, V>::NT)) void k_inv_rt(InvArgs aq,
       mem = x * M + (i - nu) / ns;
       r = (i - nu) % ns;
     }
+  } else if (T == 127 && aq.nmem < 8) {
+    // fewer members than XCDs: contiguous ranges of a member's blocks would give
+    // some XCDs only dv2uv items (two terms), others only scalar ones.  The long
+    // dv2uv items first, dealt out over all XCDs (round trips: FP64 L15, 2
+    // members, 262 -> 242 us; BF16X3 L40, 3 members, 248 -> 237; gridpointa FP64
+    // L10, one member, 232 -> 218.  At T63 and T42, whose launches last a few
+    // rounds of blocks at most, the ranges' locality counts for more: T63 L30
+    // FP64, 5 members, 159 against 165.)
+    const int i = blockIdx.x, nu = NPB * gu, ns = NPB * (gq + gj);
+    const bool uv = i < aq.nmem * nu;
+    const int k = uv ? i : i - aq.nmem * nu, n = uv ? nu : ns;
+    mem = k / n;
+    r = k - mem * n + (uv ? ns : 0);
   } else {
     const int b = xcd_block(blockIdx.x, gridDim.x);
     mem = b / per;
