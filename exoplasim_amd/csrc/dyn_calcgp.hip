@@ -5,7 +5,6 @@
 //             vertical velocity (sigma-dot), the nonlinear tendencies gtn,
 //             gqn, guz, gvz, the geopotential term gphi and dw; with it the
 //             products of gridpointa (src/plasim.f90:2436-2446) and, on
-//             request, gp = exp(gp) (:2434)
 //             request, gp = exp(gp) (:2434); in gridpointa also gp2fc of the
 //             fields that go to the direct transforms
 //   k_gpmt    the Fourier-space d/dlambda of ln(ps) (src/plasim.f90:2425-2430)
@@ -49,18 +48,24 @@ struct CalcgpPtrs {
 // ROW = 0: calcgp on the grid, 64 points per block.  ROW = N (64, 128):
 // gridpointa on rows of N longitudes, one row per block; the nine tendency fields of a
 // level and gvp then leave as the Fourier coefficients of their rows (gp2fc):
-// the wave that computed a level transforms it in LDS rows of its own, two
-// real rows per complex FFT and GpCfg::NFB FFTs at a time, so the grid values
-// of those fields never reach HBM.
+// the wave that computed a level transforms it in LDS rows of its own,
+// GpCfg::NFB rows at a time, so the grid values of those fields never reach
+// HBM.  Each real row is one complex FFT of half its length, its even points
+// the real and its odd points the imaginary parts: the rounding of a field is
+// then that of its own row.  (Two fields of a level in one FFT of full length
+// left the smaller one the rounding of the larger: the moisture tendency of
+// levels with 1e-4 of the humidity 3 digits, and a NaN in it reached the
+// temperature's.)
 template <typename R, int ROW, int WAVES = 8>
 struct GpCfg {
   static constexpr int PPL = ROW ? ROW / 64 : 1;  // points per lane
   static constexpr int P = 64 * PPL;              // points per block
   static constexpr int W = WAVES;                 // waves per block
-  // FFTs at a time: all five of a level, but two in FP64 on rows of 128, whose
-  // five would leave the level arrays too little LDS
-  static constexpr int NFB = sizeof(R) == 4 || ROW <= 64 ? 5 : 2;
-  static constexpr int NP = ROW + ROW / 32;  // padded FFT row
+  // rows at a time: all ten of a level, but four in FP64 on rows of 128, whose
+  // ten would leave the level arrays too little LDS
+  static constexpr int NFB = sizeof(R) == 4 || ROW <= 64 ? 10 : 4;
+  static constexpr int H = ROW / 2, NP = H + H / 32;  // FFT length, padded FFT row
+  static constexpr int R0 = H == 64 && NFB == 10 ? 16 : 8;  // first radix: fewest idle lanes
   // waves per SIMD asked for
   static constexpr int WPS = W > 8 ? 3 : (sizeof(R) == 4 || ROW <= 64) ? 4 : 2;
   static size_t lds(int nlev) {
@@ -88,9 +93,14 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
   R* cr = (R*)(zg + n * P);    // [level][point]: humidity term of the virtual temperature
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // where a lane's points lie in a level of zg and cr: side by side, but a wave
+  // apart where 32 bytes per lane would put two lanes on each LDS bank
+  const int l0 = PPL > 1 && sizeof(R) == 4 ? PPL * lane : lane;
+  constexpr int LS = PPL > 1 && sizeof(R) == 4 ? 1 : 64;
   // Every field is addressed by a wave-uniform base (member, level, block) and
-  // the lane's point within the block, so that the address arithmetic is
-  // scalar.  The lanes past the last point repeat it and store nothing.
+  // the lane's PPL consecutive points within the block, so that the address
+  // arithmetic is scalar.  The lanes past the last point repeat it and store
+  // nothing.
   const int h0 = blockIdx.x * P;
   const long mo = (long)blockIdx.y * mstride + h0;
   unsigned pt = lane;
@@ -99,13 +109,19 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
     live = h0 + lane < nhor;
     if (!live) pt = nhor - 1 - h0;
   }
-  auto at = [&](const R* p, int j, int i) -> R {
-    const R* b = p + (mo + (long)j * nhor + 64 * i);
-    return b[pt];
+  struct V {
+    R v[PPL];
+  } __attribute__((packed, aligned(sizeof(R))));
+  auto at = [&](const R* p, int j, R (&x)[PPL]) {
+    const V u = ((const V*)(p + (mo + (long)j * nhor)))[pt];
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) x[i] = u.v[i];
   };
-  auto put = [&](R* p, int j, int i, R x) {
-    R* b = p + (mo + (long)j * nhor + 64 * i);
-    if (live) b[pt] = x;
+  auto put = [&](R* p, int j, const R (&x)[PPL]) {
+    V u;
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) u.v[i] = x[i];
+    if (live) ((V*)(p + (mo + (long)j * nhor)))[pt] = u;
   };
   const Uni<R> dsig = (Uni<R>)v.dsigma, sigh = (Uni<R>)v.sigmah, rdsig = (Uni<R>)v.rdsig;
   const Uni<R> t0v = (Uni<R>)v.t0, t01 = (Uni<R>)v.t01s2, tkp = (Uni<R>)v.tkp;
@@ -113,16 +129,15 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
 
   // ---- surface fields ----
   R gpm[PPL], gpj[PPL], rcsq[PPL], gp[PPL];
+  at(f.gpm, 0, gpm);
+  at(f.gpj, 0, gpj);
+  at(f.gp, 0, gp);
+  if (!sid) at(f.rcsq, 0, rcsq);
 #pragma unroll
   for (int i = 0; i < PPL; ++i) {
-    gpm[i] = at(f.gpm, 0, i);
-    gpj[i] = at(f.gpj, 0, i);
-    gp[i] = at(f.gp, 0, i);
     if (sid) {
-      const double x = sid[(h0 + (int)pt + 64 * i) / nlon];
+      const double x = sid[(h0 + PPL * (int)pt + i) / nlon];
       rcsq[i] = R(1) / (R)(1.0 - x * x);
-    } else {
-      rcsq[i] = at(f.rcsq, 0, i);
     }
     if (exp_gp) gp[i] = exp(gp[i]);
   }
@@ -139,24 +154,21 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
   // the cancellation: corr = (gt + t0)(1/rdbrv - 1) zq, ztv1 = gt + corr, ztv1
   // - gt = corr and ztv2 = (gt + corr - t0 adv zq) / (1 + adv zq). ----
   for (int j = w; j < n; j += W) {
+    R gu[PPL], gv[PPL], gd[PPL], gt[PPL], zq[PPL];
+    at(f.gu, j, gu), at(f.gv, j, gv), at(f.gd, j, gd), at(f.gt, j, gt);
+    at(nqspec == 1 ? f.gq : f.dq, j, zq);
 #pragma unroll
     for (int i = 0; i < PPL; ++i) {
-      const R gu = at(f.gu, j, i), gv = at(f.gv, j, i), gd = at(f.gd, j, i);
-      const R gt = at(f.gt, j, i);
-      R zq = (nqspec == 1) ? at(f.gq, j, i) / gp[i] : at(f.dq, j, i);
-      zq = zq > R(0) ? zq : R(0);
-      zg[j * P + lane + 64 * i] = R2{rcsq[i] * (gu * gpm[i] + gv * gpj[i]), gd};
-      cr[j * P + lane + 64 * i] = (gt + t0v[j]) * (qfac * zq);
+      if (nqspec == 1) zq[i] = zq[i] / gp[i];
+      zq[i] = zq[i] > R(0) ? zq[i] : R(0);
+      zg[j * P + l0 + LS * i] = R2{rcsq[i] * (gu[i] * gpm[i] + gv[i] * gpj[i]), gd[i]};
+      cr[j * P + l0 + LS * i] = (gt[i] + t0v[j]) * (qfac * zq[i]);
     }
   }
   __syncthreads();
-  if (w == 0) {
-    // (after the barrier: every wave has read gp)
-#pragma unroll
-    for (int i = 0; i < PPL; ++i) {
-      if (exp_gp) put(f.gp, 0, i, gp[i]);
-      if (sid) put(rcsq_out, 0, i, rcsq[i]);
-    }
+  if (w == 0) {  // (after the barrier: every wave has read gp)
+    if (exp_gp) put(f.gp, 0, gp);
+    if (sid) put(rcsq_out, 0, rcsq);
   }
 
   // ---- this wave's levels [j0, j1) ----
@@ -174,17 +186,14 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
 #pragma unroll
     for (int i = 0; i < PPL; ++i) {
       if (k == j0) rz[i] = tot[i], rv[i] = vp[i];
-      const R2 x = zg[k * P + lane + 64 * i];
+      const R2 x = zg[k * P + l0 + LS * i];
       tot[i] = tot[i] + dk * x.y;
       vp[i] = vp[i] + dk * x.x;
     }
   }
 #pragma unroll
   for (int i = 0; i < PPL; ++i) tot[i] = tot[i] + vp[i];
-  if (ROW == 0 && w == 0) {
-#pragma unroll
-    for (int i = 0; i < PPL; ++i) put(f.gvp, 0, i, vp[i]);
-  }
+  if (ROW == 0 && w == 0) put(f.gvp, 0, vp);
   // the terms at the interface above level j (gtd, gqm, gud, gvd of level
   // j - 1, and tim = t01s2 (sigmah gvp - the sum of zvgpg dsigma)), carried one
   // level on; zero above the top and below the bottom
@@ -192,13 +201,14 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
   R gtd_m[PPL], gqm_m[PPL], gud_m[PPL], gvd_m[PPL], tim[PPL];
   {
     const int jm = j0 > 0 ? j0 - 1 : 0;
+    R gtm[PPL], gqm[PPL], gum[PPL], gvm[PPL];
+    at(f.gt, j0, gt), at(f.gq, j0, gq), at(f.gu, j0, gu), at(f.gv, j0, gv);
+    at(f.gt, jm, gtm), at(f.gq, jm, gqm), at(f.gu, jm, gum), at(f.gv, jm, gvm);
 #pragma unroll
     for (int i = 0; i < PPL; ++i) {
-      gt[i] = at(f.gt, j0, i), gq[i] = at(f.gq, j0, i);
-      gu[i] = at(f.gu, j0, i), gv[i] = at(f.gv, j0, i);
       const R zsdotp = sigh[jm] * tot[i] - (rz[i] + rv[i]);
-      const R a = zsdotp * (gt[i] - at(f.gt, jm, i)), b = zsdotp * (gq[i] + at(f.gq, jm, i));
-      const R c = zsdotp * (gu[i] - at(f.gu, jm, i)), d = zsdotp * (gv[i] - at(f.gv, jm, i));
+      const R a = zsdotp * (gt[i] - gtm[i]), b = zsdotp * (gq[i] + gqm[i]);
+      const R c = zsdotp * (gu[i] - gum[i]), d = zsdotp * (gv[i] - gvm[i]);
       const R e = t01[jm] * (sigh[jm] * vp[i] - rv[i]);
       gtd_m[i] = j0 > 0 ? a : R(0), gqm_m[i] = j0 > 0 ? b : R(0);
       gud_m[i] = j0 > 0 ? c : R(0), gvd_m[i] = j0 > 0 ? d : R(0);
@@ -206,18 +216,16 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
     }
   }
   C2<R>* fb = (C2<R>*)(cr + n * P) + w * C::NFB * C::NP;  // this wave's FFT rows
+  struct V2 {
+    R v[2];
+  } __attribute__((packed, aligned(sizeof(R))));
   for (int j = j0; j < j1; ++j) {
     const bool top = j == 0, bottom = j == n - 1;
     // this level's inputs first, so that they arrive during the sums below
     const int jp = bottom ? j : j + 1;
     R gz[PPL], gt1[PPL], gq1[PPL], gu1[PPL], gv1[PPL], dq[PPL];
-#pragma unroll
-    for (int i = 0; i < PPL; ++i) {
-      gz[i] = at(f.gz, j, i);
-      gt1[i] = at(f.gt, jp, i), gq1[i] = at(f.gq, jp, i);
-      gu1[i] = at(f.gu, jp, i), gv1[i] = at(f.gv, jp, i);
-      if (nqspec != 1) dq[i] = at(f.dq, j, i);
-    }
+    at(f.gz, j, gz), at(f.gt, jp, gt1), at(f.gq, jp, gq1), at(f.gu, jp, gu1), at(f.gv, jp, gv1);
+    if (nqspec != 1) at(f.dq, j, dq);
     // c(k, j) for k <= j: column j of c; ztptb = ztpta + the same sum over the
     // divergence
     R ztpta[PPL], ztptb[PPL], gphi[PPL];
@@ -229,7 +237,7 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
       const R ck = cj[k];
 #pragma unroll
       for (int i = 0; i < PPL; ++i) {
-        const R2 x = zg[k * P + lane + 64 * i];
+        const R2 x = zg[k * P + l0 + LS * i];
         ztpta[i] = ztpta[i] + ck * x.x;
         ztptb[i] = ztptb[i] + ck * x.y;
       }
@@ -239,14 +247,15 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
     for (int k = 0; k < n; ++k) {
       const R gk = gj[k];
 #pragma unroll
-      for (int i = 0; i < PPL; ++i) gphi[i] = gphi[i] + gk * cr[k * P + lane + 64 * i];
+      for (int i = 0; i < PPL; ++i) gphi[i] = gphi[i] + gk * cr[k * P + l0 + LS * i];
     }
     R out[10][PPL];  // gtn gqn guz gvz gut gvt guq gvq gke, and gvp at the top
+    R dw[PPL];
     const R rd = rdsig[j], dsj = bottom ? R(0) : dsig[j], shj = sigh[j], t01j = t01[j];
 #pragma unroll
     for (int i = 0; i < PPL; ++i) {
-      const R2 x = zg[j * P + lane + 64 * i];
-      const R zv = x.x, gd = x.y, corr = cr[j * P + lane + 64 * i];
+      const R2 x = zg[j * P + l0 + LS * i];
+      const R zv = x.x, gd = x.y, corr = cr[j * P + l0 + LS * i];
       R zq = (nqspec == 1) ? gq[i] / gp[i] : dq[i];
       zq = zq > R(0) ? zq : R(0);
       ztptb[i] = ztpta[i] + ztptb[i];
@@ -263,9 +272,7 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
       const R gvd = bottom ? R(0) : zsdotp * (gv1[i] - gv[i]);
       const R ti = bottom ? R(0) : t01j * (shj * vp[i] - rv[i]);
       const R za = top ? -gd : zv - ztptb[i], zt = top ? R(0) : tkp[j] * (zv - ztpta[i]);
-      const R dw = (top ? gd : za) * gp[i] * v.psurf * v.ww;
-      put(f.dw, j, i, dw);
-      put(f.gphi, j, i, gphi[i]);
+      dw[i] = (top ? gd : za) * gp[i] * v.psurf * v.ww;
       out[0][i] = gt[i] * gd + v.akap * ztv2 * za + zt - rd * (gtd + gtd_m[i] + ti + tim[i]);
       out[1][i] = -rd * (gqm - gqm_m[i]);
       out[2][i] = -gu[i] * gz[i] - gpj[i] * ztv1 - rd * (gvd + gvd_m[i]);
@@ -276,57 +283,57 @@ __global__ __launch_bounds__(64 * WAVES, (GpCfg<R, ROW, WAVES>::WPS)) void k_cal
       out[7][i] = gv[i] * gq[i];
       out[8][i] = gu[i] * gu[i] + gv[i] * gv[i] + gphi[i];
       out[9][i] = top ? vp[i] : R(0);
-      if constexpr (ROW > 0 && C::NFB == 5) {
-        // (straight into the FFT rows, one point's values in registers at a time)
-#pragma unroll
-        for (int q = 0; q < 5; ++q)
-          fb[q * C::NP + bix(lane + 64 * i)] = C2<R>{out[2 * q][i], out[2 * q + 1][i]};
-        __builtin_amdgcn_sched_barrier(0);
-      }
       gtd_m[i] = gtd, gqm_m[i] = gqm, gud_m[i] = gud, gvd_m[i] = gvd, tim[i] = ti;
       gt[i] = gt1[i], gq[i] = gq1[i], gu[i] = gu1[i], gv[i] = gv1[i];
     }
+    put(f.dw, j, dw);
+    put(f.gphi, j, gphi);
     R* const dst[10] = {f.gtn, f.gqn, f.guz, f.gvz, f.gut, f.gvt, f.guq, f.gvq, f.gke, f.gvp};
     if constexpr (ROW == 0) {
 #pragma unroll
       for (int q = 0; q < 9; ++q)
-        if (dst[q] && (q < 6 || q > 7 || nqspec == 1)) {
-#pragma unroll
-          for (int i = 0; i < PPL; ++i) put(dst[q], j, i, out[q][i]);
-        }
+        if (dst[q] && (q < 6 || q > 7 || nqspec == 1)) put(dst[q], j, out[q]);
     } else {
-      // gp2fc: z = out[2q] + i out[2q + 1], separated by the Hermitian pair
-      constexpr int NFB = C::NFB, NP = C::NP, N = ROW;
+      // gp2fc: Z = FFT(x[2k] + i x[2k + 1]) of half the length holds the sums E
+      // over the even and O over the odd points, E = (Z[k] + conj Z[H - k]) / 2,
+      // O = (Z[k] - conj Z[H - k]) / 2i, and with w = e^{-2 pi i k / N} X[k] = E +
+      // w O, X[H - k] = conj(E - w O); X[0] = Re Z[0] + Im Z[0], X[H / 2] = conj
+      // Z[H / 2].  RPI rows side by side in a wave.
+      constexpr int NFB = C::NFB, NP = C::NP, N = ROW, H = C::H, RPI = 128 / H;
       const C2<R>* tws = (const C2<R>*)(cr + n * P) + W * NFB * NP;
       const R sc = R(0.5) / R(N);
+      const int k = lane % (H / 2), kn = k ? H - k : H / 2, sub = lane / (H / 2);
 #pragma unroll
-      for (int q0 = 0; q0 < 5; q0 += NFB) {
-        if constexpr (NFB < 5) {
+      for (int q0 = 0; q0 < 10; q0 += NFB) {
 #pragma unroll
-          for (int q = q0; q < q0 + NFB && q < 5; ++q)
-#pragma unroll
-            for (int i = 0; i < PPL; ++i)
-              fb[(q - q0) * NP + bix(lane + 64 * i)] = C2<R>{out[2 * q][i], out[2 * q + 1][i]};
+        for (int q = q0; q < q0 + NFB && q < 10; ++q) {
+          C2<R>* row = fb + (q - q0) * NP;
+          if constexpr (PPL == 2)
+            row[wix<C::H, R>(lane)] = C2<R>{out[q][0], out[q][PPL - 1]};
+          else
+            ((R*)(row + wix<C::H, R>(lane >> 1)))[lane & 1] = out[q][0];
         }
-        if (q0 + NFB <= 5)
-          fft_wave_rows<N, NFB, -1>(fb, tws, lane);
+        if (q0 + NFB <= 10)
+          fft_wave_rows<H, C::R0, NFB, -1, 2>(fb, tws, lane);
         else
-          fft_wave_rows<N, (5 % NFB ? 5 % NFB : 1), -1>(fb, tws, lane);
+          fft_wave_rows<H, C::R0, (10 % NFB ? 10 % NFB : 1), -1, 2>(fb, tws, lane);
 #pragma unroll
-        for (int q = q0; q < q0 + NFB && q < 5; ++q) {
-          if (q == 3 && nqspec != 1) continue;
+        for (int q = q0; q < q0 + NFB && q < 10; q += RPI) {
+          const int r = q + sub;
+          R* d = dst[q];
 #pragma unroll
-          for (int k0 = 0; k0 < N / 2; k0 += 64) {
-            const int k = k0 + lane;
-            if (N / 2 % 64 && k >= N / 2) break;
-            const C2<R> zk = fb[(q - q0) * NP + bix(k)];
-            const C2<R> zn = fb[(q - q0) * NP + bix(k ? N - k : 0)];
-            const long o = mo + (long)j * nhor + 2 * k0;
-            ((R2*)(dst[2 * q] + o))[(unsigned)lane] = R2{(zk.x + zn.x) * sc, (zk.y - zn.y) * sc};
-            if (q < 4 || top)
-              ((R2*)(dst[2 * q + 1] + o))[(unsigned)lane] =
-                  R2{(zk.y + zn.y) * sc, (zn.x - zk.x) * sc};
+          for (int u = 1; u < RPI; ++u) {
+            R* const du = dst[q + u < 10 ? q + u : 9];
+            d = sub == u ? du : d;
           }
+          if (r >= q0 + NFB || r > 9 || (r == 9 && !top) || (r / 2 == 3 && nqspec != 1)) continue;
+          const C2<R>* row = fb + (r - q0) * NP;
+          const C2<R> zk = row[wix<C::H, R>(k)], zn = row[wix<C::H, R>(kn)];
+          const R ex = zk.x + zn.x, ey = zk.y - zn.y;
+          const C2<R> t = cmul(tws[k], C2<R>{zk.x - zn.x, zk.y + zn.y});
+          V2* o = (V2*)(d + (mo + (long)j * nhor));
+          o[k] = V2{{(k ? ex + t.y : R(2) * (zk.x + zk.y)) * sc, (k ? ey - t.x : R(0)) * sc}};
+          o[kn] = V2{{(k ? ex - t.y : R(2) * zn.x) * sc, (k ? -(ey + t.x) : R(-2) * zn.y) * sc}};
         }
         wave_lds_sync();  // the rows are read before the next ones are written
       }

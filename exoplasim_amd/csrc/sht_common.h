@@ -608,9 +608,20 @@ __device__ __forceinline__ void fft_wave(C2<F>* row, const C2<F>* tw, int lane, 
   wave_lds_sync();
 }
 
+// Where value i lies in a row of N complex values that one wave transforms.
+// FP64, N = 64: the first of two radix-8 passes writes 128 bytes apart, which
+// bix's pads leave on every fourth lane's banks; the exclusive or with the
+// group of 8 spreads its writes and reads over all of them (T42 L40,
+// 16 members, gridpointa 663 -> 632 us, L20, 32 members, 452 -> 442).  N = 32 has
+// no registers left for its addresses (T21 L10, 32 members, 66 -> 77).
+template <int N, typename F>
+__device__ __forceinline__ int wix(int i) {
+  return sizeof(F) == 8 && N == 64 ? i ^ ((i >> 3) & 7) : bix(i);
+}
+
 // One Stockham pass (radix R, stride NS) of the NF rows of N + N/32 complex
-// values in `buf`, in place, by one wave; tw[k] = e^{S 2 pi i k / N}.
-template <int N, int R, int NS, int NF, int S, typename F>
+// values in `buf`, in place, by one wave; tw[TS k] = e^{S 2 pi i k / N}.
+template <int N, int R, int NS, int NF, int S, int TS, typename F>
 __device__ __forceinline__ void fft_wave_pass(C2<F>* buf, const C2<F>* tw, int lane) {
   constexpr int NB = N / R, NP = N + N / 32, TOT = NF * NB, BPT = (TOT + 63) / 64;
   C2<F> v[BPT][R];
@@ -620,7 +631,7 @@ __device__ __forceinline__ void fft_wave_pass(C2<F>* buf, const C2<F>* tw, int l
     if (b < TOT) {
       const int f = b / NB, j = b - f * NB;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[t][r] = buf[f * NP + bix(j + r * NB)];
+      for (int r = 0; r < R; ++r) v[t][r] = buf[f * NP + wix<N, F>(j + r * NB)];
     }
   }
   wave_lds_sync();
@@ -631,27 +642,24 @@ __device__ __forceinline__ void fft_wave_pass(C2<F>* buf, const C2<F>* tw, int l
       const int f = b / NB, j = b - f * NB, jm = j % NS;
       if (NS > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) v[t][r] = cmul(v[t][r], tw[jm * r * (N / (NS * R))]);
+        for (int r = 1; r < R; ++r) v[t][r] = cmul(v[t][r], tw[jm * r * (TS * N / (NS * R))]);
       }
       Dft<R, S, F>::run(v[t]);
       const int o = (j / NS) * NS * R + jm;
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[f * NP + bix(o + r * NS)] = v[t][r];
+      for (int r = 0; r < R; ++r) buf[f * NP + wix<N, F>(o + r * NS)] = v[t][r];
     }
   }
   wave_lds_sync();
 }
 
 // FFTs of the NF rows in `buf`, in place, by one wave (only the calling wave
-// touches them), with the radices of FftPlan<N>
-template <int N, int NF, int S, typename F>
+// touches them), with radices R0 and N / R0; tw is the table of length TS N
+template <int N, int R0, int NF, int S, int TS, typename F>
 __device__ __forceinline__ void fft_wave_rows(C2<F>* buf, const C2<F>* tw, int lane) {
-  using P = FftPlan<N>;
-  static_assert(P::NP == 2 || P::NP == 3, "two or three passes");
   wave_lds_sync();
-  fft_wave_pass<N, P::R[0], 1, NF, S>(buf, tw, lane);
-  fft_wave_pass<N, P::R[1], P::R[0], NF, S>(buf, tw, lane);
-  if constexpr (P::NP == 3) fft_wave_pass<N, P::R[2], P::R[0] * P::R[1], NF, S>(buf, tw, lane);
+  fft_wave_pass<N, R0, 1, NF, S, TS>(buf, tw, lane);
+  fft_wave_pass<N, N / R0, R0, NF, S, TS>(buf, tw, lane);
 }
 
 // ---- split-BF16 helpers ----

@@ -409,3 +409,92 @@ def test_noalloc_last_chunk(gpu, ntru, nlev, nmem, mode):
     torch.cuda.synchronize()
     assert torch.equal(gp, gp2) and torch.equal(y, y2)
     plan.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 10, 1), (21, 9, 9), (42, 20, 1), (42, 7, 5)])
+@pytest.mark.parametrize("mode", ["f64", "f32", "bf16x3"])
+def test_gridpointa_dry_levels(oracle, gpu, ntru, nlev, nmem, mode):
+    """humidity falling by 1e4 from the surface to the top: the rounding of a
+    level's moisture tendency is that of its own terms, however much larger
+    the other fields are.  Per level, the tolerances of the whole fields: a
+    level's terms reach one level up and down, whose humidity is at most 4.6
+    times its own (1e4^(1/6), L7), and cancel no more than the whole fields'
+    do: 1e-12 and 2e-5.  A field that shared its row FFT with one 1e4 to 1e5
+    times as large would keep 1e-16 * 1e5 and 1e-7 * 1e5."""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.dynamics import Dynamics
+
+    print(f"dry levels T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    v = _vertical(oracle, nlev)
+    plan, dyn = sht.Plan(ntru), Dynamics.from_vertical(v, *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, nmem, mode)
+    states = np.stack([gridpointa_state(ntru, nlev, 0.9 + 0.02 * k) for k in range(nmem)])
+    states[:, 3 * nlev:4 * nlev] *= np.logspace(-4, 0, nlev)[:, None]
+    st.copy_(torch.from_numpy(states).to(st.dtype))
+    dyn.gridpointa(plan, mode, st, work, tend)
+    got, host = tend.double().cpu().numpy(), st.double().cpu().numpy()
+    for k in (0, nmem - 1):
+        want, _ = oracle.gridpointa(ntru, nlev, host[k], v, PLASIM_SCAL, 1)
+        for j in range(3 * nlev, 4 * nlev):
+            assert rel(got[k, j], want[j]) < (1e-12 if mode == "f64" else 2e-5), (k, j)
+    dyn.close()
+    plan.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 10, 1), (21, 9, 9), (42, 20, 1), (42, 7, 5),
+                                            (63, 5, 1)])
+@pytest.mark.parametrize("mode", ["f64", "f32", "bf16x3"])
+def test_gridpointa_fields_apart(gpu, ntru, nlev, nmem, mode):
+    """no field's values reach another through the transforms: a state
+    without humidity has a moisture tendency of zeros, a humidity that is not
+    a number at one level (which the virtual temperature takes as none)
+    leaves the other tendencies as those of that level dry, to the last bit,
+    and so does whatever lies in the grid humidity gq without spectral
+    humidity, where only dq enters the temperature"""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.dynamics import Dynamics, work_slots
+
+    print(f"fields apart T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    x = np.arange(1, nlev + 1) / nlev
+    sh = 0.75 * x + 1.75 * x ** 3 - 1.5 * x ** 4
+    ds = np.diff(np.concatenate([[0.0], sh]))
+    g = np.tril(np.full((nlev, nlev), 0.2))
+    v = dict(sigmah=sh, dsigma=ds, rdsig=0.5 / ds, t0=np.linspace(220.0, 288.0, nlev) / CT,
+             t01s2=np.full(nlev, 0.01), tkp=np.full(nlev, 0.08), c=g.T, g=g, akap=0.286)
+    plan, dyn = sht.Plan(ntru), Dynamics.from_vertical(v, *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, nmem, mode)
+    st.copy_(torch.from_numpy(np.stack([gridpointa_state(ntru, nlev, 0.9 + 0.02 * k)
+                                        for k in range(nmem)])).to(st.dtype))
+    sl, sq = work_slots(nlev), slice(3 * nlev, 4 * nlev)
+    other = [i for i in range(4 * nlev + 1) if not 3 * nlev <= i < 4 * nlev]
+
+    def run(nq=1):
+        tend.fill_(float("nan"))
+        dyn.gridpointa(plan, mode, st, work, tend, nqspec=nq)
+        torch.cuda.synchronize()
+        return tend[:, other].clone()
+
+    wet = st[:, sq].clone()
+    st[:, sq] = 0
+    run()
+    assert not bool(tend[:, sq].any())
+    st[:, sq] = wet
+    st[:, 3 * nlev + 2] = 0
+    dry = run()
+    assert bool(torch.isfinite(dry).all())
+    st[:, 3 * nlev + 2] = float("nan")
+    assert torch.equal(run(), dry)
+    assert bool(torch.isfinite(tend[:, 4 * nlev - 1]).all())
+    work[:, sl["dq"]:sl["dq"] + nlev] = 1e-3
+    work[:, sl["gq"]:sl["gq"] + nlev] = 0
+    dry = run(0)
+    assert bool(torch.isfinite(dry).all())
+    for bad in (1e30, float("inf"), float("nan")):
+        work[:, sl["gq"]:sl["gq"] + nlev] = bad
+        assert torch.equal(run(0), dry), bad
+    dyn.close()
+    plan.close()
