@@ -230,7 +230,11 @@ def _register_ops():
         L, s = _proto(), _stream()
         M, dev = gy.shape[0], gy.device
         ws = [w.contiguous() for w in (w1, w2, w3, w4)]
-        g = gy.float().contiguous()
+        if gy.shape == (M, NOUT):
+            g = gy.float().contiguous()
+        else:  # broadcast, or refused: the kernels read M x 21 values
+            g = torch.empty((M, NOUT), dtype=f32, device=dev)
+            g[:] = gy
         dw = [torch.empty((nout, nin), dtype=f32, device=dev) for nin, nout in LAYERS]
         db = [torch.empty(nout, dtype=f32, device=dev) for _, nout in LAYERS]
         work = torch.empty(L.exo_mlp_train_work(M, 1), dtype=torch.uint8, device=dev)

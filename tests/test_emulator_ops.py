@@ -2,6 +2,9 @@
 schemas, and their fake-tensor rules and the registered autograd formula
 give the shapes and dtypes of the network's output and of every parameter
 gradient (FakeTensorMode runs no kernel)."""
+import ctypes
+
+import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
@@ -25,3 +28,43 @@ def test_ops_register_and_trace():
         y.sum().backward()
         for p in ps:
             assert p.grad is not None and p.grad.shape == p.shape
+
+
+@pytest.mark.parametrize("shape", [(5, 20), (5, 22), (4,), (5, 2), (5, 0)])
+def test_backward_refuses_wrong_gradients(monkeypatch, shape):
+    """an output gradient that does not broadcast to (rows, 21) raises and
+    reaches no kernel, which would read past its end; one that does is read
+    broadcast"""
+    from exoplasim_amd import radiation as r
+
+    r.emulator_op()
+    seen = []
+
+    class Native:
+        @staticmethod
+        def exo_mlp_train_work(m, backward):
+            return 16
+
+        @staticmethod
+        def exo_mlp_train_backward(m, gy, *rest):
+            seen.append(list((ctypes.c_float * (m * r.NOUT)).from_address(gy)))
+            return 0
+
+    monkeypatch.setattr(r, "_proto", lambda: Native)
+    monkeypatch.setattr(r, "_stream", lambda: None)
+    f32, bf = torch.float32, torch.bfloat16
+
+    def backward(gy):
+        m = gy.shape[0]
+        return torch.ops.exoplasim_amd.lw_mlp_backward(
+            gy, torch.zeros(m, r.KIN, dtype=bf), *[torch.zeros(m, r.NHID) for _ in range(3)],
+            *[torch.zeros(m, r.NHID, dtype=bf) for _ in range(3)],
+            *[torch.zeros(nout, nin) for nin, nout in r.LAYERS])
+
+    with pytest.raises(RuntimeError):
+        backward(torch.ones(shape))
+    assert not seen
+    col = torch.arange(5, dtype=f32)[:, None]
+    for gy in (col, col.double(), col.expand(5, r.NOUT)):
+        backward(gy)
+        assert seen.pop() == [float(i) for i in range(5) for _ in range(r.NOUT)]
