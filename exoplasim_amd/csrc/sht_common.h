@@ -179,9 +179,14 @@ template <typename R>
 __device__ __forceinline__ C2<R> cadd(C2<R> a, C2<R> b) { return {a.x + b.x, a.y + b.y}; }
 template <typename R>
 __device__ __forceinline__ C2<R> csub(C2<R> a, C2<R> b) { return {a.x - b.x, a.y - b.y}; }
+// (Which of its products a sum is fused with is written out, so that a row's
+// FFT gives the same bits in every kernel: left to the compiler, the choice
+// differed between tile variants on rows of 128 and 384 points, and with it
+// the last bits of a member's fields with the size of the call.)
 template <typename R>
 __device__ __forceinline__ C2<R> cmul(C2<R> a, C2<R> b) {
-  return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+  return {__builtin_elementwise_fma(a.x, b.x, -(a.y * b.y)),
+          __builtin_elementwise_fma(a.x, b.y, a.y * b.x)};
 }
 // multiply by s*i (s = +1 or -1)
 template <int S, typename R>

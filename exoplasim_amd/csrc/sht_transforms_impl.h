@@ -164,8 +164,7 @@ static int inv_auto(long nblk3) {
 }
 
 // blocks at V = 3 of the call that a launch belongs to: a call that runs its
-// members in chunks uses the same tiles, and returns the same bits, as one
-// launch of them all
+// members in chunks uses the tiles of one launch of them all
 template <int T, int MODE>
 static long inv_rule(InvArgs a) {
   if (a.nrule > 0) a.nmem = a.nrule;

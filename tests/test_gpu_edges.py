@@ -498,3 +498,95 @@ def test_gridpointa_fields_apart(gpu, ntru, nlev, nmem, mode):
         assert torch.equal(run(0), dry), bad
     dyn.close()
     plan.close()
+
+
+@pytest.mark.parametrize("ntru", [21, 42, 63, 127])
+@pytest.mark.parametrize("mode", ["f64", "f32", "f32mfma", "bf16x3"])
+def test_tile_variants_same_bits(gpu, ntru, mode):
+    """the tile variants sum in the same order and round in the same places,
+    so that the choice among them, by tuning or by the size of a call, does
+    not show in the results: equal to the last bit, in the inverse, the wind
+    and the direct transforms"""
+    import torch
+
+    from exoplasim_amd import sht
+
+    print(f"variants T{ntru} {mode}", flush=True)
+    plan, nlev = sht.Plan(ntru), 5
+    x, gp, y = plan.alloc_roundtrip(3, nlev, mode)
+    x.normal_()
+    first = None
+    for v in range(4):
+        plan.set_tiles(mode, v, v, v)
+        gp.fill_(float("nan"))
+        plan.inverse_all(mode, x, gp, nlev)
+        out = [gp.clone()]
+        plan.inverse_uv(mode, x, gp, nlev, 0, nlev, 3 * nlev + 2, 4 * nlev + 2)
+        out.append(gp.clone())
+        y.fill_(float("nan"))
+        plan.direct(mode, out[0] if first is None else first[0], y, 3 * nlev + 1)
+        out.append(y.clone())
+        torch.cuda.synchronize()
+        first = first or out
+        assert all(torch.equal(a, b) for a, b in zip(out, first)), v
+    plan.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 20, 40), (42, 10, 9), (42, 20, 16), (63, 10, 16),
+                                            (127, 5, 9)])
+@pytest.mark.parametrize("mode", ["f64", "f32", "f32mfma", "bf16x3"])
+def test_member_alone_same_bits(gpu, ntru, nlev, nmem, mode):
+    """a member's round trip and dynamics step on an untuned plan are the same
+    to the last bit alone, in a call whose tiles and waves per block are the
+    small ones, and among as many members as take the large ones"""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd.dynamics import Dynamics
+
+    print(f"member alone T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    plan = sht.Plan(ntru)
+    x, gp, y = plan.alloc_roundtrip(nmem, nlev, mode)
+    x.normal_()
+    plan.roundtrip(mode, x, gp, y, nlev)
+    x1, gp1, y1 = plan.alloc_roundtrip(1, nlev, mode)
+    x1.copy_(x[nmem - 1:])
+    plan.roundtrip(mode, x1, gp1, y1, nlev)
+    torch.cuda.synchronize()
+    assert torch.equal(gp1[0], gp[nmem - 1]) and torch.equal(y1[0], y[nmem - 1])
+    del x, gp, y
+    s = np.arange(1, nlev + 1) / nlev
+    g = np.tril(np.full((nlev, nlev), 0.2))
+    v = dict(sigmah=s, dsigma=np.full(nlev, 1 / nlev), rdsig=np.full(nlev, nlev / 2),
+             t0=np.linspace(220.0, 288.0, nlev) / CT, t01s2=np.full(nlev, 0.01),
+             tkp=np.full(nlev, 0.08), c=g.T, g=g, akap=0.286)
+    dyn = Dynamics.from_vertical(v, *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, nmem, mode)
+    st.copy_(torch.from_numpy(np.stack([gridpointa_state(ntru, nlev, 0.9 + 0.01 * k)
+                                        for k in range(nmem)])).to(st.dtype))
+    dyn.gridpointa(plan, mode, st, work, tend)
+    st1, work1, tend1 = dyn.alloc_gridpointa(plan, 1, mode)
+    st1.copy_(st[nmem - 1:])
+    dyn.gridpointa(plan, mode, st1, work1, tend1)
+    torch.cuda.synchronize()
+    assert torch.equal(work1[0], work[nmem - 1]) and torch.equal(tend1[0], tend[nmem - 1])
+    dyn.close()
+    plan.close()
+
+
+def test_emulator_columns_same_bits(gpu):
+    """a column's heating and a row's network output are the same to the last
+    bit in calls of 16 and of 32 columns per block"""
+    import torch
+
+    from exoplasim_amd import radiation as R
+    from exoplasim_amd.columns import make_columns
+
+    em = R.LwEmulator(seed=5)
+    cols = R.columns_to_device(make_columns(8192, 20, 3), torch.float32)
+    part = {k: v[..., 100:2000].contiguous() for k, v in cols.items()}
+    (heat, olr), (h, o) = em.predict(cols), em.predict(part)
+    assert torch.equal(heat[:, 100:2000], h) and torch.equal(olr[100:2000], o)
+    x = R.features(cols)
+    with torch.no_grad():
+        assert torch.equal(em.raw(x)[100:2000], em.raw(x[100:2000]))
