@@ -481,8 +481,8 @@ extern "C" int exo_sht_roundtrip_noalloc(exo_sht_plan_t p, int mode, int nmem, i
 
 extern "C" int exo_sht_set_tiles(exo_sht_plan_t p, int mode, int inv_var, int uv_var,
                                  int fwd_var) {
-  if (!p || !mode_ok(mode) || inv_var < 0 || inv_var > 3 || uv_var < 0 || uv_var > 3 ||
-      fwd_var < 0 || fwd_var > 3)
+  if (!p || !mode_ok(mode) || inv_var < -1 || inv_var > 3 || uv_var < -1 || uv_var > 3 ||
+      fwd_var < -1 || fwd_var > 3)
     return EXO_ERR_ARG;
   std::lock_guard<std::mutex> lk(p->mu);
   p->inv_var[mode] = inv_var;
@@ -494,8 +494,9 @@ extern "C" int exo_sht_set_tiles(exo_sht_plan_t p, int mode, int inv_var, int uv
 extern "C" int exo_sht_get_tiles(exo_sht_plan_t p, int mode, int* vars) {
   if (!p || !mode_ok(mode) || !vars) return EXO_ERR_ARG;
   std::lock_guard<std::mutex> lk(p->mu);
-  const int v[3] = {p->inv_var[mode], p->uv_var[mode], p->fwd_var[mode]};
-  for (int k = 0; k < 3; ++k) vars[k] = v[k] < 0 ? 0 : v[k];
+  vars[0] = p->inv_var[mode];
+  vars[1] = p->uv_var[mode];
+  vars[2] = p->fwd_var[mode];
   return EXO_OK;
 }
 

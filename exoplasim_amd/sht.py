@@ -432,6 +432,8 @@ class Plan:
                                    _ptr(ut), _ptr(vt), fs, _stream()), "mktend")
 
     def set_tiles(self, mode, inv_var=0, uv_var=0, fwd_var=0):
+        """Tile variants 0-3 of the fused kernels, or -1: by the size of each
+        call, as on a plan that was neither set nor tuned."""
         check(lib().exo_sht_set_tiles(self._h, mode_id(mode), inv_var, uv_var, fwd_var),
               "set_tiles")
 

@@ -223,8 +223,8 @@ int exo_sht_mktend(exo_sht_plan_t plan, int mode, int nmem, int nlev, void *d, v
  * per block (half the LDS, twice the blocks in flight), 2 = default tiles
  * on 512-thread blocks (twice the waves per block), 3 = half the
  * field-levels on 512-thread blocks.  The results do not depend on the
- * variant, to the last bit.  A plan that was neither set nor tuned chooses
- * by the size of each call (and reports 0).  exo_sht_autotune times each variant (two untimed calls, then the
+ * variant, to the last bit.  -1 = by the size of each call, as a plan that
+ * was neither set nor tuned chooses (and reports).  exo_sht_autotune times each variant (two untimed calls, then the
  * average of eight back-to-back calls) on a round trip of nmem members x nlev
  * levels, keeps the fastest of each for this mode and returns them in vars[3]
  * (may be NULL).

@@ -590,3 +590,22 @@ def test_emulator_columns_same_bits(gpu):
     x = R.features(cols)
     with torch.no_grad():
         assert torch.equal(em.raw(x)[100:2000], em.raw(x[100:2000]))
+
+
+def test_tiles_saved_and_restored(gpu):
+    """the choice by the size of each call is reported and can be set back"""
+    from exoplasim_amd import sht
+    from exoplasim_amd._lib import ExoError
+
+    plan = sht.Plan(21)
+    fresh = plan.tiles("f64")
+    assert fresh == (-1, -1, -1)
+    plan.set_tiles("f64", 2, 1, 3)
+    assert plan.tiles("f64") == (2, 1, 3) and plan.tiles("f32") == fresh
+    plan.set_tiles("f64", *fresh)
+    assert plan.tiles("f64") == fresh
+    for bad in ((-2, 0, 0), (0, 4, 0), (0, 0, -3)):
+        with pytest.raises(ExoError):
+            plan.set_tiles("f64", *bad)
+    assert plan.tiles("f64") == fresh
+    plan.close()
