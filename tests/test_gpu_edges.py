@@ -609,3 +609,76 @@ def test_tiles_saved_and_restored(gpu):
             plan.set_tiles("f64", *bad)
     assert plan.tiles("f64") == fresh
     plan.close()
+
+
+@pytest.mark.parametrize("nbatch", [1, 17, 64, 321, 1000])
+def test_mlp_layer_entry_points(gpu, nbatch):
+    """the layer-by-layer C entry points (casts, forward, input and weight
+    gradients), chained as a caller of include/exo_rad.h would, against the
+    FP64 oracle with the kernels' bf16 roundings, at ragged tiles of 64 rows
+    and one and several batch splits.  What is left is FP32 accumulation and
+    the bf16 values it flips to their neighbour: at most 2^-8 of a value,
+    below 2^-9 = 2e-3 in the norm."""
+    import ctypes
+    import sys as _sys
+
+    _sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(__file__)), "oracle"))
+    import mlp_oracle as MO
+    import torch
+
+    from exoplasim_amd import radiation as R
+    from exoplasim_amd._lib import lib
+
+    print(f"mlp layers {nbatch}", flush=True)
+    L, M, ci = lib(), nbatch, ctypes.c_int
+    p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    bf, f32 = torch.bfloat16, torch.float32
+    new = lambda *s, dt=f32: torch.full(s, float("nan"), dtype=dt, device="cuda")  # noqa: E731
+    g = torch.Generator(device="cpu").manual_seed(nbatch)
+    ws = [torch.randn(o, i, generator=g) * (2.0 / i) ** 0.5 for i, o in R.LAYERS]
+    bs = [0.1 * torch.randn(o, generator=g) for _, o in R.LAYERS]
+    x, gy = torch.randn(M, R.NIN, generator=g), torch.randn(M, R.NOUT, generator=g)
+    wd, bd = [w.cuda() for w in ws], [b.cuda() for b in bs]
+    wb, wt = [], []
+    for (nin, nout), (K, N), w in zip(R.LAYERS, R.PADDED, wd):
+        wb.append(new(N, K, dt=bf))
+        wt.append(new(K, N, dt=bf))
+        assert L.exo_mlp_cast_weights(p(w), ci(nout), ci(nin), ci(N), ci(K), p(wb[-1]),
+                                      p(wt[-1]), None) == 0
+    xd, h = x.cuda(), [new(M, R.KIN, dt=bf)]
+    assert L.exo_mlp_cast_rows(p(xd), ci(M), ci(R.NIN), ci(R.KIN), p(h[0]), None) == 0
+    z = []
+    for li in range(4):
+        K, N = R.PADDED[li]
+        out = new(M, N) if li < 3 else None
+        hn, y = (new(M, N, dt=bf), None) if li < 3 else (None, new(M, N))
+        assert L.exo_mlp_forward(p(h[li]), p(wb[li]), p(bd[li]), ci(M), ci(K), ci(N),
+                                 ci(R.LAYERS[li][1]), ci(int(li < 3)), p(out), p(hn), p(y),
+                                 None) == 0
+        z.append(out)
+        h.append(hn)
+    dz32 = torch.zeros(M, R.NOUTP, device="cuda")
+    dz32[:, :R.NOUT] = gy.cuda()
+    dz = new(M, R.NOUTP, dt=bf)
+    assert L.exo_mlp_cast_rows(p(dz32), ci(M), ci(R.NOUTP), ci(R.NOUTP), p(dz), None) == 0
+    nsplit = max(1, min(64, M // 256))
+    part, keep, grads = new(nsplit * R.NHID * R.NHID), [], [None] * 8
+    for li in (3, 2, 1, 0):
+        K, N = R.PADDED[li]
+        nin, nout = R.LAYERS[li]
+        dw, db = new(N, K), new(N)
+        assert L.exo_mlp_backward_dw(p(dz), p(h[li]), p(dz32), ci(M), ci(N), ci(K), ci(nsplit),
+                                     p(part), p(dw), p(db), None) == 0
+        grads[2 * li], grads[2 * li + 1] = dw[:nout, :nin], db[:nout]
+        if li:
+            keep += [dz, dz32]
+            ndz, ndz32 = new(M, K, dt=bf), new(M, K)
+            assert L.exo_mlp_backward_dx(p(dz), p(wt[li]), p(z[li - 1]), ci(M), ci(N), ci(K),
+                                         ci(R.LAYERS[li - 1][1]), p(ndz), p(ndz32), None) == 0
+            dz, dz32 = ndz, ndz32
+    torch.cuda.synchronize()
+    ps = [t.double().numpy() for w, b in zip(ws, bs) for t in (w, b)]
+    want, saved = MO.forward(x.double().numpy(), ps)
+    assert rel(y[:, :R.NOUT].double().cpu().numpy(), want) < 2e-3
+    for i, w in enumerate(MO.backward(gy.double().numpy(), ps, saved)):
+        assert rel(grads[i].double().cpu().numpy(), w) < 2e-3, i
