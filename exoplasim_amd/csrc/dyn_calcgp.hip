@@ -444,7 +444,8 @@ extern "C" int exo_dyn_destroy(exo_dyn_t d) {
 template <typename R>
 static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int exp_gp,
                     const exo_calcgp_fields* f, hipStream_t s, const double* sid = nullptr,
-                    int nlon = 1, void* rcsq_out = nullptr, const void* tw = nullptr) {
+                    int nlon = 1, void* rcsq_out = nullptr, const void* tw = nullptr,
+                    bool in_place = false) {
   CalcgpPtrs<R> p;
   p.gu = (const R*)f->gu;
   p.gv = (const R*)f->gv;
@@ -503,8 +504,25 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
         if (!few) return launch(k_calcgp<R, 128, 4>, 128, 4, GpCfg<R, 128, 4>::lds(n));
       }
       return launch(k_calcgp<R, 128, 8>, 128, 8, GpCfg<R, 128>::lds(n));
-    default: return launch(k_calcgp<R, 0, 8>, 64, 8, GpCfg<R, 0>::lds(n));
+    default:
+      // An output in the place of an input: a wave reads its neighbours' levels
+      // next to its own, so one wave takes them all, which has read a level and
+      // the next one before it writes the first.
+      if (in_place) return launch(k_calcgp<R, 0, 1>, 64, 1, GpCfg<R, 0, 1>::lds(n));
+      return launch(k_calcgp<R, 0, 8>, 64, 8, GpCfg<R, 0>::lds(n));
   }
+}
+
+// Does an output of a member overlap an input that is read level by level?
+static bool calcgp_in_place(const exo_calcgp_fields* f, size_t bytes) {
+  const void* in[] = {f->gu, f->gv, f->gt, f->gq, f->gz, f->dq};
+  const void* out[] = {f->gtn, f->gqn, f->guz, f->gvz, f->gphi, f->dw,
+                       f->gut, f->gvt, f->gke, f->guq, f->gvq};
+  for (const void* i : in)
+    for (const void* o : out)
+      if (i && o && (uintptr_t)i < (uintptr_t)o + bytes && (uintptr_t)o < (uintptr_t)i + bytes)
+        return true;
+  return false;
 }
 
 // Does gridpointa's calcgp transform its rows itself?  On rows of 64 and 128
@@ -536,8 +554,12 @@ extern "C" int exo_dyn_calcgp(exo_dyn_t d, int mode, int nmem, long member_strid
     if (!q) return EXO_ERR_ARG;
   if (nqspec == 0 && !f->dq) return EXO_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  if (mode == EXO_F64) return calcgp_t<double>(d, nmem, member_stride, nhor, nqspec, exp_gp, f, s);
-  return calcgp_t<float>(d, nmem, member_stride, nhor, nqspec, exp_gp, f, s);
+  const size_t es = mode == EXO_F64 ? 8 : 4;
+  const bool in_place = calcgp_in_place(f, es * d->nlev * nhor);
+  return mode == EXO_F64 ? calcgp_t<double>(d, nmem, member_stride, nhor, nqspec, exp_gp, f, s,
+                                            nullptr, 1, nullptr, nullptr, in_place)
+                         : calcgp_t<float>(d, nmem, member_stride, nhor, nqspec, exp_gp, f, s,
+                                           nullptr, 1, nullptr, nullptr, in_place);
 }
 
 extern "C" int exo_dyn_gpmt(int mode, int nlon, long nrow, const void* in, void* out,

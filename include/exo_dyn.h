@@ -50,7 +50,9 @@ typedef struct {
 /* calcgp (src/plasim.f90:2587) for nmem members whose fields all lie
  * member_stride elements apart; exp_gp != 0 first replaces gp by exp(gp)
  * (src/plasim.f90:2434).  Element type double for EXO_F64, float for the
- * other modes (and arithmetic in that type); asynchronous on stream. */
+ * other modes (and arithmetic in that type); asynchronous on stream.  An
+ * output may take the place of an input (slower: one wave then runs down all
+ * levels). */
 int exo_dyn_calcgp(exo_dyn_t dyn, int mode, int nmem, long member_stride, int nhor, int nqspec,
                    int exp_gp, const exo_calcgp_fields *f, void *stream);
 

@@ -682,3 +682,50 @@ def test_mlp_layer_entry_points(gpu, nbatch):
     assert rel(y[:, :R.NOUT].double().cpu().numpy(), want) < 2e-3
     for i, w in enumerate(MO.backward(gy.double().numpy(), ps, saved)):
         assert rel(grads[i].double().cpu().numpy(), w) < 2e-3, i
+
+
+@pytest.mark.parametrize("nlev,nhor,nmem", [(2, 1, 1), (7, 130, 2), (20, 512, 1), (64, 65, 2)])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+@pytest.mark.parametrize("nq", [1, 0])
+def test_calcgp_in_place(oracle, gpu, nlev, nhor, nmem, mode, nq):
+    """outputs in the place of the inputs that a level reads from the next and
+    the one before (temperature, humidity, winds) and of the vorticity: the
+    same as in arrays of their own, to the last bit"""
+    import torch
+
+    from exoplasim_amd.dynamics import CALCGP_OUT, PRODUCTS, Dynamics
+
+    print(f"calcgp in place L{nlev} x{nhor} x{nmem} {mode} nqspec={nq}", flush=True)
+    dyn = Dynamics.from_vertical(_vertical(oracle, nlev), *PLASIM_SCAL)
+    dt = torch.float64 if mode == "f64" else torch.float32
+    host = {k: x[..., :nhor] for k, x in plasim_inputs(nlev, 512, 5)[1].items()}
+
+    def fields():
+        f = {}
+        for k, x in host.items():
+            x = np.stack([x * (1 + 0.1 * m) for m in range(nmem)])
+            full = np.zeros((nmem, nlev, nhor))
+            full[:, :x.shape[1] if x.ndim == 3 else 1] = x if x.ndim == 3 else x[:, None]
+            f[k] = torch.from_numpy(full).to("cuda", dt)
+        for k in CALCGP_OUT + PRODUCTS + ("gvp",):
+            f[k] = torch.zeros((nmem, nlev, nhor), dtype=dt, device="cuda")
+        return f
+
+    def run(f):
+        flat = {k: (x[0] if x.dim() == 3 else x).contiguous() if nmem == 1 else x
+                for k, x in f.items()}
+        if nmem == 1:
+            for k in ("gp", "gpj", "gpm", "rcsq", "gvp"):
+                flat[k] = f[k][0, 0]
+        dyn.calcgp(mode, flat, nqspec=nq, nmem=nmem, member_stride=nlev * nhor if nmem > 1 else 0)
+        torch.cuda.synchronize()
+
+    a, b = fields(), fields()
+    places = dict(gtn="gt", gqn="gq", guz="gv", gvz="gu", gke="gz", gphi="gd")
+    for o, i in places.items():
+        b[o] = b[i]
+    run(a)
+    run(b)
+    for k in CALCGP_OUT + PRODUCTS + ("gvp",):
+        assert torch.equal(a[k], b[k]), k
+    dyn.close()
