@@ -509,6 +509,12 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
       // next to its own, so one wave takes them all, which has read a level and
       // the next one before it writes the first.
       if (in_place) return launch(k_calcgp<R, 0, 1>, 64, 1, GpCfg<R, 0, 1>::lds(n));
+      // Few levels on many points: with 8 waves each has one or two levels to
+      // pay for its sums over all of them (L10, 294912 points, FP64 131 us against
+      // 116 with 4 waves, FP32 48 against 41; 73728 points 24.9 and 24.8, 16.3 and
+      // 14.5; 18432 points 10.5 and 10.9; L20, 147456 points, FP32 43.9 and 45.1).
+      if (n <= 16 && ((nhor + 63L) / 64) * nmem > 1024)
+        return launch(k_calcgp<R, 0, 4>, 64, 4, GpCfg<R, 0, 4>::lds(n));
       return launch(k_calcgp<R, 0, 8>, 64, 8, GpCfg<R, 0>::lds(n));
   }
 }

@@ -729,3 +729,34 @@ def test_calcgp_in_place(oracle, gpu, nlev, nhor, nmem, mode, nq):
     for k in CALCGP_OUT + PRODUCTS + ("gvp",):
         assert torch.equal(a[k], b[k]), k
     dyn.close()
+
+
+@pytest.mark.parametrize("nlev", [2, 10, 16, 17])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+def test_calcgp_many_points(oracle, gpu, nlev, mode):
+    """more than 1024 blocks of 64 points, whose few levels 4 waves share
+    instead of 8: points at both ends as in a call of their own (8 waves,
+    against the oracle above), to the last bit"""
+    import torch
+
+    from exoplasim_amd.dynamics import CALCGP_OUT, PRODUCTS, Dynamics
+
+    print(f"calcgp many points L{nlev} {mode}", flush=True)
+    dyn = Dynamics.from_vertical(_vertical(oracle, nlev), *PLASIM_SCAL)
+    dt, nhor = torch.float64 if mode == "f64" else torch.float32, 64 * 1025 + 1
+    f = {k: torch.from_numpy(np.ascontiguousarray(x)).to("cuda", dt)
+         for k, x in plasim_inputs(nlev, nhor, 5)[1].items()}
+
+    def run(f):
+        out = {k: torch.zeros((nlev, f["gt"].shape[1]), dtype=dt, device="cuda")
+               for k in CALCGP_OUT + PRODUCTS}
+        out["gvp"] = torch.zeros(f["gt"].shape[1], dtype=dt, device="cuda")
+        dyn.calcgp(mode, {**f, **out}, nqspec=1)
+        torch.cuda.synchronize()
+        return out
+
+    whole = run(f)
+    for s in (slice(0, 130), slice(nhor - 70, nhor)):
+        for k, x in run({k: x[..., s].contiguous() for k, x in f.items()}).items():
+            assert torch.equal(x, whole[k][..., s]), k
+    dyn.close()
