@@ -952,6 +952,20 @@ extern "C" int exo_sht_fft(exo_sht_plan_t p, int mode, int dir, void* a, long lo
 // status of a launch_dirx on device arrays
 static int dirx_status(int rc) { return rc == 0 ? EXO_OK : EXO_ERR_LAUNCH; }
 
+// Do two device arrays of nmem members (la and lb values, sa and sb apart)
+// overlap?  Members of equal strides are compared one by one, as they may
+// lie within each other's gaps.
+static bool overlap(const void* a, long la, long sa, const void* b, long lb, long sb, int nmem,
+                    size_t es) {
+  const long d = (long)((intptr_t)a - (intptr_t)b), e = (long)es;
+  if (nmem == 1 || sa != sb || sa <= 0)
+    return d < e * ((nmem - 1) * sb + lb) && -d < e * ((nmem - 1) * sa + la);
+  const long s = e * sa, k0 = d / s;  // a + k s for member k further on
+  for (long k = k0 - 1; k <= k0 + 1; ++k)
+    if (-nmem < k && k < nmem && d - k * s < e * lb && k * s - d < e * la) return true;
+  return false;
+}
+
 static bool all_set(std::initializer_list<const void*> ps) {
   for (const void* q : ps)
     if (!q) return false;
@@ -991,7 +1005,27 @@ extern "C" int exo_sht_mktend(exo_sht_plan_t p, int mode, int nmem, int nlev, vo
     return EXO_ERR_ARG;
   if (nmem == 0 || nlev == 0) return EXO_OK;
   std::lock_guard<std::mutex> lk(p->mu);
+  hipStream_t s = (hipStream_t)stream;
+  // t or z in the place of an input: the transforms one after the other, as
+  // the reference runs them (D, T, Z), z beside the inputs until all are read
+  const long fl = (long)nlev * p->tb.nlat * p->tb.nlon, sl = (long)nlev * 2 * p->tb.ncsp;
+  const size_t es = mode == MODE_F64 ? 8 : 4;
+  bool over = false;
+  for (const void* i : {tn, fu, fv, ke, ut, vt})
+    for (const void* o : {t, z}) over = over || overlap(o, sl, s_stride, i, fl, f_stride, nmem, es);
+  if (over) {
+    const size_t need = es * ((nmem - 1) * s_stride + sl);
+    const int rc = plan_grow(&p->scratch, &p->scratch_bytes, need);
+    if (rc) return rc;
+    const DirxArgs dz = mktend_dz(ke, fv, fu, d, p->scratch, nlev, nmem, f_stride, s_stride);
+    const DirxArgs tt = mktend_t(vt, tn, ut, t, nlev, nmem, f_stride, s_stride);
+    if (launch_dirx(p->tb, mode, &dz, 1, s) || launch_dirx(p->tb, mode, &tt, 1, s))
+      return EXO_ERR_LAUNCH;
+    const size_t pitch = es * (nmem > 1 ? s_stride : sl);
+    HIPCK(hipMemcpy2DAsync(z, pitch, p->scratch, pitch, es * sl, nmem, hipMemcpyDeviceToDevice, s));
+    return EXO_OK;
+  }
   const DirxArgs a[2] = {mktend_dz(ke, fv, fu, d, z, nlev, nmem, f_stride, s_stride),
                          mktend_t(vt, tn, ut, t, nlev, nmem, f_stride, s_stride)};
-  return dirx_status(launch_dirx(p->tb, mode, a, 2, (hipStream_t)stream));
+  return dirx_status(launch_dirx(p->tb, mode, a, 2, s));
 }

@@ -197,8 +197,9 @@ int exo_sht_roundtrip_noalloc(exo_sht_plan_t plan, int mode, int nmem, int nlev,
  *   exo_sht_qtend   qtend (src/legmod.f90:433)
  *   exo_sht_mktend  mktend (src/legmod.f90:505); the model passes fu <- gvz,
  *                   fv <- guz (src/plasim.f90:2478)
- * The multi-input direct transforms (uv2dv, qtend, mktend) sum on the vector
- * ALUs in FP64 (EXO_F64) or FP32 (every other mode). */
+ * The multi-input direct transforms (uv2dv, qtend, mktend) sum in FP64
+ * (EXO_F64) or FP32 (every other mode).  Their outputs overlap no input, but
+ * t and z of mktend may lie where ke and, z, also where tn, ut or vt does. */
 int exo_sht_sp2fc(exo_sht_plan_t plan, int mode, int table, int nmem, const void *sp,
                   long sp_stride, int src0, void *fc, long fc_stride, int dst0, int nfield,
                   void *stream);

@@ -760,3 +760,31 @@ def test_calcgp_many_points(oracle, gpu, nlev, mode):
         for k, x in run({k: x[..., s].contiguous() for k, x in f.items()}).items():
             assert torch.equal(x, whole[k][..., s]), k
     dyn.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,nmem", [(21, 3, 1), (42, 9, 2)])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+def test_mktend_in_place(gpu, ntru, nlev, nmem, mode):
+    """the temperature tendency in the memory of ke and the vorticity's in that
+    of tn, vt or ke, which the transforms before them have read: as in arrays
+    of their own, to the last bit"""
+    import torch
+
+    from exoplasim_amd import sht
+
+    print(f"mktend in place T{ntru} L{nlev} x{nmem} {mode}", flush=True)
+    p = sht.Plan(ntru)
+    dt = p.dtype_of(mode)
+    tn, fu, fv, ke, ut, vt = (torch.randn(nmem, nlev, p.nlat, p.nlon, dtype=dt, device="cuda")
+                              for _ in range(6))
+    want = [torch.zeros((nmem, nlev, p.nrsp), dtype=dt, device="cuda") for _ in range(3)]
+    p.mktend(mode, *want, tn, fu, fv, ke, ut, vt, nlev)
+    for tat, zat in ((3, 0), (None, 5), (None, 3), (3, None)):
+        f = [x.clone() for x in (tn, fu, fv, ke, ut, vt)]
+        out = [torch.zeros_like(want[0])] + [
+            torch.zeros_like(want[0]) if k is None
+            else f[k].view(-1)[:want[0].numel()].view_as(want[0]) for k in (tat, zat)]
+        p.mktend(mode, *out, *f, nlev)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want)), (tat, zat)
+    p.close()
