@@ -532,7 +532,7 @@ static bool calcgp_in_place(const exo_calcgp_fields* f, size_t bytes) {
 }
 
 // Does gridpointa's calcgp transform its rows itself?  On rows of 64 and 128
-// whose level arrays fit a CU's LDS (all levels but FP64 above L40 on 128).
+// whose level arrays fit a CU's LDS (all levels but FP64 above L41 on 128).
 // Three points per lane on rows of 192 spill (T63 L20, 16 members, FP32: 479 us
 // against 390 with calcgp on the grid and the row FFT as a launch; FP64, 3
 // members: 289 against 253).

@@ -788,3 +788,28 @@ def test_mktend_in_place(gpu, ntru, nlev, nmem, mode):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, want)), (tat, zat)
     p.close()
+
+
+@pytest.mark.parametrize("ntru,nlev,mode", [(42, 42, "f64"), (42, 64, "f64"), (21, 64, "f64"),
+                                            (42, 64, "f32")])
+@pytest.mark.parametrize("nq", [1, 0])
+def test_gridpointa_most_levels(oracle, gpu, ntru, nlev, mode, nq):
+    """the level arrays of FP64 rows of 128 points fit a block's LDS up to L41
+    (3072 L + 35840 bytes of 163840; above): from L42 on calcgp runs on the
+    grid and the rows are transformed in a launch of their own.  The largest
+    level count of the other row kernels, whose 10 waves then ask for 152128
+    bytes.  Tolerances as above."""
+    test_gridpointa_edges(oracle, gpu, ntru, nlev, mode, nq)
+
+
+@pytest.mark.parametrize("ntru", [42, 63])
+@pytest.mark.parametrize("mode", ["f64", "f32", "bf16x3"])
+def test_untuned_tiles_many_blocks(oracle, gpu, ntru, mode):
+    """calls far above the sizes where untuned plans take other tiles: 16
+    members of L20.  Blocks at half the fields per block (V = 3), against the
+    limits 256 and 512: inverse T42 4 pair blocks x (16 + 1 + 10) groups x 16
+    members = 1728, T63 6 x (21 + 1 + 20) x 16 = 4032 (FP64, two fields per block,
+    4 and 6 x (31 + 1 + 20) x 16 = 3328 and 4992); direct 61 fields x 16 = 976
+    (T63 FP64, two latitude blocks: 1952).  So the whole tiles: V = 2, in the
+    FP64 direct of T42 V = 0."""
+    test_untuned_tiles(oracle, gpu, ntru, 20, 16, mode)
