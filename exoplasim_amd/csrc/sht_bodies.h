@@ -934,12 +934,12 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int blk, const void* 
   else
     outp = (R*)scratch + ((long)pb * a.nmem + mem) * a.nfield * S::NRSP;
   const bool qtab = table_is_q(a.table);
-  // the table [t][pair / G][w][G], one 16-byte load per G = 2 (FP64) or 4 pairs
+  // the table [pair / G][w][G], one 16-byte load per G = 2 (FP64) or 4 pairs
   // (a wave's loads cost the same whatever their width; FP64 with one 8-byte
   // load per pair: T42 L20 round trip of 32 members 169 us against 164)
   constexpr int G = 16 / (int)sizeof(R);
   static_assert(PB % G == 0, "pair blocks of whole groups");
-  const R* tv = (const R*)tabv + (long)a.table * S::NPAIR * S::NCSP + (long)pb * PB * S::NCSP;
+  const R* tv = (const R*)tabv + (long)pb * PB * S::NCSP;
   const __amdgpu_buffer_rsrc_t trs = buffer_rsrc(tv, PB * S::NCSP * (int)sizeof(R));
   for (int w = tid; w < S::NCSP; w += NT) {
     const int m = m_of_w(T, w);

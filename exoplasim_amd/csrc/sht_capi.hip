@@ -76,8 +76,8 @@ static int build_tables(Tables& t, int ntru, const double* sid, const double* gw
   HIPCK(hipMalloc(&t.tab, sizeof(double) * NTAB * tsz));
   HIPCK(hipMalloc(&t.filt64, sizeof(double) * NTAB * tsz));
   HIPCK(hipMalloc(&t.filt32, sizeof(float) * NTAB * tsz));
-  HIPCK(hipMalloc(&t.fwd4, sizeof(float) * NTAB * tsz));
-  HIPCK(hipMalloc(&t.fwd2, sizeof(double) * NTAB * tsz));
+  HIPCK(hipMalloc(&t.fwd4, sizeof(float) * tsz));
+  HIPCK(hipMalloc(&t.fwd2, sizeof(double) * tsz));
   HIPCK(hipMalloc(&t.skgpsp, sizeof(double) * (ntru + 1)));
   HIPCK(hipMalloc(&t.skspgp, sizeof(double) * (ntru + 1)));
   HIPCK(hipMalloc(&t.tw64, sizeof(double) * 2 * t.nlon));
@@ -101,8 +101,9 @@ static int build_tables(Tables& t, int ntru, const double* sid, const double* gw
   k_filtered<<<(unsigned)((nf + 255) / 256), 256>>>(ntru, t.npair, t.tab, t.skgpsp, t.skspgp,
                                                     t.filt64, t.filt32);
   HIPCK(hipGetLastError());
-  k_pack_fwd<float><<<(unsigned)((nf + 255) / 256), 256>>>(t.npair, t.ncsp, t.filt32, t.fwd4);
-  k_pack_fwd<double><<<(unsigned)((nf + 255) / 256), 256>>>(t.npair, t.ncsp, t.filt64, t.fwd2);
+  const unsigned nfw = (unsigned)((tsz + 255) / 256);
+  k_pack_fwd<float><<<nfw, 256>>>(t.npair, t.ncsp, t.filt32 + TQC * tsz, t.fwd4);
+  k_pack_fwd<double><<<nfw, 256>>>(t.npair, t.ncsp, t.filt64 + TQC * tsz, t.fwd2);
   HIPCK(hipGetLastError());
   // 512 (FP32) and 256 (FP64) elements per (pair block, m, n block)
   const long inv_blocks = (long)(t.npair / 8) * (ntru + 1) * t.kbmax;

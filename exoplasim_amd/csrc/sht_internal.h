@@ -38,8 +38,9 @@ struct Tables {
   double* tab = nullptr;      // [8][npair][ncsp] unfiltered
   double* filt64 = nullptr;   // [8][npair][ncsp] filter folded in
   float* filt32 = nullptr;
-  float* fwd4 = nullptr;      // [8][npair/4][ncsp][4]: filt32 with 4 pairs side by side
-  double* fwd2 = nullptr;     // [8][npair/2][ncsp][2]: filt64 with 2 pairs side by side
+  // the direct transform's table qc, its pairs of 16 bytes together side by side
+  float* fwd4 = nullptr;      // [npair/4][ncsp][4] of filt32
+  double* fwd2 = nullptr;     // [npair/2][ncsp][2] of filt64
   double* skgpsp = nullptr;   // [ntru+1]
   double* skspgp = nullptr;
   // split-BF16 inverse table operands (3 planes): qi, qj, and under TQV qv and

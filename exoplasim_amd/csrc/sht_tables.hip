@@ -250,22 +250,19 @@ __global__ void k_pack_dir(int ntru, int npair, int rb, int t, const double* fil
                        : 0.0f;
 }
 
-// ---- the tables of the direct transform (k_fwd): G latitude pairs of 16
-// bytes together side by side (FP32: 4, FP64: 2), [t][pair / G][w][pair % G],
+// ---- a table [pair][w] for the direct transform (k_fwd): G latitude pairs of
+// 16 bytes together side by side (FP32: 4, FP64: 2), [pair / G][w][pair % G],
 // so that a lane summing coefficient w reads G pairs in one 16-byte load and
 // the lanes of a wave (consecutive w) read one contiguous run ----
 template <typename R>
 __global__ void k_pack_fwd(int npair, int ncsp, const R* filt, R* out) {
   constexpr int G = 16 / sizeof(R);
-  const long total = (long)NTAB * npair * ncsp;
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= total) return;
+  if (i >= (long)npair * ncsp) return;
   const int u = (int)(i % G);
   const int w = (int)((i / G) % ncsp);
-  const long tg = i / ((long)G * ncsp);  // t * (npair / G) + pair group
-  const int g = (int)(tg % (npair / G));
-  const int t = (int)(tg / (npair / G));
-  out[i] = filt[((long)t * npair + G * g + u) * ncsp + w];
+  const int g = (int)(i / ((long)G * ncsp));
+  out[i] = filt[((long)G * g + u) * ncsp + w];
 }
 template __global__ void k_pack_fwd<float>(int, int, const float*, float*);
 template __global__ void k_pack_fwd<double>(int, int, const double*, double*);

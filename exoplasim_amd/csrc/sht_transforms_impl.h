@@ -257,7 +257,7 @@ static int fwd_tv(const Tables& tb, bool fused, const FwdArgs& a, void* scratch,
   if (nblk <= 0) return 0;
   if (C::NPB > 1 && (scratch == nullptr || sbytes < fwd_scratch_t<T, MODE>(a.nmem, a.nfield)))
     return -4;
-  // the direct sums read tables whose pairs lie side by side by 16 bytes
+  if (a.table != TQC) return -2;  // the table whose pairs lie side by side by 16 bytes
   const void* tv = (MODE == MODE_F64) ? (const void*)tb.fwd2 : (const void*)tb.fwd4;
   const void* tw = (MODE == MODE_F64) ? (const void*)tb.tw64 : (const void*)tb.tw32;
   dim3 grid((unsigned)nblk), block(C::NT);

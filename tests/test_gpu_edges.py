@@ -813,3 +813,23 @@ def test_untuned_tiles_many_blocks(oracle, gpu, ntru, mode):
     (T63 FP64, two latitude blocks: 1952).  So the whole tiles: V = 2, in the
     FP64 direct of T42 V = 0."""
     test_untuned_tiles(oracle, gpu, ntru, 20, 16, mode)
+
+
+def test_plan_memory(gpu):
+    """device memory of a T127 plan.  Tables of 96 x 8256 values: 8 in FP64 as
+    built, 8 with the filters in FP64 and FP32 (50.7, 50.7 and 25.4 MB), the
+    direct transform's one in both (9.5); the four inverse tables as matrix
+    operands (2 x 50.3 MB, and split BF16) and the four direct ones: about 300
+    MB.  All eight tables in the direct transform's order would add 67."""
+    import torch
+
+    from exoplasim_amd import sht
+
+    sht.Plan(127).close()  # the library's own memory
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan = sht.Plan(127)
+    used = free - torch.cuda.mem_get_info()[0]
+    plan.close()
+    print(f"T127 plan {used / 1e6:.0f} MB", flush=True)
+    assert used < 320e6
