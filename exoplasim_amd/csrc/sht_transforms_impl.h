@@ -145,22 +145,23 @@ static int inv_tv(const Tables& tb, bool fused, const InvArgs& a, hipStream_t s)
 }
 
 // The tile variant of a fused inverse on a plan that was not tuned, from the
-// blocks it would have with half the fields per block (V = 3).  While those fit
-// the 256 CUs (two per CU where a block's LDS and its half-filled matrix tile
-// allow it: below T63, and in the FP32 mode, which uses no matrix tiles, at
-// T63) they only engage idle CUs; above, whole blocks on 512 threads.  Round
-// trip inverses in us, V = 0, 2, 3: T42 L20 BF16X3, 1 member 17.7, 13.8, 13.2;
-// 4 members 19.1, 15.2, 18.2; T63 L20 FP64, 1 member 24.9, 21.0, 27.5; L10
-// 24.0, 20.1, 18.1; T127 L10 FP32MFMA, 4 members 272, 155, 206.  The two
-// exceptions: FP64 at T21, whose short rows keep 256 threads busy (L20, 16
-// members 18.7, 21.0, 29.9), and FP32 up to T42, whose vector sums want the
-// most waves (T42 L20, 16 members 233, 145, 111).
+// blocks it would have with half the fields per block (V = 3).  While those
+// have a CU each (256) they only engage idle CUs; above, whole blocks on 512
+// threads, whose matrix tiles are full.  Round trip inverses in us, V = 0, 2, 3, by
+// those blocks: T42 BF16X3 108: 18.2, 13.5, 12.4; 224: 18.7, 14.1, 13.1; 280:
+// 19.0, 14.6, 16.8; 432: 19.9, 15.7, 18.5; FP32MFMA 216: 24.9, 17.4, 15.8; 280: 25.0, 17.6,
+// 19.2; T21 BF16X3 224: 11.8, 10.6, 10.2; 270: 12.2, 10.9, 12.1; T63 BF16X3 252: 26.6,
+// 19.1, 17.5; 264: 26.6, 19.1, 23.0.  Exceptions: FP64 at T21, whose short rows
+// keep 256 threads busy (L20, 16 members 18.7, 21.0, 29.9); FP32, which has no
+// matrix tiles and whose vector sums want the most waves, up to T42 (L20, 16
+// members 233, 145, 111) and to two and a half blocks per CU at T63 (sp2fc alone
+// 504: 95, 75, 57; 630: 94, 75, 73; 756: 95, 76, 82; the round trip's inverse 528:
+// 218, 145, 118; 1008: 278, 177, 196).
 template <int T, int MODE>
 static int inv_auto(long nblk3) {
   if (MODE == MODE_F64 && T == 21) return 0;
   if (MODE == MODE_F32 && T <= 42) return 3;
-  constexpr bool two = MODE == MODE_F32 ? T < 127 : (MODE != MODE_F64 && T <= 42);
-  return nblk3 <= (two ? 512 : 256) ? 3 : 2;
+  return nblk3 <= (MODE == MODE_F32 && T == 63 ? 640 : 256) ? 3 : 2;
 }
 
 // blocks at V = 3 of the call that a launch belongs to: a call that runs its
