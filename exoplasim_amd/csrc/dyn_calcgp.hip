@@ -15,16 +15,17 @@
 // share the levels, a lane owning the same points at each.  What a level needs
 // of the others -- v . grad ln ps, the divergence and the humidity term --
 // meets in LDS, and c and g are read through scalar loads (a wave's lanes all
-// work on one level).  The kernel is bound by HBM and L2: 6 fields are read
-// and 11 written per level.
+// work on one level).  6 fields are read and 11 written per level.  On large
+// calls the vector ALUs (65% busy at T42 L20, 32 members, FP32) and HBM (3.7 TB/s
+// there) bound it together, on small ones the chain of a wave's levels.
 //
 // (One thread per column with its level arrays in registers held 202 VGPRs at
 // L20 in FP32 and spilled at L40 in FP64; level counts without an
 // instantiation of their own kept the arrays in scratch.  gridpointa of T42
 // L20, 32 members, FP32: 336 us with it and the row FFT as a launch, 318 with
-// this kernel on the grid, 273 with the rows transformed in it; T21 L10, one
-// member, FP64: 49, 39.5, 37.5 us; T63 L20, 3 members, FP64: 294 and 253 us on
-// the grid.)
+// this kernel on the grid, 273 with the rows transformed in it, and 239 -> 222 by a
+// lane's points side by side and rows of half the length; T21 L10, one member,
+// FP64: 49, 39.5, 37.5 us; T63 L20, 3 members, FP64: 294 and 253 us on the grid.)
 #include "../../include/exo_dyn.h"
 #include "sht_plan.h"
 
@@ -483,12 +484,13 @@ static int calcgp_t(exo_dyn_t d, int nmem, long ms, int nhor, int nqspec, int ex
   };
   const int n = d->nlev;
   // Waves per block of a row kernel.  Up to one block per CU its own chain of
-  // levels is the time, and 10 waves shorten it (T21 L10 FP64, one member,
-  // gridpointa 28.8 -> 26.6 us; T42 L13 FP32 42.9 -> 40.9), but in FP64 on rows
-  // of 128, whose registers do not allow it (T42 L10 49 -> 62).  Above, FP64
-  // takes 4: twice the blocks fit a CU's LDS, and the levels come out evenly
-  // (T42 L20, 8 members, 133.5 -> 125.4; T21 L10, 32 members, 73.4 -> 67.1; FP32
-  // T42 L20, 32 members, 235.6 against 244.4).
+  // levels is the time, and 10 waves shorten it (gridpointa, 10 against 8 and 4
+  // waves: T21 L10 FP64, one member, 26.6, 26.9, 29.4 us; T42 L10 FP32 38.3, 39.4,
+  // 42.1), but in FP64 on rows of 128, whose registers do not allow it (T42 L10
+  // 54.3, 46.7, 50.7).  Above, FP64 takes 4, two of whose blocks fit a CU's LDS (8
+  // against 4: T42 L20, 8 members, 126.3, 119.7; T21 L10, 32 members, 68.5, 65.4;
+  // from L20 on 8 would do better at T21: 103, 111), FP32 8 (T42 L20, 32 members,
+  // 10, 8 and 4: 278.7, 247.9, 255.7).
   const bool few = (long)(nhor / (nlon > 0 ? nlon : 1)) * nmem <= 256;
   switch (tw ? nlon : 0) {
     case 64:
@@ -533,7 +535,7 @@ static bool calcgp_in_place(const exo_calcgp_fields* f, size_t bytes) {
 
 // Does gridpointa's calcgp transform its rows itself?  On rows of 64 and 128
 // whose level arrays fit a CU's LDS (all levels but FP64 above L41 on 128).
-// Three points per lane on rows of 192 spill (T63 L20, 16 members, FP32: 479 us
+// Three points per lane on rows of 192 spilled (T63 L20, 16 members, FP32: 479 us
 // against 390 with calcgp on the grid and the row FFT as a launch; FP64, 3
 // members: 289 against 253).
 constexpr size_t GP_LDS = 160 * 1024;

@@ -44,9 +44,9 @@ struct InvCfg {
   // phase, of which 8 then run the FFT rows (one row buffer each)
   static constexpr int NT = (V == 2 || V == 3) ? ((STAGED && V == 2) ? 1024 : 512) : 256;
   static constexpr int NWF = (NT / 64 < 8) ? NT / 64 : 8;  // staged: FFT waves
-  // MFMA work items in flight per wave, one table (D1) or two (D2; dv2uv
-  // carries two tables per item, and one item ahead keeps its registers
-  // within four waves per SIMD)
+  // MFMA work items in flight per wave: sp2fc (D1), dv2uv (D2: two products
+  // per item, of two tables or, in split BF16, of the two in one operand; one
+  // item ahead keeps its registers within four waves per SIMD)
   static constexpr int D1 = 2;
   static constexpr int D2 = 1;
   // Latitude-pair blocks per tile of the block order (scalar, dv2uv items):
@@ -232,8 +232,8 @@ __device__ __forceinline__ void inv_body(const InvArgs& a, int blk, const void* 
     // FP32 form, whose rows hold zeros at every other n and whose columns 2 FB
     // .. 15 are empty at FB = 4; the spectral loads use all lanes.  (Round trip
     // of T42 L20, 32 members, 288 -> 184 us; gridpointa of T63 L20, 3 members,
-    // 272 -> 189; a T21 L10 step 43 -> 37.  The FP64 matrix rate then bounds
-    // the Legendre sums: 64 cycles per instruction, half of it used.)
+    // 272 -> 189; a T21 L10 step 43 -> 37.  What is left is latency: at T42 the
+    // matrix units are busy 24% of the time, the vector ALUs 40%.)
     // The wave index is read into a scalar register, so that the item loop
     // (m, kb), its branches and the operand offsets are wave-uniform scalar
     // work rather than per-lane vector arithmetic.

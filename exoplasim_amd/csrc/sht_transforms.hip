@@ -199,9 +199,9 @@ static int fft_t(const void* tw, int dir, R* a, long lot, int nmem, long mstride
 // the four runs (h, re/im) of j = 4g .. 4g + 3.  Consecutive lanes read
 // consecutive bytes and write whole 64-byte groups; the wavenumber of a group
 // comes from a table.  Coefficients past the truncation are zeros.  (128
-// members of T42 L20: 22.1 us, against 32.7 with 64 bytes per thread, whose loads
-// and stores touch a line per lane, and 23.2 for rows of one component and
-// parity, 32 bytes per thread and m found by bisection.)
+// members of T42 L20: 22.1 us; rows of one component and parity, 32 bytes per
+// thread and m found by bisection, took 23.0, and this order with 64 bytes per
+// thread, whose loads and stores touch a line per lane, 32.7.)
 // ---------------------------------------------------------------------------
 template <int T>
 struct PkWave {  // m of each 32 values of a field's operand
