@@ -833,3 +833,36 @@ def test_plan_memory(gpu):
     plan.close()
     print(f"T127 plan {used / 1e6:.0f} MB", flush=True)
     assert used < 320e6
+
+
+@pytest.mark.parametrize("ntru,nlev", [(21, 10), (42, 7)])
+@pytest.mark.parametrize("mode", ["f64", "f32"])
+def test_gridpointa_unaligned_work(oracle, gpu, ntru, nlev, mode):
+    """a work array that starts one value past an allocation, its members an
+    odd number of values apart: a lane's two points are then not on their own
+    size, and every value is that of the aligned call"""
+    import torch
+
+    from exoplasim_amd import sht
+    from exoplasim_amd._lib import lib
+    from exoplasim_amd.dynamics import Dynamics
+
+    print(f"unaligned work T{ntru} L{nlev} {mode}", flush=True)
+    plan, dyn = sht.Plan(ntru), Dynamics.from_vertical(_vertical(oracle, nlev), *PLASIM_SCAL)
+    st, work, tend = dyn.alloc_gridpointa(plan, 3, mode)
+    st.copy_(torch.from_numpy(np.stack([gridpointa_state(ntru, nlev, 0.9 + 0.1 * k)
+                                        for k in range(3)])).to(st.dtype))
+    dyn.gridpointa(plan, mode, st, work, tend)
+    n, per = work[0].numel(), work[0].numel() + 3
+    buf = torch.zeros(3 * per + 1, dtype=st.dtype, device="cuda")
+    out = torch.zeros_like(tend)
+    assert lib().exo_gridpointa(plan._h, dyn._h, 0 if mode == "f64" else 1, 3, 1, st.data_ptr(),
+                                st[0].numel(), buf.data_ptr() + buf.element_size(), per,
+                                out.data_ptr(), out[0].numel(),
+                                torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, tend)
+    for k in range(3):
+        assert torch.equal(buf[1 + k * per:1 + k * per + n], work[k].view(-1))
+    dyn.close()
+    plan.close()
